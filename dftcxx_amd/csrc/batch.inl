@@ -292,60 +292,54 @@ int batch_mol_of_atom(const dg_handle* h, int k) {
   return m;
 }
 
-// Work list of the cross-atom potentials: for every atom k, the points of its
-// molecule outside its own cell, in ranges of at most len (<= kMaxItem) points,
-// k ascending: {k, p_begin, p_end, offset of the item's point order in perm}.
-// An item's order holds its points and at most one pad slot per spline
-// interval group (nrad + 1 groups); *perm_len receives the total.  A range is
-// cut into equal items of at most cap points, cap chosen so that an item's
-// padded order never exceeds len slots: the cross kernel walks an item in
-// passes of 2048 slots, and an order just over a multiple of that would take
-// a nearly empty extra pass.
-std::vector<int> cross_items(const dg_handle* h, int len, long* perm_len) {
-  std::vector<int> items;
-  long off = 0;
-  const long cap = std::max<long>(len / 2, len - (h->nrad + 1));
-  auto add = [&](int k, long b, long e) {
-    const long m = (e - b + cap - 1) / cap;
-    for (long r = 0; r < m; ++r) {
-      const long p = b + (e - b) * r / m, q = b + (e - b) * (r + 1) / m;
-      items.push_back(k);
-      items.push_back((int)p);
-      items.push_back((int)q);
-      items.push_back((int)off);
-      off += (q - p) + std::min<long>(q - p, h->nrad + 1);
-    }
-  };
+// Points of a cross-potential item of at most about len points: whole shells, one
+// at least.
+int cross_item_pts(const dg_handle* h, int len) { return std::max(1, len / h->nang) * h->nang; }
+
+// Work list of the cross-atom potentials: for every atom k, every other cell of its
+// molecule in equal runs of at most cross_item_pts(len) points, k ascending.
+std::vector<CrossItem> cross_items(const dg_handle* h, int len) {
+  std::vector<CrossItem> items;
+  const int cap = cross_item_pts(h, len) / h->nang, runs = (h->nrad + cap - 1) / cap;
   for (int k = 0; k < h->natoms; ++k) {
-    long p0 = 0, p1 = h->npts;
+    int a0 = 0, a1 = h->natoms;
     if (h->nmol) {
       const int m = batch_mol_of_atom(h, k);
-      p0 = (long)h->h_mol_atom0[m] * h->cell;
-      p1 = (long)h->h_mol_atom0[m + 1] * h->cell;
+      a0 = h->h_mol_atom0[m];
+      a1 = h->h_mol_atom0[m + 1];
     }
-    if (p1 - p0 <= h->cell) continue;
-    add(k, p0, (long)k * h->cell);
-    add(k, (long)(k + 1) * h->cell, p1);
+    for (int a = a0; a < a1; ++a)
+      for (int r = 0; r < runs && a != k; ++r) {
+        const int p = h->nrad * r / runs, q = h->nrad * (r + 1) / runs;
+        items.push_back({k, a, p, q - p});
+      }
   }
-  if (perm_len) *perm_len = off;
   return items;
 }
 
+// Points per item: 4096 where that makes four items per CU, else halved down to 512.
+// Longer items group better (C30H62: 7 % of the lanes idle at 4096, 11 at 2048) and a
+// work-group costs its launch; shorter ones spread a small molecule over the chip
+// (cross kernel, us at 4096 / 2048 / 1024 / 512: H2O 50 x 110 30 / 25 / 20 / 20, ethane
+// 20 x 146 35 / 29 / 22 / 20, benzene 85 / 80 / 87 / 127, C10H22 417 / 431 / 466 / 736).
+int cross_item_len(const dg_handle* h) {
+  int len = 4096;
+  while (len > 512 && cross_items(h, len).size() < 4 * 256) len /= 2;
+  return len;
+}
+
 int set_items(dg_handle* h, int len) {
-  long plen = 0;
-  std::vector<int> items = cross_items(h, len, &plen);
-  if (items.size() > h->items_cap || plen > h->npairs)
+  const std::vector<CrossItem> items = cross_items(h, len);
+  const int pts = cross_item_pts(h, len), maxt = cross_max_tasks(pts, h->nrad);
+  if (items.size() > h->items_cap || items.size() * maxt > h->task_cap)
     return fail(DG_ERR_INVALID, "cross-potential item list exceeds its buffer");
   if (!items.empty())
-    HIP_TRY(hipMemcpy(h->items, items.data(), items.size() * 4, hipMemcpyHostToDevice));
-  h->nitems = (int)items.size() / 4;
-  DG_TRY(sort_items(h));
-  int cus = 0;
-  HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device));
-  const int per_cu = std::max(1, (int)((160 * 1024) / std::max<size_t>(h->cross_lds, 1)));
-  h->cross_wgs = std::max(1, std::min(h->nitems, cus * std::min(per_cu, 2)));
+    HIP_TRY(hipMemcpy(h->items, items.data(), items.size() * sizeof(CrossItem), hipMemcpyHostToDevice));
+  h->nitems = (int)items.size();
+  h->item_pts = pts;
+  h->max_tasks = maxt;
   h->item_len = len;
-  return DG_OK;
+  return sort_items(h);
 }
 
 std::vector<int> batch_chunks(const dg_handle* h, int len, std::vector<int>* first) {
@@ -376,7 +370,6 @@ int set_bchunks(dg_handle* h, int len) {
 }
 
 constexpr int kChunkCandidates[] = {256, 512, 1024, 2048, 4096};
-constexpr int kItemCandidates[] = {1024, 2048, 4096};
 
 int batch_alloc(dg_handle* h, const BatchSpec* bs, const std::vector<int>&) {
   const int nm = bs->nmol;

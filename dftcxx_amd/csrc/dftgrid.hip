@@ -22,6 +22,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/dftgrid.h"
@@ -906,12 +907,11 @@ __global__ __launch_bounds__(256) void k_poisson(const double* __restrict__ rho_
 // (src/atomicgrid.cpp:434-462): tile (shells i0.., angular points j0..) of atom a.
 // |r_p - R_a| is the radial node r_i (the point is R_a + r_i Omega_j with a unit
 // Omega_j), which spares the coordinate reads.
-// (Four waves per work-group, one tile each: tile 4 blockIdx.x + wave.)
-__global__ __launch_bounds__(256) void k_vcell(const double* __restrict__ U, const double* __restrict__ ylm,
-                                               const double* __restrict__ rad, int nrad, int nang, int nlm,
-                                               long ntiles, double* vcell) {
+// One wave per tile.
+__device__ __forceinline__ void vcell_tile(const double* __restrict__ U, const double* __restrict__ ylm,
+                                           const double* __restrict__ rad, int nrad, int nang, int nlm, long tile,
+                                           long ntiles, double* vcell) {
   const int ti = (nrad + 15) / 16, tj = (nang + 15) / 16;
-  const long tile = 4L * blockIdx.x + (threadIdx.x >> 6);
   if (tile >= ntiles) return;
   const int a = (int)(tile / (ti * tj)), rem = (int)(tile % (ti * tj));
   const int i0 = 16 * (rem / tj), j0 = 16 * (rem % tj);
@@ -938,31 +938,15 @@ __global__ __launch_bounds__(256) void k_vcell(const double* __restrict__ U, con
   }
 }
 
-struct CrossArgs {
-  const double* rad;    // radial nodes (nrad)
-  const double* leb;    // Lebedev directions and weights (4 nang)
-  const double* atoms;
-  const double* knots;  // ascending, nrad
-  const double* invh;   // 1/(x_t - x_{t-1})
-  const double* tab;    // [natoms][nrad][nlm]{y, D}
-  const int* items;     // {k, p_begin, p_end, perm offset} point ranges outside cell k, k ascending
-  const unsigned short* perm;  // per item, its points by distance to atom k, interval groups padded to even
-  const unsigned short* pkey;  // interval key (spline_key) of every perm slot
-  const int* plen;             // per item, the padded length of its perm range
-  double* vpart;        // partial potentials, atom k's at vpart + vbase[k] + p
-  const long* vbase;
-  int nitems, nrad, nlm, l0, l1, accumulate, nang;
-  double inv_nang, inv_nrad;  // 1/nang, 1/nrad: grid indices of a point
-};
-
-// Distance r of a point from an atom centre and its distance rxy from the
-// atom's z axis, given the offset (dx, dy, dz).  One definition for the item
-// sort and the potential kernel, so that both see the same r.
-__device__ __forceinline__ void point_polar(double dx, double dy, double dz, double& rxy, double& r) {
-  const double rxy2 = dx * dx + dy * dy;
-  r = sqrt(rxy2 + dz * dz);
-  rxy = sqrt(rxy2);
-}
+// --- cross-atom potentials ---------------------------------------------------
+// V_k(p) = sum_lm Y_lm(r_p - R_k) S_{k,lm}(|r_p - R_k|) / |r_p - R_k| outside cell
+// k (src/moleculargrid.cpp:349-376).  On one spline interval S is a cubic in
+// t = r - x_{s-1} and Y_lm = N_lm Re/Im[(x + iy)^m] q_lm(z) with (x, y, z) the unit
+// vector and q_lm a polynomial in z, so that V_k r is
+//   sum_j t^j sum_m { Re[(x+iy)^m] sum_i C+_{j,m,i} z^i + Im[(x+iy)^m] sum_i C-_{j,m,i} z^i },
+// 4 (lmax+1)^2 coefficients per (atom, interval).  The coefficients are formed once
+// per build (cross_coef below); the potential kernel is then Horner's rule, one
+// multiply-add per coefficient and point, with no recurrence.
 
 // Spline interval of r over the ascending knots kn[0..n): the reference's first
 // knot s >= 1 with r <= kn[s] (the interval is [s-1, s]), or 0 / n for r below
@@ -981,326 +965,317 @@ __device__ __forceinline__ int spline_key(double r, const double* kn, int n) {
   return lo;
 }
 
-// Inclusive scan (maximum or sum) of a[0..len) by the whole work-group, ping-ponging
-// between a and b; returns the buffer that holds the result.
-template <bool MAX>
-__device__ int* block_scan(int* a, int* b, int len) {
-  for (int d = 1; d < len; d <<= 1) {
-    for (int i = threadIdx.x; i < len; i += blockDim.x) {
-      const int v = a[i];
-      b[i] = (i >= d) ? (MAX ? max(v, a[i - d]) : v + a[i - d]) : v;
-    }
-    __syncthreads();
-    int* t = a;
-    a = b;
-    b = t;
+// One (atom, interval key, output group) of the coefficients.  Group q of the nlm
+// groups: grp[q] = {m, i, sign, offset}, its four cubic coefficients go to
+// coef[(k (nrad+1) + key) 4 nlm + offset + j].  mono[(l L1 + m) L1 + i], L1 = lmax+1,
+// is the coefficient of z^i in (-1)^m (2m-1)!! q_lm / c_lm (monic up to the sign and
+// the double factorial; tab carries N_lm c_lm).
+struct CoefArgs {
+  const double* tab;   // [natoms][nrad][nlm]{y, D}, see k_poisson
+  const double* invh;  // 1/(x_t - x_{t-1})
+  const double* mono;
+  const int4* grp;
+  int nrad, nlm, lmax;
+  long total;  // natoms (nrad+1) nlm
+  double* coef;
+};
+
+__device__ __forceinline__ void cross_coef(const CoefArgs& A, long e) {
+  if (e >= A.total) return;
+  const int q = (int)(e % A.nlm);
+  const long ks = e / A.nlm;
+  const int key = (int)(ks % (A.nrad + 1)), k = (int)(ks / (A.nrad + 1));
+  const int4 g = A.grp[q];
+  const int m = g.x, i = g.y, L1 = A.lmax + 1, n = A.nrad;
+  const bool clamp = key == 0 || key == n;
+  const int s1 = clamp ? (key == 0 ? 0 : n - 1) : key, s0 = clamp ? s1 : key - 1;
+  const double2* T0 = reinterpret_cast<const double2*>(A.tab) + ((long)k * n + s0) * A.nlm;
+  const double2* T1 = reinterpret_cast<const double2*>(A.tab) + ((long)k * n + s1) * A.nlm;
+  double y0 = 0.0, d0 = 0.0, y1 = 0.0, d1 = 0.0;
+  for (int l = m + i; l <= A.lmax; l += 2) {  // q_lm has the parity of l - m
+    const double c = A.mono[(l * L1 + m) * L1 + i];
+    const int lm = l * l + l + (g.z ? -m : m);
+    const double2 a = T0[lm], b = T1[lm];
+    y0 += c * a.x;
+    d0 += c * a.y;
+    y1 += c * b.x;
+    d1 += c * b.y;
   }
-  return a;
+  dbl4 o = {y0, 0.0, 0.0, 0.0};
+  if (!clamp) {
+    const double h = A.invh[s1], dy = (y1 - y0) * h;
+    o[1] = d0;
+    o[2] = h * (3.0 * dy - 2.0 * d0 - d1);
+    o[3] = h * h * (-2.0 * dy + d0 + d1);
+  }
+  *reinterpret_cast<dbl4*>(A.coef + ks * 4 * A.nlm + g.w) = o;
 }
 
-// Points of every cross-potential item in order of their distance to the
-// item's atom, grouped by spline interval, each group padded to an even count:
-// perm[off + i] is the offset (from p_begin) of the i-th point, 0xFFFF a pad
-// slot (always at an odd position), pkey[off + i] the slot's interval key
-// (spline_key) and plen[item] the padded length.  Two consecutive slots from an
-// even position then always share their interval.  One work-group per item (at
-// most kMaxItem points), bitonic sort in LDS.
-constexpr int kMaxItem = 4096;
-constexpr unsigned short kPadSlot = 0xFFFF;
-__global__ __launch_bounds__(1024) void k_sort_items(const int* __restrict__ items, const double* __restrict__ atoms,
-                                                     const double* __restrict__ px, const double* __restrict__ py,
-                                                     const double* __restrict__ pz, const double* __restrict__ knots,
-                                                     int nrad, unsigned short* perm, unsigned short* pkey,
-                                                     int* plen) {
-  __shared__ double key[kMaxItem];
-  __shared__ unsigned short idx[kMaxItem];
-  __shared__ int grp[kMaxItem];
-  const int* it = items + 4 * blockIdx.x;
-  const int k = it[0];
-  const long pb = it[1];
-  const int len = it[2] - it[1];
-  int n2 = 1;
-  while (n2 < len) n2 <<= 1;
-  const double ax = atoms[4 * k], ay = atoms[4 * k + 1], az = atoms[4 * k + 2];
-  for (int i = threadIdx.x; i < n2; i += blockDim.x) {
-    double r = 1e300;
+// k_vcell's tiles (the first nvb work-groups) and the cross-potential coefficients
+// (the others) in one launch: both need only U and the spline table, and a build of
+// a small molecule is bound by its launches.
+__global__ __launch_bounds__(256) void k_vcell_coef(const double* __restrict__ U, const double* __restrict__ ylm,
+                                                    const double* __restrict__ rad, int nrad, int nang, int nlm,
+                                                    long ntiles, double* vcell, int nvb, CoefArgs C) {
+  if ((int)blockIdx.x < nvb)
+    vcell_tile(U, ylm, rad, nrad, nang, nlm, 4L * blockIdx.x + (threadIdx.x >> 6), ntiles, vcell);
+  else
+    cross_coef(C, (long)(blockIdx.x - nvb) * 256 + threadIdx.x);
+}
+
+// Work items: runs of whole shells (the nang points of one radius) of one cell other
+// than k.
+struct CrossItem {
+  int k;       // atom whose expansion is evaluated
+  int cell;    // atom whose shells these are
+  int i0;      // first radial index
+  int nshell;
+};
+
+constexpr int kMaxItem = 4096;    // points of an item (their potentials sit in LDS)
+constexpr int kCrossThreads = 512;
+constexpr int kTaskPts = 128;     // points of a task: two per lane of one wave
+
+// Upper bound of an item's tasks: full tasks of its points and one partial task per
+// spline interval it touches.
+__host__ __device__ inline int cross_max_tasks(int item_pts, int nrad) {
+  return item_pts / kTaskPts + (item_pts < nrad + 1 ? item_pts : nrad + 1) + 1;
+}
+
+// Groups every item's points by spline interval (counting sort in LDS) and cuts the
+// groups into tasks of at most kTaskPts points, one wave each:
+//   perm[vbase[k] + p_begin + s]   offset (from p_begin) of the item's s-th point,
+//   task[item maxt + t]            first s | (points - 1) << 12 | interval key << 19
+// (keys up to nrad + 1 <= 3777, see dg_create's bound on the radial grid).
+// The order inside a group does not matter: a point's potential does not depend on
+// its slot.
+__global__ __launch_bounds__(kCrossThreads) void k_sort_items(
+    const CrossItem* __restrict__ items, const double* __restrict__ atoms, const double* __restrict__ px,
+    const double* __restrict__ py, const double* __restrict__ pz, const double* __restrict__ knots,
+    const long* __restrict__ vbase, int nrad, int nang, int maxt, unsigned short* perm, unsigned* task, int* ntask) {
+  __shared__ unsigned short out[kMaxItem];
+  extern __shared__ int lds_int[];
+  int* cnt = lds_int;             // [nrad + 1] points per key
+  int* base = cnt + nrad + 1;     // [nrad + 1] first slot
+  int* tbase = base + nrad + 1;   // [nrad + 1] first task
+  const CrossItem it = items[blockIdx.x];
+  const long pb = ((long)it.cell * nrad + it.i0) * nang;
+  const int len = it.nshell * nang;
+  for (int i = threadIdx.x; i <= nrad; i += kCrossThreads) cnt[i] = 0;
+  __syncthreads();
+  const double ax = atoms[4 * it.k], ay = atoms[4 * it.k + 1], az = atoms[4 * it.k + 2];
+  int key[kMaxItem / kCrossThreads], rank[kMaxItem / kCrossThreads];
+#pragma unroll
+  for (int u = 0; u < kMaxItem / kCrossThreads; ++u) {
+    const int i = threadIdx.x + kCrossThreads * u;
+    key[u] = rank[u] = 0;
     if (i < len) {
-      double rxy;
-      point_polar(px[pb + i] - ax, py[pb + i] - ay, pz[pb + i] - az, rxy, r);
+      const double dx = px[pb + i] - ax, dy = py[pb + i] - ay, dz = pz[pb + i] - az;
+      key[u] = spline_key(sqrt(dx * dx + dy * dy + dz * dz), knots, nrad);
+      rank[u] = atomicAdd(&cnt[key[u]], 1);
     }
-    key[i] = r;
-    idx[i] = (unsigned short)i;
   }
   __syncthreads();
-  for (int size = 2; size <= n2; size <<= 1)
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int i = threadIdx.x; i < n2; i += blockDim.x) {
-        const int j = i ^ stride;
-        if (j > i) {
-          const bool up = (i & size) == 0;
-          const double ki = key[i], kj = key[j];
-          if ((ki > kj) == up && ki != kj) {
-            key[i] = kj;
-            key[j] = ki;
-            const unsigned short t = idx[i];
-            idx[i] = idx[j];
-            idx[j] = t;
-          }
+  if (threadIdx.x < 64) {  // exclusive scans over the keys, 64 at a time
+    int s = 0, t = 0;
+    for (int i0 = 0; i0 <= nrad; i0 += 64) {
+      const int i = i0 + threadIdx.x, c = i <= nrad ? cnt[i] : 0, w = (c + kTaskPts - 1) / kTaskPts;
+      int cs = c, ws = w;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int a = __shfl_up(cs, o), b = __shfl_up(ws, o);
+        if ((int)threadIdx.x >= o) {
+          cs += a;
+          ws += b;
         }
       }
-      __syncthreads();
-    }
-  for (int i = threadIdx.x; i < len; i += blockDim.x) grp[i] = spline_key(key[i], knots, nrad);
-  __syncthreads();
-  // the keys are done with: their space holds two scan buffers
-  int* sa = reinterpret_cast<int*>(key);
-  int* sb = sa + kMaxItem;
-  for (int i = threadIdx.x; i < len; i += blockDim.x) sa[i] = (i == 0 || grp[i] != grp[i - 1]) ? i : 0;
-  __syncthreads();
-  const int* gs = block_scan<true>(sa, sb, len);  // first sorted position of each point's group
-  int flag[kMaxItem / 1024];
-#pragma unroll
-  for (int r = 0; r < kMaxItem / 1024; ++r) {
-    const int i = threadIdx.x + 1024 * r;
-    flag[r] = 0;
-    if (i < len) {
-      const bool last = i == len - 1 || grp[i + 1] != grp[i];
-      flag[r] = (last && ((i - gs[i] + 1) & 1)) ? 1 : 0;
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < kMaxItem / 1024; ++r) {
-    const int i = threadIdx.x + 1024 * r;
-    if (i < len) sa[i] = flag[r];
-  }
-  __syncthreads();
-  const int* pads = block_scan<false>(sa, sb, len);  // pad slots up to and including i's group end
-  unsigned short* out = perm + it[3];
-  unsigned short* okey = pkey + it[3];
-#pragma unroll
-  for (int r = 0; r < kMaxItem / 1024; ++r) {
-    const int i = threadIdx.x + 1024 * r;
-    if (i < len) {
-      const int pos = i + pads[i] - flag[r];
-      out[pos] = idx[i];
-      okey[pos] = (unsigned short)grp[i];
-      if (flag[r]) {
-        out[pos + 1] = kPadSlot;
-        okey[pos + 1] = (unsigned short)grp[i];
+      if (i <= nrad) {
+        base[i] = s + cs - c;
+        tbase[i] = t + ws - w;
       }
+      s += __shfl(cs, 63);
+      t += __shfl(ws, 63);
     }
+    if (threadIdx.x == 0) ntask[blockIdx.x] = t;
   }
-  if (threadIdx.x == 0) plen[blockIdx.x] = len > 0 ? len + pads[len - 1] : 0;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kMaxItem / kCrossThreads; ++u) {
+    const int i = threadIdx.x + kCrossThreads * u;
+    if (i < len) out[base[key[u]] + rank[u]] = (unsigned short)i;
+  }
+  unsigned* tk = task + (long)blockIdx.x * maxt;
+  for (int i = threadIdx.x; i <= nrad; i += kCrossThreads)
+    for (int c = 0; kTaskPts * c < cnt[i]; ++c)
+      tk[tbase[i] + c] = (unsigned)(base[i] + kTaskPts * c) |
+                         (unsigned)(min(kTaskPts, cnt[i] - kTaskPts * c) - 1) << 12 | (unsigned)i << 19;
+  __syncthreads();
+  unsigned short* pm = perm + vbase[it.k] + pb;
+  for (int i = threadIdx.x; i < len; i += kCrossThreads) pm[i] = out[i];
 }
 
-// Potential of atom k's spherical-harmonic expansion at every point outside
-// cell k: V_k(p) = sum_lm Y_lm(r_p - R_k) S_{k,lm}(|r_p - R_k|) / |r_p - R_k|
-// (src/moleculargrid.cpp:349-376).  Persistent: work-group g walks the items
-// [g n/G, (g+1) n/G) of the (atom, point range) list, reloading atom k's spline
-// table for l in [l0, l1) into LDS when k changes.  Each thread takes Q
-// consecutive slots of the item's padded order (perm: by distance to atom k,
-// interval groups padded to even), runs the associated-Legendre / Chebyshev
-// recurrences for each and forms the four sums sum Y y_{s-1}, sum Y D_{s-1},
-// sum Y y_s, sum Y D_s per point, from which the cubic on interval s is
-// evaluated once (linear in the per-lm coefficients).  The Q = 2 slots of a
-// thread share their interval (a pad slot repeats its partner's point and is
-// not written), taken from the sort (pkey), so each table entry is read from
-// LDS once for both.  A slot's coordinates are formed from its grid indices
-// (grid_xyz), not read: the sorted order scatters reads over the item's range.
-// The item's potentials are collected in LDS (vbuf, by offset in the item) and
-// written to vpart in point order once the item is done.
+struct CrossArgs {
+  const double* rad;    // radial nodes (nrad)
+  const double* leb;    // Lebedev directions and weights (4 nang)
+  const double* atoms;
+  const double* knots;  // ascending, nrad
+  const double* coef;   // see cross_coef
+  const CrossItem* items;
+  const unsigned short* perm;
+  const unsigned* task;
+  const int* ntask;
+  double* vpart;        // partial potentials, atom k's at vpart + vbase[k] + p
+  const long* vbase;
+  int nrad, nang, maxt;
+  float inv_nang;
+};
+
+// s += v c with a wave-uniform c read as a scalar operand (left to itself the compiler
+// sums into copies and moves coefficients into vector registers first).
+__device__ __forceinline__ void fma_scalar(double& s, double v, double c) {
+  asm volatile("v_fma_f64 %0, %1, %2, %0" : "+v"(s) : "v"(v), "s"(c));
+}
+
+// f(B), f(B+1), ..., f(E-1) with compile-time arguments (std::integral_constant).
+template <int B, int E, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    static_for<B + 1, E>(f);
+  }
+}
+
+// N wave-uniform doubles read in order through the scalar cache, kChunk at a time.
+// The next chunk is requested right after the first use of the current one (scalar
+// loads return out of order, so a wait is for all of them: a request made before that
+// use would be waited for too) and has the rest of the chunk's work to arrive in.
+template <int N>
+struct ScalarStream {
+  typedef const double __attribute__((address_space(4))) * cptr;
+    static constexpr int kChunk = 20;
+  cptr src;
+  double buf[2][kChunk];
+  __device__ __forceinline__ explicit ScalarStream(const double* p) : src((cptr)p) { load<0>(); }
+  template <int C>
+  __device__ __forceinline__ void load() {
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<0, (N - C * kChunk < kChunk ? N - C * kChunk : kChunk)>(
+        [&](auto i) { buf[C & 1][i] = src[C * kChunk + i]; });
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // use(value P); P ascending from 0
+  template <int P, typename F>
+  __device__ __forceinline__ void take(F&& use) {
+    use(buf[(P / kChunk) & 1][P % kChunk]);
+    if constexpr (P % kChunk == 0 && P + kChunk < N) load<P / kChunk + 1>();
+  }
+};
+
+// V_k r at Q points with unit vectors (x, y, z) and t = r - x_{s-1}, all on the interval
+// whose coefficients start at coef.
 template <int LMAX, int Q>
-__global__ __launch_bounds__(1024) void k_hartree_cross(CrossArgs A) {
-  static_assert(Q == 2, "slots are paired by the item sort");
-  extern __shared__ double lds[];
-  const int n = A.nrad;
-  const int lmb = A.l0 * A.l0, nlmc = A.l1 * A.l1 - lmb;
-  const unsigned lbits = __builtin_amdgcn_readfirstlane(((1u << A.l1) - 1u) & ~((1u << A.l0) - 1u));
-  double* kn = lds;
-  double* ih = lds + n;
-  double* tab = lds + 2 * n;
-  double* vbuf = tab + (long)n * nlmc * 2;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    kn[i] = A.knots[i];
-    ih[i] = A.invh[i];
-  }
-  const int it0 = (int)((long)blockIdx.x * A.nitems / gridDim.x);
-  const int it1 = (int)((long)(blockIdx.x + 1) * A.nitems / gridDim.x);
-  int cur = -1;
-  for (int it = it0; it < it1; ++it) {
-    const int k = A.items[4 * it];
-    if (k != cur) {
-      __syncthreads();
-      const double* src = A.tab + (long)k * n * A.nlm * 2;
-      for (int i = threadIdx.x; i < n * nlmc * 2; i += blockDim.x) {
-        const int t = i / (nlmc * 2), rem = i % (nlmc * 2);
-        tab[i] = src[(long)t * A.nlm * 2 + lmb * 2 + rem];
-      }
-      __syncthreads();
-      cur = k;
-    }
-    const int pb = A.items[4 * it + 1], npt = A.items[4 * it + 2] - pb;
-    const int len = A.plen[it];
-    const unsigned short* pm = A.perm + A.items[4 * it + 3];
-    const unsigned short* pk = A.pkey + A.items[4 * it + 3];
-    const double Ax = A.atoms[4 * k], Ay = A.atoms[4 * k + 1], Az = A.atoms[4 * k + 2];
-    for (int q0 = threadIdx.x * Q; q0 < len; q0 += blockDim.x * Q) {
-      int eq[Q];
-      double rinv[Q], ct[Q], st[Q], cp[Q], sp[Q], tq[Q];
-      bool valid[Q];
-      unsigned short e0 = pm[q0];
-      if (e0 == kPadSlot) e0 = 0;  // not produced by the sort; kept in range regardless
-      const int key = pk[q0];
-      const bool clamp = key == 0 || key == n;
-      const int s1 = clamp ? (key == 0 ? 0 : n - 1) : key;
-      const int s0 = clamp ? s1 : key - 1;
-
-      // knot rows s0 and s1 of the table, indexed by lm from 0 (entries below lmb are not read)
-      const double* T0 = tab + (s0 * nlmc - lmb) * 2;
-      const double* T1 = tab + (s1 * nlmc - lmb) * 2;
-#pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        // a pad slot or a missing tail slot repeats the thread's first point
-        const unsigned short e = (q0 + q < len) ? pm[q0 + q] : kPadSlot;
-        valid[q] = e != kPadSlot;
-        eq[q] = valid[q] ? e : e0;
-        // p = (a nrad + i) nang + j
-        const int p = pb + eq[q];
-        const int ai = (int)(((double)p + 0.5) * A.inv_nang);
-        const int j = p - ai * A.nang;
-        const int a = (int)(((double)ai + 0.5) * A.inv_nrad);
-        const int i = ai - a * n;
-        double x, y, z;
-        grid_xyz(A.atoms, A.rad, A.leb, a, i, j, x, y, z);
-        const double dx = x - Ax, dy = y - Ay, dz = z - Az;
-        double rxy, r;
-        point_polar(dx, dy, dz, rxy, r);
-        rinv[q] = 1.0 / r;
-        ct[q] = dz * rinv[q];
-        st[q] = rxy * rinv[q];
-        cp[q] = 1.0;
-        sp[q] = 0.0;
-        if (rxy > 0.0) {
-          const double ir = 1.0 / rxy;
-          cp[q] = dx * ir;
-          sp[q] = dy * ir;
-        }
-        tq[q] = clamp ? 0.0 : r - kn[s0];
-      }
-      double sy0[Q], sd0[Q], sy1[Q], sd1[Q], pmm[Q], cm[Q], sm[Q];
-#pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        sy0[q] = sd0[q] = sy1[q] = sd1[q] = 0.0;
-        pmm[q] = 1.0;
-        cm[q] = 1.0;
-        sm[q] = 0.0;
-      }
-#pragma unroll
-      for (int m = 0; m <= LMAX; ++m) {
-        if (m > 0) {
-#pragma unroll
-          for (int q = 0; q < Q; ++q) {
-            pmm[q] *= -(double)(2 * m - 1) * st[q];
-            const double c2 = cm[q] * cp[q] - sm[q] * sp[q];
-            sm[q] = sm[q] * cp[q] + cm[q] * sp[q];
-            cm[q] = c2;
-          }
-        }
-        double p1[Q], p2[Q];
-#pragma unroll
-        for (int q = 0; q < Q; ++q) p1[q] = p2[q] = 0.0;
-#pragma unroll
-        for (int l = m; l <= LMAX; ++l) {
-          // scaled recurrence Q_l = P_l / c_lm (legendre_scale; c_lm is folded into
-          // the table): Q_l = ct Q_{l-1} - beta Q_{l-2}, beta = (l+m-1)/(l-m) c_{l-2,m} / c_lm,
-          // a constant after unrolling (a global read of it waited on its full latency)
-          const double beta = (l >= m + 2) ? (double)(l + m - 1) / (double)(l - m) * legendre_scale(l - 2, m) /
-                                                 legendre_scale(l, m)
-                                           : 0.0;
-          double yp[Q], yn[Q];
-#pragma unroll
-          for (int q = 0; q < Q; ++q) {
-            double pl;
-            if (l == m)
-              pl = pmm[q];
-            else if (l == m + 1)
-              pl = ct[q] * pmm[q];
+__device__ __forceinline__ void cross_eval(const double* coef, const double (&x)[Q], const double (&y)[Q],
+                                           const double (&z)[Q], const double (&t)[Q], double (&out)[Q]) {
+  ScalarStream<4 * (LMAX + 1) * (LMAX + 1)> C(coef);
+  double S[Q][4], b[Q][2], cm[Q], sm[Q];
+  static_for<0, LMAX + 1>([&](auto m) {
+    static_for<0, Q>([&](auto q) {  // b = Re, Im of (x + iy)^m z^i
+      b[q][0] = m > 0 ? cm[q] : 1.0;
+      b[q][1] = m > 0 ? sm[q] : 0.0;
+    });
+    static_for<0, LMAX + 1 - m>([&](auto i) {
+      constexpr int w = m > 0 ? 8 : 4;  // coefficients per (m, i): cubic of Re, cubic of Im
+      constexpr int o = (m > 0 ? 4 * (LMAX + 1) + 8 * ((m - 1) * (LMAX + 1) - m * (m - 1) / 2) : 0) + w * i;
+      if constexpr (i > 0)
+        static_for<0, Q>([&](auto q) {
+          b[q][0] = (m == 0 && i == 1) ? z[q] : b[q][0] * z[q];
+          if constexpr (m > 0) b[q][1] *= z[q];
+        });
+      static_for<0, w>([&](auto c) {
+        C.template take<o + c>([&](double v) {
+          static_for<0, Q>([&](auto q) {
+            if constexpr (o + c < 4)
+              S[q][c] = v;
             else
-              pl = ct[q] * p1[q] - beta * p2[q];
-            p2[q] = p1[q];
-            p1[q] = pl;
-            const double base = pl;  // N_lm c_lm is folded into the table
-            yp[q] = (m == 0) ? base : base * cm[q];
-            yn[q] = base * sm[q];
-          }
-          // (a run-time l range, one bit per l of a scalar, tested where it is used:
-          // the opaque copy keeps the tests from being hoisted and carried as lane
-          // masks, and the branches keep the table reads from being hoisted en masse,
-          // which would spill at 1024 threads; the rows are addressed from lm = 0, so
-          // every read's offset is a compile-time immediate)
-          unsigned lb = lbits;
-          asm volatile("" : "+s"(lb));
-          if ((__builtin_amdgcn_readfirstlane(lb) >> l) & 1u) {
-            const int ip = (l * l + l + m) * 2;
-            const int in = (l * l + l - m) * 2;
-            // 16-byte {y, D} pairs (the table and its rows start on 16-byte boundaries)
-            const double2 t0p = *reinterpret_cast<const double2*>(T0 + ip);
-            const double2 t1p = *reinterpret_cast<const double2*>(T1 + ip);
-            const double a0 = t0p.x, a1 = t0p.y, b0 = t1p.x, b1 = t1p.y;
-            double c0 = 0.0, c1 = 0.0, e0 = 0.0, e1 = 0.0;
-            if (m > 0) {
-              const double2 t0n = *reinterpret_cast<const double2*>(T0 + in);
-              const double2 t1n = *reinterpret_cast<const double2*>(T1 + in);
-              c0 = t0n.x;
-              c1 = t0n.y;
-              e0 = t1n.x;
-              e1 = t1n.y;
-            }
-            // all of the step's table reads issued before its first use
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int q = 0; q < Q; ++q) {
-              sy0[q] += yp[q] * a0;
-              sd0[q] += yp[q] * a1;
-              sy1[q] += yp[q] * b0;
-              sd1[q] += yp[q] * b1;
-            }
-            if (m > 0) {
-#pragma unroll
-              for (int q = 0; q < Q; ++q) {
-                sy0[q] += yn[q] * c0;
-                sd0[q] += yn[q] * c1;
-                sy1[q] += yn[q] * e0;
-                sd1[q] += yn[q] * e1;
-              }
-            }
-          }
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        if (!valid[q]) continue;
-        double val;
-        if (clamp) {
-          val = sy0[q];
-        } else {
-          const double hi_ = ih[s1];
-          const double t = tq[q];
-          const double dy = (sy1[q] - sy0[q]) * hi_;
-          const double c = hi_ * (3.0 * dy - 2.0 * sd0[q] - sd1[q]);
-          const double d = hi_ * hi_ * (-2.0 * dy + sd0[q] + sd1[q]);
-          val = sy0[q] + sd0[q] * t + c * t * t + d * t * t * t;
-        }
-        vbuf[eq[q]] = val * rinv[q];
-      }
-    }
-    // every point of the item has its slot: write the potentials in point order
-    __syncthreads();
-    double* out = A.vpart + A.vbase[k] + pb;
-    for (int e = threadIdx.x; e < npt; e += blockDim.x) out[e] = A.accumulate ? out[e] + vbuf[e] : vbuf[e];
-    __syncthreads();
+              fma_scalar(S[q][c & 3], b[q][c >> 2], v);
+          });
+        });
+      });
+    });
+    static_for<0, Q>([&](auto q) {
+      const double c2 = m > 0 ? cm[q] * x[q] - sm[q] * y[q] : x[q];
+      sm[q] = m > 0 ? sm[q] * x[q] + cm[q] * y[q] : y[q];
+      cm[q] = c2;
+    });
+  });
+  static_for<0, Q>([&](auto q) {
+    out[q] = __fma_rn(__fma_rn(__fma_rn(S[q][3], t[q], S[q][2]), t[q], S[q][1]), t[q], S[q][0]);
+  });
+}
+
+// Potential of atom k's expansion at the points of one item.  A wave takes tasks of
+// up to kTaskPts points that share their spline interval, so the interval's
+// coefficients are wave-uniform: they come through the scalar cache and enter the
+// multiply-adds as scalar operands, with no LDS or vector-register traffic.
+template <int LMAX>
+__global__ __launch_bounds__(kCrossThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_hartree_cross(
+    CrossArgs A) {
+  extern __shared__ double vbuf[];  // potentials by offset in the item
+  const CrossItem it = A.items[blockIdx.x];
+  const long vb = A.vbase[it.k] + ((long)it.cell * A.nrad + it.i0) * A.nang;
+  const unsigned short* pm = A.perm + vb;
+  const unsigned* tk = A.task + (long)blockIdx.x * A.maxt;
+  const int nt = A.ntask[blockIdx.x];
+  const int lane = threadIdx.x & 63;
+  const double* rad = A.rad + it.i0;
+  const double* coef = A.coef + (long)it.k * (A.nrad + 1) * (4 * (LMAX + 1) * (LMAX + 1));
+  const double Dx = A.atoms[4 * it.cell] - A.atoms[4 * it.k], Dy = A.atoms[4 * it.cell + 1] - A.atoms[4 * it.k + 1],
+               Dz = A.atoms[4 * it.cell + 2] - A.atoms[4 * it.k + 2];
+  auto points = [&](auto Q, int s, int last, int key) {
+    double x[Q], y[Q], z[Q], t[Q], v[Q];
+    int e[Q];
+    const double x0 = A.knots[max(key - 1, 0)];
+    static_for<0, Q>([&](auto q) {
+      e[q] = pm[s + min(lane + 64 * q, last)];
+      // shell of the item and angular point: e < 4096, exact in FP32 with the half-step offset
+      const int sl = (int)(((float)e[q] + 0.5f) * A.inv_nang);
+      const int j = e[q] - sl * A.nang;
+      const double rs = rad[sl];
+      x[q] = __fma_rn(A.leb[4 * j], rs, Dx);
+      y[q] = __fma_rn(A.leb[4 * j + 1], rs, Dy);
+      z[q] = __fma_rn(A.leb[4 * j + 2], rs, Dz);
+      // r and 1/r from the hardware reciprocal square root (about 2^-26) and two
+      // coupled Newton steps
+      const double r2 = x[q] * x[q] + y[q] * y[q] + z[q] * z[q];
+      double h = __builtin_amdgcn_rsq(r2), r = r2 * h;
+      h *= 0.5;
+      double d = __fma_rn(-r, h, 0.5);
+      r = __fma_rn(r, d, r);
+      h = __fma_rn(h, d, h);
+      d = __fma_rn(-r, h, 0.5);
+      r = __fma_rn(r, d, r);
+      const double ri = 2.0 * __fma_rn(h, d, h);
+      x[q] *= ri;
+      y[q] *= ri;
+      z[q] *= ri;
+      t[q] = r - x0;
+      vbuf[e[q]] = ri;  // waits in the point's own slot (lanes past the end repeat the last point)
+    });
+    cross_eval<LMAX, Q>(coef + key * (4 * (LMAX + 1) * (LMAX + 1)), x, y, z, t, v);
+    static_for<0, Q>([&](auto q) {
+      if (lane + 64 * q <= last) vbuf[e[q]] *= v[q];
+    });
+  };
+  for (int t = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); t < nt; t += kCrossThreads / 64) {
+    const unsigned T = __builtin_amdgcn_readfirstlane(tk[t]);
+    const int s = T & 4095, last = (T >> 12) & 127, key = T >> 19;
+    if (last >= 64)
+      points(std::integral_constant<int, 2>{}, s, last, key);
+    else
+      points(std::integral_constant<int, 1>{}, s, last, key);
   }
+  __syncthreads();
+  const int len = it.nshell * A.nang;
+  for (int e = threadIdx.x; e < len; e += kCrossThreads) A.vpart[vb + e] = vbuf[e];
 }
 
 // V[p] = sum_k (k == own ? vcell[p] : vpart_k[p]) over the atoms k of the
@@ -2734,8 +2709,6 @@ struct dg_handle {
   long nlda_blocks = 0;
   double zsum = 0.0, xfac = 0.0;
   VwnConst vwn{};
-  std::vector<std::pair<int, int>> lchunks;  // l ranges of the cross kernel
-  size_t cross_lds = 0;
   // device buffers
   double *atoms = nullptr, *invR = nullptr, *rad = nullptr, *wrad = nullptr, *leb = nullptr;
   double *px = nullptr, *py = nullptr, *pz = nullptr, *w = nullptr, *wb = nullptr;
@@ -2752,12 +2725,14 @@ struct dg_handle {
   double *knots = nullptr, *invh = nullptr, *KD = nullptr;
   double *rho_lm = nullptr, *U = nullptr, *tab = nullptr;
   int* blocks = nullptr;
-  int* items = nullptr;
-  unsigned short* perm = nullptr;  // per item, point order by distance to the item's atom (padded)
-  unsigned short* pkey = nullptr;  // interval key of every perm slot
-  int* plen = nullptr;             // per item, padded length of its order
-  long npairs = 0;                 // capacity of perm
-  int nitems = 0, cross_wgs = 0;
+  // cross-atom potentials: work items, their points by spline interval, their tasks
+  CrossItem* items = nullptr;
+  unsigned short* perm = nullptr;
+  unsigned* task = nullptr;
+  int* ntask = nullptr;
+  int nitems = 0, max_tasks = 0, item_pts = 0;
+  double *coef = nullptr, *mono = nullptr;
+  int4* coef_grp = nullptr;
   // screening masks
   double screen = 0.0;
   unsigned* bmask = nullptr;
@@ -2777,7 +2752,7 @@ struct dg_handle {
   long packed = 0;  // sum of nbf_m^2
   std::vector<int> h_mol_atom0, h_mol_nbf;
   std::vector<long> h_mol_poff;
-  size_t items_cap = 0, bchunks_cap = 0;
+  size_t items_cap = 0, task_cap = 0, bchunks_cap = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   const void* graph_key[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -2802,10 +2777,10 @@ struct dg_handle {
                       V,     vcell, vpart, q,      qc,    exc_part, scalars, ylm, minvT, shc,
                       knots, invh,  KD,    rho_lm, U,     tab,  cpart, J,   XC,
                       adj_ub, adj_ab, adj_udp, adj_T, adj_frag, adj_part, adj_mot, adj_lam, adj_out, adj_dP,
-                      mol_z, mol_fac, mol_qraw, atom_exc, atom_ej, qpart, uG};
+                      mol_z, mol_fac, mol_qraw, atom_exc, atom_ej, qpart, uG, coef, mono};
     for (double* b : bufs)
       if (b) (void)hipFree(b);
-    int* ibufs[] = {sh_atom, sh_L, sh_nprim, sh_off, sh_cgf, blocks, items, plen, ash_start, ash_list, adj_list, adj_loff,
+    int* ibufs[] = {sh_atom, sh_L, sh_nprim, sh_off, sh_cgf, blocks, ntask, ash_start, ash_list, adj_list, adj_loff,
                     atom_mol, mol_atom0, mol_shell0, mol_nbf, bchunks, mol_chunk0,
                     tb[0].cb, tb[0].groups, tb[0].list, tb[0].loff, tb[1].cb, tb[1].groups, tb[1].list,
                     tb[1].loff};
@@ -2815,7 +2790,9 @@ struct dg_handle {
       if (t.order) (void)hipFree(t.order);
     if (vbase) (void)hipFree(vbase);
     if (perm) (void)hipFree(perm);
-    if (pkey) (void)hipFree(pkey);
+    if (items) (void)hipFree(items);
+    if (task) (void)hipFree(task);
+    if (coef_grp) (void)hipFree(coef_grp);
     if (mol_poff) (void)hipFree(mol_poff);
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (graph) (void)hipGraphDestroy(graph);
@@ -2889,12 +2866,13 @@ void tile_block_lists(const std::vector<unsigned>& mk, const std::vector<int>& c
   }
 }
 
-// Orders the points of every cross-potential item by distance to its atom.
+// Groups the points of every cross-potential item by spline interval.
 int sort_items(dg_handle* h) {
   if (h->nitems == 0) return DG_OK;
   return run(h, "sort_items", [&] {
-    hipLaunchKernelGGL(k_sort_items, dim3(h->nitems), dim3(1024), 0, h->stream, h->items, h->atoms, h->px, h->py,
-                       h->pz, h->knots, h->nrad, h->perm, h->pkey, h->plen);
+    hipLaunchKernelGGL(k_sort_items, dim3(h->nitems), dim3(kCrossThreads), 3 * sizeof(int) * (h->nrad + 1), h->stream,
+                       h->items, h->atoms, h->px, h->py, h->pz, h->knots, h->vbase, h->nrad, h->nang, h->max_tasks,
+                       h->perm, h->task, h->ntask);
   });
 }
 
@@ -3066,20 +3044,6 @@ int stage_correct(dg_handle* h) {
   return DG_OK;
 }
 
-// points per thread of the cross-potential kernel (a work-group pass covers 1024 kCrossQ slots)
-constexpr int kCrossQ = 2;
-
-template <int L>
-void launch_cross_l(dg_handle* h, CrossArgs& a, dim3 grid) {
-  hipLaunchKernelGGL((k_hartree_cross<L, kCrossQ>), grid, dim3(1024), h->cross_lds, h->stream, a);
-}
-
-template <int L>
-hipError_t allow_cross_lds(size_t bytes) {
-  return hipFuncSetAttribute((const void*)k_hartree_cross<L, kCrossQ>,
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-}
-
 // NT lm tiles per block: all of them up to lmax 8 (81 functions), else two
 // groups; one per block when the (atom, shell tile) blocks would not fill the CUs.
 void launch_rho_lm(dg_handle* h, int ti) {
@@ -3097,23 +3061,13 @@ void launch_rho_lm(dg_handle* h, int ti) {
 #undef DG_RHO
 }
 
-hipError_t allow_cross_lds_l(int lmax, size_t bytes) {
-  switch (lmax) {
-#define DG_L(N) \
-  case N:       \
-    return allow_cross_lds<N>(bytes);
-    DG_L(0) DG_L(1) DG_L(2) DG_L(3) DG_L(4) DG_L(5) DG_L(6) DG_L(7) DG_L(8) DG_L(9) DG_L(10) DG_L(11) DG_L(12)
-#undef DG_L
-    default:
-      return hipErrorInvalidValue;
-  }
-}
-
-void launch_cross(dg_handle* h, CrossArgs& a, dim3 grid) {
+void launch_cross(dg_handle* h, const CrossArgs& a) {
+  const dim3 grid(h->nitems), block(kCrossThreads);
+  const size_t lds = sizeof(double) * h->item_pts;
   switch (h->lmax) {
-#define DG_L(N)                    \
-  case N:                          \
-    launch_cross_l<N>(h, a, grid); \
+#define DG_L(N)                                                             \
+  case N:                                                                   \
+    hipLaunchKernelGGL(k_hartree_cross<N>, grid, block, lds, h->stream, a); \
     break;
     DG_L(0) DG_L(1) DG_L(2) DG_L(3) DG_L(4) DG_L(5) DG_L(6) DG_L(7) DG_L(8) DG_L(9) DG_L(10) DG_L(11) DG_L(12)
 #undef DG_L
@@ -3133,36 +3087,16 @@ int stage_hartree(dg_handle* h) {
   }));
   DG_TRY(run(h, "vcell", [&] {
     const long ntiles = (long)h->natoms * ti * ((h->nang + 15) / 16);
-    hipLaunchKernelGGL(k_vcell, dim3(nblocks(ntiles, 4)), dim3(256), 0, h->stream, h->U, h->ylm, h->rad, h->nrad,
-                       h->nang, h->nlm, ntiles, h->vcell);
+    const int nvb = (int)nblocks(ntiles, 4);
+    CoefArgs c{h->tab, h->invh, h->mono, h->coef_grp, h->nrad, h->nlm, h->lmax, 0, h->coef};
+    if (h->nitems > 0) c.total = (long)h->natoms * (h->nrad + 1) * h->nlm;
+    hipLaunchKernelGGL(k_vcell_coef, dim3(nvb + nblocks(c.total, 256)), dim3(256), 0, h->stream, h->U, h->ylm,
+                       h->rad, h->nrad, h->nang, h->nlm, ntiles, h->vcell, nvb, c);
   }));
-  if (h->natoms > 1) {
-    CrossArgs a;
-    a.rad = h->rad;
-    a.leb = h->leb;
-    a.nang = h->nang;
-    a.inv_nang = 1.0 / h->nang;
-    a.inv_nrad = 1.0 / h->nrad;
-    a.atoms = h->atoms;
-    a.knots = h->knots;
-    a.invh = h->invh;
-    a.tab = h->tab;
-    a.items = h->items;
-    a.perm = h->perm;
-    a.plen = h->plen;
-    a.pkey = h->pkey;
-    a.vpart = h->vpart;
-    a.vbase = h->vbase;
-    a.nitems = h->nitems;
-    a.nrad = h->nrad;
-    a.nlm = h->nlm;
-    dim3 grid(h->cross_wgs);
-    for (size_t ci = 0; ci < h->lchunks.size(); ++ci) {
-      a.l0 = h->lchunks[ci].first;
-      a.l1 = h->lchunks[ci].second;
-      a.accumulate = ci > 0;
-      DG_TRY(run(h, "hartree_cross", [&] { launch_cross(h, a, grid); }));
-    }
+  if (h->nitems > 0) {
+    const CrossArgs a{h->rad,  h->leb,   h->atoms, h->knots, h->coef, h->items,     h->perm,         h->task,
+                      h->ntask, h->vpart, h->vbase, h->nrad,  h->nang, h->max_tasks, 1.0f / h->nang};
+    DG_TRY(run(h, "hartree_cross", [&] { launch_cross(h, a); }));
   }
   DG_TRY(run(h, "vreduce", [&] {
     hipLaunchKernelGGL(k_vreduce, dim3(nblocks(h->npts_pad, 256)), dim3(256), 0, h->stream, h->vpart,
@@ -3512,7 +3446,10 @@ struct BatchSpec {
   int nmol = 0;
   std::vector<int> mol_atom0, mol_shell0;
 };
-std::vector<int> cross_items(const dg_handle* h, int len, long* perm_len = nullptr);
+constexpr int kItemCandidates[] = {1024, 2048, 4096};  // points per cross-potential item
+int cross_item_pts(const dg_handle* h, int len);
+int cross_item_len(const dg_handle* h);
+std::vector<CrossItem> cross_items(const dg_handle* h, int len);
 int batch_alloc(dg_handle* h, const BatchSpec* bs, const std::vector<int>& amol);
 int batch_setup(dg_handle* h);
 
@@ -3707,27 +3644,27 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
     h->tb[q].ncb = (int)cbs[q].size() / 4;
   }
   h->nlda_blocks = h->npts_pad / 256;
-  // cross kernel: l ranges whose spline table fits in LDS beside an item's potentials
-  {
-    const size_t limit = 150 * 1024;
-    auto bytes = [&](int l0, int l1) {
-      return (size_t)(2 * h->nrad + (size_t)h->nrad * (l1 * l1 - l0 * l0) * 2 + kMaxItem) * sizeof(double);
-    };
-    int l0 = 0;
-    size_t maxb = 0;
-    while (l0 <= h->lmax) {
-      int l1 = l0 + 1;
-      if (bytes(l0, l1) > limit)
-        return fail(DG_ERR_UNSUPPORTED, "dg_create: radial grid too large for the Hartree kernel");
-      while (l1 <= h->lmax && bytes(l0, l1 + 1) <= limit) ++l1;
-      h->lchunks.push_back({l0, l1});
-      maxb = std::max(maxb, bytes(l0, l1));
-      l0 = l1;
-    }
-    h->cross_lds = maxb;
+  // radial grids up to this size are taken (one l's spline table within 150 KB)
+  if ((2 * h->nrad + (size_t)h->nrad * (2 * h->lmax + 1) * 2 + kMaxItem) * sizeof(double) > 150 * 1024)
+    return fail(DG_ERR_UNSUPPORTED, "dg_create: radial grid too large for the Hartree kernel");
+  // groups of the cross-potential coefficients, in the order the kernel reads them, and the monomial coefficients of the harmonics' polynomials in cos(theta)
+  std::vector<int> cgrp;
+  const int L1 = h->lmax + 1;
+  std::vector<double> mono((size_t)L1 * L1 * L1, 0.0);
+  for (int m = 0, off = 0; m <= h->lmax; ++m) {
+    for (int i = 0; i <= h->lmax - m; ++i)
+      for (int sign = 0; sign < (m ? 2 : 1); ++sign, off += 4) cgrp.insert(cgrp.end(), {m, i, sign, off});
+    double lead = 1.0;  // (-1)^m (2m-1)!!
+    for (int k = 1; k <= m; ++k) lead *= -(2.0 * k - 1.0);
+    for (int l = m; l <= h->lmax; ++l)
+      for (int i = 0; i <= l - m; ++i) {
+        double v = l == m ? lead : (i > 0 ? mono[((size_t)(l - 1) * L1 + m) * L1 + i - 1] : 0.0);
+        if (l >= m + 2)
+          v -= (double)(l + m - 1) / (double)(l - m) * legendre_scale(l - 2, m) / legendre_scale(l, m) *
+               mono[((size_t)(l - 2) * L1 + m) * L1 + i];
+        mono[((size_t)l * L1 + m) * L1 + i] = v;
+      }
   }
-  // cross-potential work list: point ranges of at most 4096 (two work-group passes)
-  // outside each cell; fewer, longer items spend less of the kernel between items
   std::vector<long> vbase(h->natoms);
   long vtotal = 0;
   if (bs) {
@@ -3743,14 +3680,19 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
     for (int k = 0; k < h->natoms; ++k) vbase[k] = (long)k * h->npts_pad;
     vtotal = (long)h->natoms * h->npts_pad;
   }
-  std::vector<int> items = cross_items(h, 2048 * kCrossQ, &h->npairs);
-  h->nitems = (int)items.size() / 4;
-  h->items_cap = std::max<size_t>(items.size(), 4);
-  if (bs) {  // the batch autotuner may split the items down to 1024 points
-    long cap = 0;
-    h->items_cap = std::max(h->items_cap, cross_items(h, 1024, &cap).size());
-    h->npairs = std::max(h->npairs, cap);
-  }
+  h->item_len = cross_item_len(h);
+  std::vector<CrossItem> items = cross_items(h, h->item_len);
+  h->nitems = (int)items.size();
+  h->items_cap = std::max<size_t>(items.size(), 1);
+  h->task_cap = h->items_cap * cross_max_tasks(cross_item_pts(h, h->item_len), h->nrad);
+  if (bs)  // room for the item lengths the batch autotuner tries
+    for (int len : kItemCandidates) {
+      const size_t n = cross_items(h, len).size();
+      h->items_cap = std::max(h->items_cap, n);
+      h->task_cap = std::max(h->task_cap, n * cross_max_tasks(cross_item_pts(h, len), h->nrad));
+    }
+  h->item_pts = cross_item_pts(h, h->item_len);
+  h->max_tasks = cross_max_tasks(h->item_pts, h->nrad);
   // host-side checks and tables are done: from here on the device is used
   HIP_TRY(hipGetDevice(&h->device));
   HIP_TRY(hipStreamCreate(&h->stream));
@@ -3761,9 +3703,6 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
     // small contraction: exactly one round of resident work-groups (two per CU);
     // a partial second round measured slower, and so did fewer splits
     h->nsplit_small = (int)std::max(1L, std::min(2L * cus, h->npts_pad / 256));
-    const size_t lds = h->cross_lds;
-    const int per_cu = std::max(1, (int)((160 * 1024) / std::max<size_t>(lds, 1)));
-    h->cross_wgs = std::max(1, std::min(h->nitems, cus * std::min(per_cu, 2)));
     // 2-D contraction: splits per tile block such that the work-groups make about
     // three rounds of the resident slots (3 FP64 / 2 FP32 work-groups per CU); with
     // the longest blocks first, the short ones even out the last round (C30H62: one
@@ -3839,9 +3778,12 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
   DG_TRY(dalloc(&h->tab, (size_t)h->natoms * h->nrad * h->nlm * 2));
   DG_TRY(dalloc(&h->blocks, blocks.size()));
   DG_TRY(dalloc(&h->items, h->items_cap));
-  DG_TRY(dalloc(&h->plen, h->items_cap / 4));
-  HIP_TRY(hipMalloc((void**)&h->perm, std::max<long>(h->npairs, 1) * sizeof(unsigned short)));
-  HIP_TRY(hipMalloc((void**)&h->pkey, std::max<long>(h->npairs, 1) * sizeof(unsigned short)));
+  DG_TRY(dalloc(&h->ntask, h->items_cap));
+  DG_TRY(dalloc(&h->task, h->task_cap));
+  DG_TRY(dalloc(&h->perm, h->nitems > 0 ? (size_t)vtotal : 1));
+  DG_TRY(dalloc(&h->coef, h->nitems > 0 ? (size_t)h->natoms * (h->nrad + 1) * h->nlm * 4 : 1));
+  DG_TRY(dalloc(&h->mono, mono.size()));
+  DG_TRY(dalloc(&h->coef_grp, cgrp.size() / 4));
   // partials: two outputs of the 4 x 2 blocks, one of the 4 x 4 blocks
   DG_TRY(dalloc(&h->cpart, std::max({(size_t)h->nsplit_small * h->ngroups * 2 * 1024,
                                       (size_t)h->tb[0].nsplit * h->tb[0].ncb * 4 * 2 * 1024,
@@ -3886,7 +3828,9 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
     HIP_TRY(up(h->tb[q].cb, cbs[q].data(), cbs[q].size() * 4));
     HIP_TRY(up(h->tb[q].groups, cbg[q].data(), cbg[q].size() * 4));
   }
-  if (!items.empty()) HIP_TRY(up(h->items, items.data(), items.size() * 4));
+  if (!items.empty()) HIP_TRY(up(h->items, items.data(), items.size() * sizeof(CrossItem)));
+  HIP_TRY(up(h->mono, mono.data(), mono.size() * 8));
+  HIP_TRY(up(h->coef_grp, cgrp.data(), cgrp.size() * 4));
   HIP_TRY(hipMemsetAsync(h->phi, 0, (size_t)(np + 1) * h->ldphi * 8, h->stream));
   HIP_TRY(up(h->vbase, vbase.data(), vbase.size() * 8));
   HIP_TRY(hipMemsetAsync(h->vpart, 0, (size_t)vtotal * 8, h->stream));
@@ -3894,7 +3838,6 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
   HIP_TRY(hipMemsetAsync(h->vcell, 0, (size_t)np * 8, h->stream));
   HIP_TRY(hipMemsetAsync(h->scalars, 0, 4 * 8 * (size_t)std::max(1, h->nmol), h->stream));
 
-  HIP_TRY(allow_cross_lds_l(h->lmax, h->cross_lds));
   if (!bs) {
     if ((size_t)h->natoms * 64 * 8 > 160 * 1024)
       return fail(DG_ERR_UNSUPPORTED, "dg_create: too many atoms for the Becke kernel's LDS");
