@@ -22,11 +22,11 @@
 #include <memory>
 #include <mutex>
 #include <string>
-#include <type_traits>
 #include <vector>
 
 #include "../../include/dftgrid.h"
 #include "grid_tables.h"
+#include "unroll.h"
 
 namespace {
 
@@ -42,6 +42,8 @@ int fail(int code, const std::string& msg) {
 void dg::set_last_error(const std::string& msg) { g_last_error = msg; }
 
 namespace {
+
+using dg::static_for;
 
 #define HIP_TRY(expr)                                                                      \
   do {                                                                                     \
@@ -1133,15 +1135,6 @@ struct CrossArgs {
 // sums into copies and moves coefficients into vector registers first).
 __device__ __forceinline__ void fma_scalar(double& s, double v, double c) {
   asm volatile("v_fma_f64 %0, %1, %2, %0" : "+v"(s) : "v"(v), "s"(c));
-}
-
-// f(B), f(B+1), ..., f(E-1) with compile-time arguments (std::integral_constant).
-template <int B, int E, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (B < E) {
-    f(std::integral_constant<int, B>{});
-    static_for<B + 1, E>(f);
-  }
 }
 
 // N wave-uniform doubles read in order through the scalar cache, kChunk at a time.
