@@ -70,6 +70,39 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// v of the lane that the DPP control selects, 0 where the row mask is off.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_move(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+  return __longlong_as_double((long long)hi << 32 | (unsigned)lo);
+}
+
+// Wave-level sum in a fixed order, valid in lane 63: the DPP moves stay in the vector
+// unit, where a shuffle goes through LDS and its latency.
+__device__ __forceinline__ double wave_total(double v) {
+  v += dpp_move<0xB1, 0xf>(v);   // quad_perm [1, 0, 3, 2]
+  v += dpp_move<0x4E, 0xf>(v);   // quad_perm [2, 3, 0, 1]
+  v += dpp_move<0x141, 0xf>(v);  // row_half_mirror
+  v += dpp_move<0x140, 0xf>(v);  // row_mirror: every lane holds its row's sum
+  v += dpp_move<0x142, 0xa>(v);  // row_bcast15 into rows 1 and 3
+  v += dpp_move<0x143, 0xc>(v);  // row_bcast31 into rows 2 and 3
+  return v;
+}
+
+// 1/sqrt(x) and 1/x from the hardware estimates (about 2^-26) and Newton steps.
+__device__ __forceinline__ double rsqrt64(double x) {
+  double y = __builtin_amdgcn_rsq(x);
+  for (int k = 0; k < 2; ++k) y = y * __fma_rn(-0.5 * x * y, y, 1.5);
+  return y;
+}
+__device__ __forceinline__ double rcp64(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  for (int k = 0; k < 2; ++k) y = __fma_rn(y, __fma_rn(-x, y, 1.0), y);
+  return y;
+}
+
 constexpr int kMaxL = 12;  // largest lmax compiled
 constexpr double kPiD = 3.14159265358979323846;
 
@@ -2020,8 +2053,7 @@ constexpr double kShellReach = 100.0;
 // each taking every fourth shell; the bits are OR-ed over the block.
 __global__ __launch_bounds__(256) void k_tile_mask(const double* __restrict__ atoms, int nshell,
                                                    const int* __restrict__ sh_atom, const int* __restrict__ sh_L,
-                                                   const int* __restrict__ sh_nprim, const int* __restrict__ sh_off,
-                                                   const int* __restrict__ sh_cgf, const double* __restrict__ alpha,
+                                                   const int* __restrict__ sh_cgf, const double* __restrict__ sh_amin,
                                                    long npts, const double* __restrict__ px,
                                                    const double* __restrict__ py, const double* __restrict__ pz,
                                                    unsigned* mask) {
@@ -2035,9 +2067,7 @@ __global__ __launch_bounds__(256) void k_tile_mask(const double* __restrict__ at
       const int a = sh_atom[s];
       const double dx = x - atoms[4 * a], dy = y - atoms[4 * a + 1], dz = z - atoms[4 * a + 2];
       const double r2 = dx * dx + dy * dy + dz * dz;
-      double amin = alpha[sh_off[s]];
-      for (int k = 1; k < sh_nprim[s]; ++k) amin = fmin(amin, alpha[sh_off[s] + k]);
-      if (amin * r2 <= 1.01 * kShellReach) {
+      if (sh_amin[s] * r2 <= 1.01 * kShellReach) {
         const int L = sh_L[s], i0 = sh_cgf[s], i1 = i0 + (L + 1) * (L + 2) / 2 - 1;
         for (int t = i0 >> 4; t <= (i1 >> 4); ++t) m |= 1u << t;
       }
@@ -2058,8 +2088,8 @@ __global__ __launch_bounds__(256) void k_tile_mask(const double* __restrict__ at
 __global__ __launch_bounds__(64) void k_force_basis(
     const double* __restrict__ atoms, int natoms, const int* __restrict__ ash_start,
     const int* __restrict__ ash_list, const int* __restrict__ sh_L, const int* __restrict__ sh_nprim,
-    const int* __restrict__ sh_off, const int* __restrict__ sh_cgf, const double* __restrict__ alpha,
-    const double* __restrict__ cn0, const double* __restrict__ cn1, long npts,
+    const int* __restrict__ sh_off, const int* __restrict__ sh_cgf, const double* __restrict__ sh_amin,
+    const double* __restrict__ alpha, const double* __restrict__ cn0, const double* __restrict__ cn1, long npts,
     const double* __restrict__ px, const double* __restrict__ py, const double* __restrict__ pz,
     int ldphi, const double* __restrict__ tmat, const double* __restrict__ ub, long nblk, double* part,
     double* mot) {
@@ -2078,18 +2108,18 @@ __global__ __launch_bounds__(64) void k_force_basis(
         const int s = ash_list[t];
         // every primitive's exp(-alpha r2) below e^-kShellReach (1e-43): the shell's
         // terms are below the rounding of the sums they would enter, and it is skipped
-        double amin = alpha[sh_off[s]];
-        for (int k = 1; k < sh_nprim[s]; ++k) amin = fmin(amin, alpha[sh_off[s] + k]);
-        if (amin * r2 > kShellReach) continue;
+        if (sh_amin[s] * r2 > kShellReach) continue;
         double r0 = 0.0, d0 = 0.0, r1 = 0.0, d1 = 0.0;
         for (int k = 0; k < sh_nprim[s]; ++k) {
           const int q = sh_off[s] + k;
           const double e = exp(-alpha[q] * r2);
           const double m2a = -2.0 * alpha[q];
           r0 += cn0[q] * e;
-          r1 += cn1[q] * e;
           d0 += cn0[q] * m2a * e;
-          d1 += cn1[q] * m2a * e;
+          if (sh_L[s] == 2) {  // the xy, xz, yz functions' own norm
+            r1 += cn1[q] * e;
+            d1 += cn1[q] * m2a * e;
+          }
         }
         const int L = sh_L[s], nc = (L + 1) * (L + 2) / 2;
         for (int c = 0; c < nc; ++c) {
@@ -2104,8 +2134,8 @@ __global__ __launch_bounds__(64) void k_force_basis(
     }
     for (int d = 0; d < 3; ++d) {
       G[d] += g[d];
-      const double t = wave_sum(g[d]);
-      if (threadIdx.x == 0) part[((long)A * 3 + d) * nblk + blockIdx.x] = -4.0 * t;
+      const double t = wave_total(g[d]);
+      if (threadIdx.x == 63) part[((long)A * 3 + d) * nblk + blockIdx.x] = -4.0 * t;
     }
   }
   if (valid)
@@ -2243,19 +2273,20 @@ __global__ __launch_bounds__(256) void k_density_grad(
 // dP_n/dR_B = P_n sum_m (s'/s)(mu_nm) d mu_nm/d R_B with
 // d mu_nm/d R_n = -(u_n + mu_nm e_nm)/R_nm, d mu_nm/d R_m = (u_m + mu_nm e_nm)/R_nm,
 // u_k = (r - R_k)/|r - R_k|, e_nm = (R_n - R_m)/R_nm.
-__device__ __forceinline__ void cutoff_and_ratio(double mu, double& s, double& ratio) {
-  // s = (1 - f(f(f(mu))))/2, s' = -f'(f2) f'(f1) f'(mu)/2, f'(x) = 1.5 - 1.5 x^2
-  const double f1 = 1.5 * mu - 0.5 * mu * mu * mu;
-  const double f2 = 1.5 * f1 - 0.5 * f1 * f1 * f1;
-  const double f3 = 1.5 * f2 - 0.5 * f2 * f2 * f2;
-  s = 0.5 * (1.0 - f3);
-  const double sp = -0.5 * (1.5 - 1.5 * f2 * f2) * (1.5 - 1.5 * f1 * f1) * (1.5 - 1.5 * mu * mu);
-  ratio = (s > 0.0) ? sp / s : 0.0;
+// The ratio s'/s of the cutoff s = (1 - f(f(f(mu))))/2, s' = -f'(f2) f'(f1) f'(mu)/2,
+// f'(x) = 1.5 - 1.5 x^2; 0 where s rounds to 0.
+__device__ __forceinline__ double cutoff_ratio(double mu) {
+  const double m2 = mu * mu, f1 = mu * __fma_rn(-0.5, m2, 1.5);
+  const double q1 = f1 * f1, f2 = f1 * __fma_rn(-0.5, q1, 1.5);
+  const double q2 = f2 * f2, f3 = f2 * __fma_rn(-0.5, q2, 1.5);
+  const double s = __fma_rn(-0.5, f3, 0.5);
+  const double sp = -1.6875 * (__fma_rn(-f1, f1, 1.0) * __fma_rn(-f2, f2, 1.0) * __fma_rn(-mu, mu, 1.0));
+  return s > 0.0 ? sp * rcp64(s) : 0.0;
 }
 
 __device__ __forceinline__ double becke_s(double mu) {
-  for (int it = 0; it < 3; ++it) mu = 1.5 * mu - 0.5 * (mu * mu * mu);
-  return 0.5 * (1.0 - mu);
+  for (int it = 0; it < 3; ++it) mu = mu * __fma_rn(-0.5, mu * mu, 1.5);
+  return __fma_rn(-0.5, mu, 0.5);
 }
 
 // Terms of an atom n whose cell function P_n is at most kBeckeSkip times
@@ -2270,12 +2301,15 @@ constexpr double kBeckeSkip = 1e-20;
 // caller reports the gradient as unsupported.
 constexpr int kBeckeActive = 24;
 
-// Active entries per pass of the Becke-term loops (held in registers).
-constexpr int kBeckeBlock = 8;
+// Active entries per pass of the Becke-term loops (held in registers).  Six leave two
+// waves per SIMD; with eight the branch-free pair loop takes over 256 registers and one
+// wave (C30H62 18.5 ms against 10.2; eight forced to two waves 11.3, four 11.6).
+constexpr int kBeckeBlock = 6;
 
 __device__ __forceinline__ double atom_dist(const double* __restrict__ atoms, int m, double x, double y, double z) {
   const double dx = x - atoms[4 * m], dy = y - atoms[4 * m + 1], dz = z - atoms[4 * m + 2];
-  return fmax(sqrt(dx * dx + dy * dy + dz * dz), 1e-300);
+  const double d2 = fmax(dx * dx + dy * dy + dz * dz, 1e-300);
+  return d2 * rsqrt64(d2);
 }
 
 // Cell function P_n at the point, its factors taken with the nearest atom
@@ -2293,8 +2327,36 @@ __device__ __forceinline__ double cell_function(const double* __restrict__ atoms
   return prod;
 }
 
+// order[a natoms + r]: the r-th nearest atom to atom a (itself first).
+__global__ __launch_bounds__(256) void k_atom_order(const double* __restrict__ atoms, int natoms, int* order) {
+  const long e = (long)blockIdx.x * 256 + threadIdx.x;
+  if (e >= (long)natoms * natoms) return;
+  const int a = (int)(e / natoms), m = (int)(e % natoms);
+  auto d2 = [&](int k) {
+    const double dx = atoms[4 * k] - atoms[4 * a], dy = atoms[4 * k + 1] - atoms[4 * a + 1],
+                 dz = atoms[4 * k + 2] - atoms[4 * a + 2];
+    return dx * dx + dy * dy + dz * dz;
+  };
+  const double d = d2(m);
+  int rank = 0;
+  for (int k = 0; k < natoms; ++k) {
+    const double x = d2(k);
+    rank += (x < d || (x == d && k < m)) ? 1 : 0;
+  }
+  order[(long)a * natoms + rank] = m;
+}
+
+// Bound by the FP64 vector unit: per point, the cell functions (phase 1) and one ratio
+// s'/s per (active cell, atom) pair (phase 2).  C30H62, 2.08 M points: 18.1 -> 10.3 ms,
+// benzene 278 -> 170 us, by (a) dropping points whose owner's cell function is itself
+// below the skip level (every term of theirs carries it), (b) taking the factors of a cell
+// function nearest atom of the owner first, so that a vanishing product ends after a few
+// factors, (c) sums per atom and per cell of the two scalars f and f mu / R (and the latter
+// times one vector) instead of two vectors per pair, Newton reciprocals and DPP wave sums,
+// (d) the sums in LDS and (e) a pair loop without branches.
 __global__ __launch_bounds__(64) void k_force_becke(const double* __restrict__ atoms,
-                                                    const double* __restrict__ invR, int natoms,
+                                                    const double* __restrict__ invR,
+                                                    const int* __restrict__ order, int natoms,
                                                     long npts, long cell, int nrad, int nang,
                                                     const double* __restrict__ rad,
                                                     const double* __restrict__ wrad,
@@ -2308,6 +2370,9 @@ __global__ __launch_bounds__(64) void k_force_becke(const double* __restrict__ a
   // recomputed where needed: 10 bytes per entry keep ten work-groups per CU)
   __shared__ unsigned short act_n[kBeckeActive * 64];
   __shared__ double act_P[kBeckeActive * 64];
+  // the work-group's sums per atom (lane 63 adds, in program order), added to part at
+  // the end: a read-modify-write of part per sum made the kernel wait on memory
+  extern __shared__ double bsum[];  // [3 natoms]
   const int lane = threadIdx.x;
   const long p = (long)blockIdx.x * 64 + lane;
   double w0a = 0.0;  // weight without the Becke factor, times a_p
@@ -2319,17 +2384,24 @@ __global__ __launch_bounds__(64) void k_force_becke(const double* __restrict__ a
   }
   // points with |w0 a_p| <= 1e-30 (far out, where the density has vanished and
   // many cells overlap) add nothing that survives rounding and are skipped
-  const bool valid = p < npts && fabs(w0a) > 1e-30;
-  const double x = valid ? px[p] : 0.0, y = valid ? py[p] : 0.0, z = valid ? pz[p] : 0.0;
+  bool on = p < npts && fabs(w0a) > 1e-30;
+  if (__ballot(on) == 0) return;
+  const double x = on ? px[p] : 0.0, y = on ? py[p] : 0.0, z = on ? pz[p] : 0.0;
+  const int own = on ? (int)(p / cell) : 0;
   int near = 0;
-  double dnear = atom_dist(atoms, 0, x, y, z);
-  for (int m = 1; m < natoms; ++m) {
-    const double d = atom_dist(atoms, m, x, y, z);
-    if (d < dnear) {
-      dnear = d;
+  double d2near = 1e300;
+  for (int m = 0; m < natoms; ++m) {
+    const double dx = x - atoms[4 * m], dy = y - atoms[4 * m + 1], dz = z - atoms[4 * m + 2];
+    const double d2 = dx * dx + dy * dy + dz * dz;
+    if (d2 < d2near) {
+      d2near = d2;
       near = m;
     }
   }
+  // the atoms by distance from the owner of the wave's first point (one order for the
+  // wave: it only decides how soon a vanishing product is recognised)
+  const int* ord = order + (long)__builtin_amdgcn_readfirstlane((int)((long)blockIdx.x * 64 / cell)) * natoms;
+  const double dnear = atom_dist(atoms, near, x, y, z);
   // Z: the nearest atom's P is a lower bound, and a product that drops below
   // 1e-4 kBeckeSkip of it (below the skip level) is kept as truncated, which
   // changes Z by less than 1e-24 Z per atom.  The same pass lists the
@@ -2337,63 +2409,81 @@ __global__ __launch_bounds__(64) void k_force_becke(const double* __restrict__ a
   // (Z >= pnear) whose P are exact (a product above the skip level never
   // reaches the truncation); the list is then cut to the active ones.
   double pnear = 1.0, Z = 1.0, Pown = 0.0;
-  const int own = valid ? (int)(p / cell) : 0;
   int ncand = 0;
   bool cand_full = false;
-  if (valid) {
-    pnear = cell_function(atoms, invR, natoms, near, near, dnear, dnear, x, y, z, 0.0);
-    const double cut0 = 1e-4 * kBeckeSkip * pnear, pre = kBeckeSkip * pnear;
-    Z = pnear;
-    // the cell functions of kBeckeBlock atoms at a time, each factor sequence as in
-    // cell_function (the nearest atom first, then m ascending, stopped once the
-    // product is at most cut0), the distance to each atom m shared by the block
-    for (int n0 = 0; n0 < natoms; n0 += kBeckeBlock) {
-      double dn[kBeckeBlock], prod[kBeckeBlock];
-      bool alive = false;
+  {
+    double pr = 1.0;
+    for (int r = 0; r < natoms; ++r) {
+      const int m = ord[r];
+      if (m != near) pr *= becke_s((dnear - atom_dist(atoms, m, x, y, z)) * invR[near * natoms + m]);
+    }
+    pnear = pr;
+    // every term of the point carries wb = P_own / Z or the owner's own dP: with the
+    // owner's cell below the skip level there are none
+    if (on) {
+      Pown = pnear;
+      if (near != own) {
+        const double dn = atom_dist(atoms, own, x, y, z);
+        Pown = becke_s((dn - dnear) * invR[own * natoms + near]);
+        for (int r = 0; r < natoms && Pown > kBeckeSkip * pnear; ++r) {
+          const int m = ord[r];
+          if (m != own && m != near) Pown *= becke_s((dn - atom_dist(atoms, m, x, y, z)) * invR[own * natoms + m]);
+        }
+      }
+      on = Pown > kBeckeSkip * pnear;
+    }
+  }
+  if (__ballot(on) == 0) return;
+  const double cut0 = on ? 1e-4 * kBeckeSkip * pnear : 2.0, pre = on ? kBeckeSkip * pnear : 2.0;
+  Z = pnear;
+  // the cell functions of kBeckeBlock atoms at a time, each product with the nearest
+  // atom's factor first, then in the wave's order, stopped once it is at most cut0; the
+  // distance to each atom m is shared by the block
+  for (int r0 = 0; r0 < natoms; r0 += kBeckeBlock) {
+    double dn[kBeckeBlock], prod[kBeckeBlock];
+    bool alive = false;
+#pragma unroll
+    for (int k = 0; k < kBeckeBlock; ++k) {
+      const int n = ord[min(r0 + k, natoms - 1)];
+      const bool in = r0 + k < natoms && n != near;
+      dn[k] = atom_dist(atoms, n, x, y, z);
+      prod[k] = in ? becke_s((dn[k] - dnear) * invR[n * natoms + near]) : 0.0;
+      alive |= prod[k] > cut0;
+    }
+    for (int r = 0; r < natoms && __ballot(alive) != 0; ++r) {
+      const int m = ord[r];
+      const double dm = atom_dist(atoms, m, x, y, z);
+      alive = false;
 #pragma unroll
       for (int k = 0; k < kBeckeBlock; ++k) {
-        const int n = n0 + k;
-        const bool in = n < natoms && n != near;
-        const int ns = in ? n : near;
-        dn[k] = atom_dist(atoms, ns, x, y, z);
-        prod[k] = in ? becke_s((dn[k] - dnear) * invR[ns * natoms + near]) : 0.0;
+        const int n = ord[min(r0 + k, natoms - 1)];  // past the last atom: prod[k] = 0, no factor taken
+        if (m != n && m != near && prod[k] > cut0) prod[k] *= becke_s((dn[k] - dm) * invR[n * natoms + m]);
         alive |= prod[k] > cut0;
       }
-      for (int m = 0; m < natoms && __ballot(alive) != 0; ++m) {
-        const double dm = atom_dist(atoms, m, x, y, z);
-        alive = false;
+    }
 #pragma unroll
-        for (int k = 0; k < kBeckeBlock; ++k) {
-          const int n = min(n0 + k, natoms - 1);  // past the last atom: prod[k] = 0, no factor taken
-          if (m != n && m != near && prod[k] > cut0) prod[k] *= becke_s((dn[k] - dm) * invR[n * natoms + m]);
-          alive |= prod[k] > cut0;
-        }
+    for (int k = 0; k < kBeckeBlock; ++k) {
+      if (r0 + k >= natoms) break;
+      const int n = ord[r0 + k];
+      double P = pnear;
+      if (n != near) {
+        P = prod[k];
+        Z += P;
       }
-#pragma unroll
-      for (int k = 0; k < kBeckeBlock; ++k) {
-        const int n = n0 + k;
-        if (n >= natoms) break;
-        double P = pnear;
-        if (n != near) {
-          P = prod[k];
-          Z += P;
-        }
-        if (n == own) Pown = P;
-        if (P > pre) {
-          if (ncand < kBeckeActive) {
-            act_n[ncand * 64 + lane] = (unsigned short)n;
-            act_P[ncand * 64 + lane] = P;
-            ++ncand;
-          } else {
-            cand_full = true;
-          }
+      if (P > pre) {
+        if (ncand < kBeckeActive) {
+          act_n[ncand * 64 + lane] = (unsigned short)n;
+          act_P[ncand * 64 + lane] = P;
+          ++ncand;
+        } else {
+          cand_full = true;
         }
       }
     }
   }
   const double skip = kBeckeSkip * Z;
   int nact = 0;
-  if (!cand_full) {
+  if (on && !cand_full) {
     for (int t = 0; t < ncand; ++t) {
       const double P = act_P[t * 64 + lane];
       if (P > skip) {
@@ -2402,7 +2492,7 @@ __global__ __launch_bounds__(64) void k_force_becke(const double* __restrict__ a
         ++nact;
       }
     }
-  } else {
+  } else if (on) {
     // more candidates than slots: list the active cells from scratch
     for (int n = 0; n < natoms; ++n) {
       const double dn = (n == near) ? dnear : atom_dist(atoms, n, x, y, z);
@@ -2418,76 +2508,95 @@ __global__ __launch_bounds__(64) void k_force_becke(const double* __restrict__ a
       }
     }
   }
-  const double pref = (valid && Z > 0.0) ? w0a / Z : 0.0;
-  const double wbv = (valid && Z > 0.0) ? Pown / Z : 0.0;
-  const bool on = valid && pref != 0.0;
+  const double pref = (on && Z > 0.0) ? w0a / Z : 0.0;
+  const double wbv = (on && Z > 0.0) ? Pown / Z : 0.0;
+  on = on && pref != 0.0;
+  if (on) {  // the owner first: entry 0 of pass 0 is its share
+    for (int t = 1; t < nact; ++t)
+      if (act_n[t * 64 + lane] == own) {
+        act_n[t * 64 + lane] = act_n[lane];
+        act_n[lane] = (unsigned short)own;
+        act_P[t * 64 + lane] = act_P[lane];
+        act_P[lane] = Pown;
+      }
+  }
+  for (int e = lane; e < 3 * natoms; e += 64) bsum[e] = 0.0;
   double own_acc[3] = {0.0, 0.0, 0.0};
   // Every pair (active n, atom m != n) enters twice with the same
-  // rho = ratio(mu_nm), f = P_n rho / R_nm and e_nm: into dP_n/dR_m as
-  // f (u_m + mu e_nm), and into dP_n/dR_n as -f (u_n + mu e_nm).  Passes over
-  // kBeckeBlock active entries at a time (registers), atoms m in order: output m
-  // is complete at the end of its step; output n sums F = sum_m f and
-  // G = sum_m f mu e_nm over the pass and is added after it, as
-  // dP_n/dR_n = -(u_n F + G).  Per atom B the sums go to part[B] in a fixed order:
-  // the m terms of pass 0, the n terms of pass 0, then those of pass 1, ...
+  // rho = ratio(mu_nm), f = P_n rho / R_nm and g = f mu / R_nm: into dP_n/dR_m as
+  // f u_m + g (R_n - R_m), and into dP_n/dR_n as -(f u_n + g (R_n - R_m)).  Passes over
+  // kBeckeBlock active entries at a time (registers), atoms m in order: with
+  // w_n = R_n - r and v_m = r - R_m, output m is u_m sum f + sum g w_n + v_m sum g over
+  // the pass's n, complete at the end of its step; output n sums F = sum f, Gs = sum g and
+  // Gv = sum g v_m over m and is added after the pass, as dP_n/dR_n =
+  // -(u_n F + w_n Gs + Gv).  Per atom B the sums go to part[B] in a fixed order: the m
+  // terms of pass 0, the n terms of pass 0, then those of pass 1, ...
   int nmax = on ? nact : 0;
   for (int o = 32; o > 0; o >>= 1) nmax = max(nmax, __shfl_xor(nmax, o));
   for (int t0 = 0; t0 < nmax; t0 += kBeckeBlock) {
     int nk[kBeckeBlock];
-    double Pk[kBeckeBlock], dk[kBeckeBlock], wk[kBeckeBlock][3], F[kBeckeBlock], G[kBeckeBlock][3];
+    unsigned rk[kBeckeBlock];  // byte offset of row n of invR
+    double Pk[kBeckeBlock], dk[kBeckeBlock], wk[kBeckeBlock][3], F[kBeckeBlock], Gs[kBeckeBlock], Gv[kBeckeBlock][3];
 #pragma unroll
     for (int k = 0; k < kBeckeBlock; ++k) {
+      // no entry left: the owner again with P = 0; the pair n = m drops out through
+      // invR[n][n] = 0: no branch in the pair loop, so the entries' chains overlap
       const bool in = on && t0 + k < nact;
-      nk[k] = in ? act_n[(t0 + k) * 64 + lane] : -1;
+      nk[k] = in ? act_n[(t0 + k) * 64 + lane] : own;
       Pk[k] = in ? act_P[(t0 + k) * 64 + lane] : 0.0;
-      const int n = in ? nk[k] : 0;
-      // w = R_n - r
+      const int n = nk[k];
+      rk[k] = 8u * (unsigned)(n * natoms);
       wk[k][0] = atoms[4 * n] - x;
       wk[k][1] = atoms[4 * n + 1] - y;
       wk[k][2] = atoms[4 * n + 2] - z;
       dk[k] = atom_dist(atoms, n, x, y, z);
-      F[k] = G[k][0] = G[k][1] = G[k][2] = 0.0;
+      F[k] = Gs[k] = Gv[k][0] = Gv[k][1] = Gv[k][2] = 0.0;
     }
+    const double own_pass = t0 == 0 && nk[0] == own ? 1.0 : 0.0;  // (the owner may fall between pre and skip)
     for (int m = 0; m < natoms; ++m) {
-      const double dm = atom_dist(atoms, m, x, y, z);
-      const double vm[3] = {x - atoms[4 * m], y - atoms[4 * m + 1], z - atoms[4 * m + 2]};  // r - R_m
-      const double um[3] = {vm[0] / dm, vm[1] / dm, vm[2] / dm};
-      double S[3] = {0.0, 0.0, 0.0}, Dp[3] = {0.0, 0.0, 0.0};
+      const double vm[3] = {x - atoms[4 * m], y - atoms[4 * m + 1], z - atoms[4 * m + 2]};
+      const double d2 = fmax(vm[0] * vm[0] + vm[1] * vm[1] + vm[2] * vm[2], 1e-300);
+      const double im = rsqrt64(d2), dm = d2 * im;  // |v_m| and its inverse
+      double sf = 0.0, sg = 0.0, sw[3] = {0.0, 0.0, 0.0}, of = 0.0, og = 0.0;
 #pragma unroll
       for (int k = 0; k < kBeckeBlock; ++k) {
-        const int n = nk[k];
-        if (n < 0 || n == m) continue;
-        const double iR = invR[n * natoms + m];
+        const double iR = *reinterpret_cast<const double*>(reinterpret_cast<const char*>(invR + m) + rk[k]);
         const double mu = (dk[k] - dm) * iR;
-        double sv, rt;
-        cutoff_and_ratio(mu, sv, rt);
-        const double f = Pk[k] * rt * iR, fm = f * mu;
+        const double f = Pk[k] * cutoff_ratio(mu) * iR, g = f * mu * iR;
         F[k] += f;
+        Gs[k] += g;
+        sf += f;
+        sg += g;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-          const double me = fm * ((wk[k][d] + vm[d]) * iR);  // f mu e_nm
-          const double tv = f * um[d] + me;
-          S[d] += tv;
-          if (n == own) Dp[d] = tv;
-          G[k][d] += me;
+          sw[d] = __fma_rn(g, wk[k][d], sw[d]);
+          Gv[k][d] = __fma_rn(g, vm[d], Gv[k][d]);
+        }
+        if (k == 0) {  // the owner's share of output m, in pass 0 only
+          of = own_pass * f;
+          og = own_pass * g;
         }
       }
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        const double gm = (on && m != own) ? pref * (Dp[d] - wbv * S[d]) : 0.0;
+        const double S = sf * (vm[d] * im) + (sw[d] + vm[d] * sg);
+        const double Dp = of * (vm[d] * im) + og * (wk[0][d] + vm[d]);
+        const double gm = (on && m != own) ? pref * (Dp - wbv * S) : 0.0;
         own_acc[d] -= gm;
-        const double t = wave_sum(gm);
-        if (lane == 0) part[((long)m * 3 + d) * nblk + blockIdx.x] += t;
+        const double t = wave_total(gm);
+        if (lane == 63) bsum[3 * m + d] += t;
       }
     }
-    // the pass's entries n: d wb/dR_n gains pref wbv (u_n F + G), u_n = -w / d_n
+    // the pass's entries n: d wb/dR_n gains pref wbv (u_n F + w_n Gs + Gv), u_n = -w_n / d_n
+    bool any[kBeckeBlock];
 #pragma unroll
     for (int k = 0; k < kBeckeBlock; ++k) {
-      const bool use = nk[k] >= 0 && nk[k] != own;
+      any[k] = on && nk[k] != own;
+      const double q = Gs[k] - F[k] / dk[k];
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        G[k][d] = use ? pref * wbv * (G[k][d] - wk[k][d] / dk[k] * F[k]) : 0.0;
-        own_acc[d] -= G[k][d];
+        Gv[k][d] = any[k] ? pref * wbv * __fma_rn(wk[k][d], q, Gv[k][d]) : 0.0;
+        own_acc[d] -= Gv[k][d];
       }
     }
     for (int B = 0; B < natoms; ++B) {
@@ -2495,21 +2604,23 @@ __global__ __launch_bounds__(64) void k_force_becke(const double* __restrict__ a
       bool has = false;
 #pragma unroll
       for (int k = 0; k < kBeckeBlock; ++k)
-        if (nk[k] == B) {
+        if (any[k] && nk[k] == B) {
           has = true;
 #pragma unroll
-          for (int d = 0; d < 3; ++d) v[d] = G[k][d];
+          for (int d = 0; d < 3; ++d) v[d] = Gv[k][d];
         }
       if (__ballot(has) == 0) continue;
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        const double t = wave_sum(v[d]);
-        if (lane == 0) part[((long)B * 3 + d) * nblk + blockIdx.x] += t;
+        const double t = wave_total(v[d]);
+        if (lane == 63) bsum[3 * B + d] += t;
       }
     }
   }
+  __syncthreads();
+  for (int e = lane; e < 3 * natoms; e += 64) part[e * nblk + blockIdx.x] += bsum[e];
   // the owner atom's share (translation invariance), per point
-  if (valid)
+  if (on)
     for (int d = 0; d < 3; ++d) mot[d * npts + p] += own_acc[d];
 }
 
@@ -2707,6 +2818,7 @@ struct dg_handle {
   double *px = nullptr, *py = nullptr, *pz = nullptr, *w = nullptr, *wb = nullptr;
   double* phi = nullptr;
   int *sh_atom = nullptr, *sh_L = nullptr, *sh_nprim = nullptr, *sh_off = nullptr, *sh_cgf = nullptr;
+  double* sh_amin = nullptr;  // per shell, its smallest exponent
   double *pr_alpha = nullptr, *pr_cn0 = nullptr, *pr_cn1 = nullptr;
   double *P = nullptr, *pfrag = nullptr, *rho = nullptr, *uxc = nullptr, *exd = nullptr;
   double *uJ = nullptr, *V = nullptr, *vcell = nullptr, *vpart = nullptr;
@@ -2753,6 +2865,7 @@ struct dg_handle {
   double *adj_ub = nullptr, *adj_ab = nullptr, *adj_udp = nullptr, *adj_T = nullptr, *adj_frag = nullptr;
   double *adj_part = nullptr, *adj_mot = nullptr, *adj_lam = nullptr, *adj_out = nullptr, *adj_dP = nullptr;
   int *ash_start = nullptr, *ash_list = nullptr;
+  int* atom_order = nullptr;  // per atom, all atoms by distance
   unsigned* adj_tmask = nullptr;  // per 64-point block, the function tiles the force terms read
   int *adj_list = nullptr, *adj_loff = nullptr;  // dE/dP: point blocks per one-output tile block
   // state
@@ -2770,10 +2883,10 @@ struct dg_handle {
                       V,     vcell, vpart, q,      qc,    exc_part, scalars, ylm, minvT, shc,
                       knots, invh,  KD,    rho_lm, U,     tab,  cpart, J,   XC,
                       adj_ub, adj_ab, adj_udp, adj_T, adj_frag, adj_part, adj_mot, adj_lam, adj_out, adj_dP,
-                      mol_z, mol_fac, mol_qraw, atom_exc, atom_ej, qpart, uG, coef, mono};
+                      mol_z, mol_fac, mol_qraw, atom_exc, atom_ej, qpart, uG, coef, mono, sh_amin};
     for (double* b : bufs)
       if (b) (void)hipFree(b);
-    int* ibufs[] = {sh_atom, sh_L, sh_nprim, sh_off, sh_cgf, blocks, ntask, ash_start, ash_list, adj_list, adj_loff,
+    int* ibufs[] = {sh_atom, sh_L, sh_nprim, sh_off, sh_cgf, blocks, ntask, ash_start, ash_list, atom_order, adj_list, adj_loff,
                     atom_mol, mol_atom0, mol_shell0, mol_nbf, bchunks, mol_chunk0,
                     tb[0].cb, tb[0].groups, tb[0].list, tb[0].loff, tb[1].cb, tb[1].groups, tb[1].list,
                     tb[1].loff};
@@ -2979,7 +3092,7 @@ int ensure_tile_mask(dg_handle* h) {
   DG_TRY(dalloc(&h->adj_tmask, nblk));
   return run(h, "adj_tile_mask", [&] {
     hipLaunchKernelGGL(k_tile_mask, dim3(nblk), dim3(256), 0, h->stream, h->atoms, h->nshell, h->sh_atom, h->sh_L,
-                       h->sh_nprim, h->sh_off, h->sh_cgf, h->pr_alpha, h->npts, h->px, h->py, h->pz, h->adj_tmask);
+                       h->sh_cgf, h->sh_amin, h->npts, h->px, h->py, h->pz, h->adj_tmask);
   });
 }
 
@@ -3540,7 +3653,7 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
   h->ldphi = (int)round_up(nbf, 32);
   h->ntb = (nbf + 15) / 16;
   if (h->ntb > 32) return fail(DG_ERR_UNSUPPORTED, "dg_create: more than 512 basis functions");
-  std::vector<double> alpha(nprim_tot), cn0(nprim_tot), cn1(nprim_tot);
+  std::vector<double> alpha(nprim_tot), cn0(nprim_tot), cn1(nprim_tot), amin(h->nshell);
   for (int s = 0; s < h->nshell; ++s) {
     const int L = basis->L[s];
     for (int k = 0; k < basis->nprim[s]; ++k) {
@@ -3548,6 +3661,7 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
       const double a = basis->alpha[i], c = basis->coef[i];
       if (!(a > 0.0)) return fail(DG_ERR_INVALID, "dg_create: primitive exponent must be positive");
       alpha[i] = a;
+      amin[s] = k ? std::min(amin[s], a) : a;
       cn0[i] = c * dg::gto_norm(a, L, 0, 0);
       cn1[i] = c * dg::gto_norm(a, L == 2 ? 1 : L, L == 2 ? 1 : 0, 0);
     }
@@ -3740,6 +3854,7 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
   DG_TRY(dalloc(&h->sh_nprim, h->nshell));
   DG_TRY(dalloc(&h->sh_off, h->nshell));
   DG_TRY(dalloc(&h->sh_cgf, h->nshell));
+  DG_TRY(dalloc(&h->sh_amin, h->nshell));
   DG_TRY(dalloc(&h->pr_alpha, nprim_tot));
   DG_TRY(dalloc(&h->pr_cn0, nprim_tot));
   DG_TRY(dalloc(&h->pr_cn1, nprim_tot));
@@ -3807,6 +3922,7 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
   HIP_TRY(up(h->sh_nprim, basis->nprim, h->nshell * 4));
   HIP_TRY(up(h->sh_off, basis->offset, h->nshell * 4));
   HIP_TRY(up(h->sh_cgf, cgf_off.data(), h->nshell * 4));
+  HIP_TRY(up(h->sh_amin, amin.data(), h->nshell * 8));
   HIP_TRY(up(h->pr_alpha, alpha.data(), nprim_tot * 8));
   HIP_TRY(up(h->pr_cn0, cn0.data(), nprim_tot * 8));
   HIP_TRY(up(h->pr_cn1, cn1.data(), nprim_tot * 8));
@@ -4126,6 +4242,11 @@ int dg_xc_adjoint(dg_handle* h, int hold_c, double* dEdP, double* grad) {
         if (at[s] == a) list.push_back(s);
     }
     start[na] = (int)list.size();
+    DG_TRY(dalloc(&h->atom_order, (size_t)na * na));
+    DG_TRY(run(h, "adj_atom_order", [&] {
+      hipLaunchKernelGGL(k_atom_order, dim3(nblocks((long)na * na, 256)), dim3(256), 0, h->stream, h->atoms, na,
+                         h->atom_order);
+    }));
     DG_TRY(dalloc(&h->ash_start, na + 1));
     DG_TRY(dalloc(&h->ash_list, std::max<size_t>(list.size(), 1)));
     HIP_TRY(hipMemcpyAsync(h->ash_start, start.data(), (na + 1) * 4, hipMemcpyHostToDevice, h->stream));
@@ -4176,13 +4297,13 @@ int dg_xc_adjoint(dg_handle* h, int hold_c, double* dEdP, double* grad) {
     DG_TRY(launch_tmat(h, true));
     DG_TRY(run(h, "adj_force_basis", [&] {
       hipLaunchKernelGGL(k_force_basis, dim3(nblk), dim3(64), 0, h->stream, h->atoms, na, h->ash_start, h->ash_list,
-                         h->sh_L, h->sh_nprim, h->sh_off, h->sh_cgf, h->pr_alpha, h->pr_cn0, h->pr_cn1, h->npts,
-                         h->px, h->py, h->pz, h->ldphi, h->adj_T, h->adj_ub, nblk, h->adj_part, h->adj_mot);
+                         h->sh_L, h->sh_nprim, h->sh_off, h->sh_cgf, h->sh_amin, h->pr_alpha, h->pr_cn0, h->pr_cn1,
+                         h->npts, h->px, h->py, h->pz, h->ldphi, h->adj_T, h->adj_ub, nblk, h->adj_part, h->adj_mot);
     }));
     HIP_TRY(hipMemsetAsync(h->adj_out + 6 * na, 0, sizeof(double), h->stream));
     DG_TRY(run(h, "adj_force_becke", [&] {
-      hipLaunchKernelGGL(k_force_becke, dim3(nblk), dim3(64), 0, h->stream, h->atoms, h->invR, na, h->npts,
-                         h->cell, h->nrad, h->nang, h->rad, h->wrad, h->leb, h->px, h->py, h->pz, h->adj_ab, nblk,
+      hipLaunchKernelGGL(k_force_becke, dim3(nblk), dim3(64), 3 * sizeof(double) * na, h->stream, h->atoms, h->invR, h->atom_order, na,
+                         h->npts, h->cell, h->nrad, h->nang, h->rad, h->wrad, h->leb, h->px, h->py, h->pz, h->adj_ab, nblk,
                          h->adj_part, h->adj_mot, (int*)(h->adj_out + 6 * na));
     }));
     DG_TRY(run(h, "adj_force_sum", [&] {

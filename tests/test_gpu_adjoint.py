@@ -165,3 +165,18 @@ def test_c10h22_forces_and_dEdP_full_grid():
         fd = (e[0] - e[1]) / (2 * h)
         print(f"  atom {a} dir {d}: analytic {grad[a, d]:.10f} fd {fd:.10f}", flush=True)
         assert abs(fd - grad[a, d]) < 1e-5, (a, d, fd, grad[a, d])
+
+
+@pytest.mark.parametrize("make,nrad,nang", [(M.benzene, 37, 50), (lambda b: M.alkane(4, b), 30, 38)])
+def test_gradient_of_displaced_molecules(make, nrad, nang):
+    """No symmetry, and grids fine enough that some points' owner cells lie between the
+    kernel's candidate and skip levels (1e-20 of the nearest cell's P and of their sum)."""
+    from oracle import adjoint as AD
+    mol = make("sto3g")
+    mol.xyz = mol.xyz + 0.05 * np.random.default_rng(11).standard_normal(mol.xyz.shape)
+    P = _density(mol)
+    print(f"[case] displaced {mol.name} {nrad}x{nang}", flush=True)
+    _, dP_o, grad_o = AD.xc_adjoint(mol, nrad, nang, 3, P)
+    _, _, _, dP, grad = _lib_adjoint(mol, nrad, nang, 3, P, False)
+    assert np.abs(dP - dP_o).max() < 1e-11 * np.abs(dP_o).max()
+    assert np.abs(grad - grad_o).max() < 1e-10 * max(1.0, np.abs(grad_o).max())
