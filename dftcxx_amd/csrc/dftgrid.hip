@@ -244,8 +244,10 @@ __global__ void k_phi(const double* __restrict__ atoms, int nshell, const int* _
             (int)(g % nshell));
 }
 
-// Screening mask: bit T of mask[b] is set when some |phi| of basis tile T
-// (16 functions) exceeds screen on the 64-point block b.  One wave per block.
+// Tile mask: bit T of mask[b] is set when some |phi| of basis tile T (16
+// functions) exceeds screen on the 64-point block b.  One wave per block.
+constexpr double kAmpReach = 0x1p-106;
+
 __global__ __launch_bounds__(64) void k_block_mask(const double* __restrict__ phi, int ldphi, int ntb,
                                                    double screen, unsigned* mask) {
   const long p = (long)blockIdx.x * 64 + threadIdx.x;
@@ -270,7 +272,7 @@ __global__ __launch_bounds__(64) void k_block_mask(const double* __restrict__ ph
 // Tile b holds 4(b+1) reduction steps s; entry [s][lane] is
 // P'(16b + pi(lane%16), kk(s, lane/16)), kk(s,g) = 16(s/4) + 4g + s%4,
 // pi(r) = 4(r%4) + r/4, stored from offset 128 b (b+1).  The same permutation
-// kk of the reduction index is used for phi in k_density, and pi puts
+// kk of the reduction index is used for phi in the kernels, and pi puts
 // T_b[p][16b + 4g + v] in result register v of lane (c = p%16, g): the lane
 // that holds phi[p][16b + 4g + v] as its B operand of step 4b + v, so the
 // final dot product needs no further loads.
@@ -286,124 +288,20 @@ __device__ __forceinline__ double pfrag_value(const double* __restrict__ P, int 
   return (j < nbf && k < nbf) ? f * P[j + (long)k * nbf] : 0.0;
 }
 
-__global__ void k_pfrag(const double* __restrict__ P, int nbf, int nt, double* frag) {
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// The first nfb work-groups write the fragments, the others clear rho on the
+// nempty blocks where no tile counts.
+__global__ __launch_bounds__(256) void k_pfrag(const double* __restrict__ P, int nbf, int nt, double* frag,
+                                               unsigned nfb, const int* __restrict__ empty, int nempty, double* rho) {
+  if (blockIdx.x >= nfb) {
+    const int b = 4 * (int)(blockIdx.x - nfb) + (threadIdx.x >> 6);
+    if (b < nempty) rho[64L * empty[b] + (threadIdx.x & 63)] = 0.0;
+    return;
+  }
+  const long e = (long)blockIdx.x * 256 + threadIdx.x;
   if (e >= 128L * nt * (nt + 1)) return;
   frag[e] = pfrag_value(P, nbf, e);
 }
 
-// One wave handles 16 points; lane (c = lane%16, g = lane/16) keeps
-// phi[p0+c][kk(s,g)] for every reduction step s in registers (B operand).
-// For output tile b the wave forms T_b[p][16b+4v+g] (result register v) with
-// 4(b+1) MFMAs in two accumulation chains (steps j even / odd), then dots it
-// with phi[p][16b+4v+g], which is its own B-operand register f[4b+v] (the tile
-// loop is unrolled, so every register index is a constant).  The P fragments
-// of one tile are staged in LDS and shared by the work-group's W waves
-// (16 W points), copied from global memory straight into LDS (global_load_lds,
-// 1 KB per wave instruction).  NT = ceil(nbf/16).
-// NBUF = 1: one tile buffer (<= 50 KB at NT <= 25), so that two work-groups of
-// W = 4 share a CU, one wave of each per SIMD: while one work-group copies a
-// tile, waits at its barriers or loads its amplitude rows, the other issues
-// MFMAs.  NBUF = 2: the next live tile is copied into the other buffer while the
-// current tile's MFMAs run.
-// With screening, mask (one word per 64-point block, bit T for basis tile T)
-// drops the tiles whose amplitudes are negligible on the whole block: a wave
-// skips the MFMAs of the tiles off its block's word, and the work-group walks
-// (and fetches) the tiles on any of its blocks' words, so every branch on the
-// walk is uniform over the work-group.
-template <int NT, int W, int NBUF>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(NBUF == 1 ? 2 : 1))) void k_density(
-    const double* __restrict__ phi, int ldphi, const double* __restrict__ frag, double* rho,
-    const unsigned* __restrict__ mask) {
-  static_assert(W % 4 == 0 && (NBUF == 1 || NBUF == 2), "whole 64-point blocks; one or two tile buffers");
-  __shared__ double pl[NBUF][4 * NT * 64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int g = lane >> 4, c = lane & 15;
-  const long p0 = (long)blockIdx.x * 16 * W + wave * 16;
-  const double* row = phi + (p0 + c) * ldphi;
-  constexpr unsigned all = NT >= 32 ? 0xffffffffu : ((1u << NT) - 1u);
-  const long blk0 = (long)blockIdx.x * W / 4;  // first 64-point block of the work-group
-  // wave-uniform (the compiler cannot see that from threadIdx)
-  const unsigned mine = __builtin_amdgcn_readfirstlane((mask ? mask[blk0 + wave / 4] : 0xffffffffu) & all);
-  unsigned mk = 0;
-  for (int b = 0; b < W / 4; ++b) mk |= (mask ? mask[blk0 + b] : 0xffffffffu) & all;
-  double f[4 * NT];
-#pragma unroll
-  for (int s = 0; s < 4 * NT; ++s) f[s] = ((mine >> (s >> 2)) & 1u) ? row[16 * (s >> 2) + 4 * g + (s & 3)] : 0.0;
-  // tile b's fragments, 256 (b + 1) doubles from offset 128 b (b + 1): chunks of
-  // 128 doubles, chunk q copied by wave q % W, 16 bytes per lane
-  auto fetch = [&](int b, double* dst) {
-    const double* src = frag + 128L * b * (b + 1);
-    for (int q = wave; q < 2 * (b + 1); q += W)
-      __builtin_amdgcn_global_load_lds((const void*)(src + q * 128 + lane * 2),
-                                       (__attribute__((address_space(3))) void*)(dst + q * 128), 16, 0, 0);
-  };
-  auto next_live = [&](int b) {  // first tile > b with its mask bit set, NT if none
-    const unsigned rest = (b + 1 >= 32) ? 0u : (mk >> (b + 1));
-    return rest ? b + 1 + __builtin_ctz(rest) : NT;
-  };
-  double acc = 0.0;
-  int buf = 0;
-  if (NBUF == 2) {
-    const int b0 = next_live(-1);
-    if (b0 < NT) fetch(b0, pl[0]);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-  }
-  // tiles in compile-time order (each skipped when off the mask), so that the
-  // amplitudes of the final dot are the B-operand registers f[4b + v]
-#pragma unroll
-  for (int b = 0; b < NT; ++b) {
-    if (!((mk >> b) & 1u)) continue;
-    if (NBUF == 2) {
-      const int nb = next_live(b);
-      if (nb < NT) fetch(nb, pl[buf ^ 1]);
-    } else {
-      fetch(b, pl[0]);
-      __builtin_amdgcn_s_waitcnt(0);  // this wave's copies have landed
-      __syncthreads();
-    }
-    const double* cur = pl[buf];
-    // two accumulation chains (steps j even / odd) over the reduction tiles k <= b
-    dbl4 d0 = {0.0, 0.0, 0.0, 0.0}, d1 = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int k = 0; k <= b; ++k) {
-      if ((mine >> k) & 1u) {
-        double av[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) av[j] = cur[(4 * k + j) * 64 + lane];
-        d0 = mfma16x16x4(av[0], f[4 * k], d0);
-        d1 = mfma16x16x4(av[1], f[4 * k + 1], d1);
-        d0 = mfma16x16x4(av[2], f[4 * k + 2], d0);
-        d1 = mfma16x16x4(av[3], f[4 * k + 3], d1);
-      }
-    }
-    // register v of lane (c, g) holds T_b[p0+c][16b + 4g + v]; f[4b + v] = phi[p0+c][16b + 4g + v]
-    if ((mine >> b) & 1u)
-      acc += (d0[0] + d1[0]) * f[4 * b] + (d0[1] + d1[1]) * f[4 * b + 1] + (d0[2] + d1[2]) * f[4 * b + 2] +
-             (d0[3] + d1[3]) * f[4 * b + 3];
-    if (NBUF == 2) {
-      __builtin_amdgcn_s_waitcnt(0);  // this wave's copies into the other buffer have landed
-      __syncthreads();
-      buf ^= 1;
-    } else {
-      __syncthreads();  // every wave is done with the buffer before the next copy
-    }
-  }
-  acc += __shfl_xor(acc, 16);
-  acc += __shfl_xor(acc, 32);
-  if (g == 0) rho[p0 + c] = 2.0 * acc;
-}
-
-// k_density without screening, its P fragments streamed through a ring.  The
-// fragments are stored tile after tile, reduction tile after reduction tile
-// (unit (b, k), k <= b: 4 steps x 64 lanes = 2 KB), which is the order the
-// tiles consume them; the stream is cut into chunks of kDensityChunk units
-// (16 KB, four 1 KB copy instructions per wave; the last chunk ends at the end
-// of the stream and overlaps the one before) and each chunk is copied two
-// chunks ahead into one of three LDS slots (48 KB: two work-groups per CU).  One wait and barrier per chunk, which then also
-// tells that every wave is done with the slot the next copy overwrites.  W = 4
-// waves share the chunks.
 constexpr int kDensityChunk = 8;
 
 // Chunks of C units of a fragment stream of U >= C units (256 doubles each):
@@ -451,26 +349,80 @@ __device__ __forceinline__ void bare_barrier() {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 }
-template <int NT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_density_ring(
-    const double* __restrict__ phi, int ldphi, const double* __restrict__ frag, double* rho) {
-  constexpr int C = kDensityChunk, U = NT * (NT + 1) / 2, NCH = (U + C - 1) / C;
+
+// One work-group takes a 64-point block on which N tiles count, 16 points a
+// wave; lane (c = lane%16, g = lane/16) keeps phi[p0+c][kk(s,g)] of those
+// tiles in registers for every reduction step s (B operand).  For output tile b
+// the wave forms T_b[p][16b+4v+g] (result register v) with 4(b+1) MFMAs in two
+// accumulation chains (steps even / odd), then dots it with phi[p][16b+4v+g],
+// which is its own B-operand register f[4b+v] (the tile loops are unrolled, so
+// every register index is a constant).
+// The P fragments come as a stream of 2 KB units (b, k), k <= b, 4 steps x 64
+// lanes each, in the order the tiles consume them, cut into chunks of
+// kDensityChunk units (16 KB; the last chunk ends at the end of the stream and
+// overlaps the one before), each copied two chunks ahead into one of three LDS
+// slots (48 KB).  One wait and barrier per chunk, which then also tells that
+// every wave is done with the slot the next copy overwrites.
+// tiles: per entry, the N tile numbers of its block as 32 bytes, ascending (255:
+// none, zeros stand in); the units are gathered by them, so the loops have no
+// branches.  (With the tiles
+// of all NT walked and the others branched over, the LDS reads no longer ran
+// ahead of the MFMAs: C30H62 2.85 ms at the default reach, 5.55 ms dense.)
+// 8 N registers hold the amplitudes, which leaves two waves per SIMD up to 25
+// tiles and one beyond (three and four waves with 8 KB chunks on the small sizes:
+// 3 % slower).  C30H62 at the default reach: 2.3 ms, 70 % of the MFMA rate; what is
+// left is the start of each block, whose amplitudes wait on HBM.
+template <int N>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N <= 25 ? 2 : 1))) void
+k_density_ring(const double* __restrict__ phi, int ldphi, const double* __restrict__ frag, double* rho,
+               const int* __restrict__ blocks, const uint4* __restrict__ tiles, int nt) {
+  constexpr int C = 8, U = N * (N + 1) / 2, NCH = (U + C - 1) / C;
+  static_assert(U >= C, "at least one whole chunk");
   __shared__ double ring[3][C * 256];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ int unit[U];  // of the stream: its place among the fragments
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int g = lane >> 4, c = lane & 15;
-  const long p0 = (long)blockIdx.x * 64 + wave * 16;
-  const double* row = phi + (p0 + c) * ldphi;
-  double f[4 * NT];
+  const uint4 ta = tiles[2 * (long)blockIdx.x], tb = tiles[2 * (long)blockIdx.x + 1];
+  const unsigned tw[8] = {ta.x, ta.y, ta.z, ta.w, tb.x, tb.y, tb.z, tb.w};
+  const unsigned char* ids = (const unsigned char*)(tiles + 2 * (long)blockIdx.x);
+  for (int u = threadIdx.x; u < U; u += 256) {
+    int b = (int)((__builtin_sqrtf(8.0f * u + 1.0f) - 1.0f) * 0.5f);
+    b += (b + 1) * (b + 2) / 2 <= u ? 1 : 0;
+    b -= b * (b + 1) / 2 > u ? 1 : 0;
+    const int tr = min((int)ids[b], nt - 1), tc = min((int)ids[u - b * (b + 1) / 2], nt - 1);
+    unit[u] = tr * (tr + 1) / 2 + tc;
+  }
+  const long p0 = 64L * blocks[blockIdx.x] + wave * 16;
+  bare_barrier();  // the table is whole; before the amplitude loads, which it need not wait for
+  const double* row = phi + (p0 + c) * ldphi + 4 * g;
+  double f[4 * N];
 #pragma unroll
-  for (int s = 0; s < 4 * NT; ++s) f[s] = row[16 * (s >> 2) + 4 * g + (s & 3)];
-  auto copy = [&](int j) { stream_copy<C, U>(frag, ring[j % 3], j, wave, lane); };
+  for (int r = 0; r < N; ++r) {
+    const int t = (int)((tw[r >> 2] >> (8 * (r & 3))) & 255u);
+    const double* x = row + 16 * min(t, nt - 1);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) f[4 * r + v] = t < nt ? x[v] : 0.0;
+  }
+  // 1 KB pieces, two a unit: wave w takes half w % 2 of units w / 2, w / 2 + 2, ... of
+  // the chunk (every wave issues C / 2 copies, which the wait relies on)
+  const double* src = frag + (wave & 1) * 128 + lane * 2;
+  auto copy = [&](int j) {
+    const int mine = unit[stream_start<C, U>(j) + 2 * (lane & (C / 2 - 1)) + (wave >> 1)];
+#pragma unroll
+    for (int q = 0; q < C / 2; ++q) {
+      const int at = __builtin_amdgcn_readlane(mine, q);
+      __builtin_amdgcn_global_load_lds((const void*)(src + 256L * at),
+                                       (__attribute__((address_space(3))) void*)(&ring[j % 3][(wave + 4 * q) * 128]),
+                                       16, 0, 0);
+    }
+  };
   copy(0);
   if (NCH > 1) copy(1);
   double acc = 0.0;
   dbl4 d0 = {0.0, 0.0, 0.0, 0.0}, d1 = d0;
   int u = 0;
 #pragma unroll
-  for (int b = 0; b < NT; ++b) {
+  for (int b = 0; b < N; ++b) {
 #pragma unroll
     for (int k = 0; k <= b; ++k, ++u) {
       if (u % C == 0) {
@@ -498,7 +450,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   if (g == 0) rho[p0 + c] = 2.0 * acc;
 }
 
-// k_density for small bases (NT <= 7): the whole fragment set (128 NT(NT+1)
+// The density of small bases (NT <= 7): the whole fragment set (128 NT(NT+1)
 // doubles, formed from P as k_pfrag does) is staged in LDS once per work-group, which then walks the 64-point
 // blocks b = blockIdx.x, blockIdx.x + G, ... with no further barriers; each
 // wave loads the next block's amplitude row while it multiplies the current.
@@ -1364,18 +1316,19 @@ __global__ __launch_bounds__(256) void k_vreduce(const double* __restrict__ vpar
 // covers the tiles (I0 + r, J0 + t), r < nI, t < nJ <= NJ, I <= J, of the NOUT
 // outputs, so a wave loads 4 + NJ amplitude tiles per step (4 points) for
 // 4 NJ NOUT MFMAs: NJ = 2 with two outputs (J and XC), NJ = 4 with one.  The
-// block's 64-point blocks (its list: all, or with screening those where its
-// tiles are significant) are split evenly over nsplit work-groups (split-K);
-// the 4 waves interleave the 16 points of each block.  The 4 waves are added in
-// LDS in wave order and written as 4 reduction groups (I0 + r, J0, nJ) in the
-// k_contract_reduce layout.
+// block's 64-point blocks (its list: those where its tiles count, tile_reach) are
+// split over work-groups of about equal cost (split-K); the 4 waves interleave
+// the 16 points of each block.  The 4 waves are added in LDS in wave order and
+// written to the work-group's partial slot as 4 reduction groups (I0 + r, J0, nJ)
+// in the k_contract_reduce layout.
 // Work-group order: the hardware deals work-groups round-robin to the kXcds
-// XCDs, each with its own L2.  Work-group L (1-D grid, padded to a multiple of
-// kXcds) takes virtual id v = (L % kXcds) per + L / kXcds and order[v] = {tile
-// block, split}: consecutive v are the tile blocks of one split, so an XCD runs
-// whole splits, and within an XCD's range the blocks with the most MFMAs come
-// first, so that the short diagonal blocks fill the last round.
+// XCDs, each with its own L2.  Work-group L (1-D grid, a multiple of kXcds) takes
+// virtual id v = (L % kXcds) per + L / kXcds and order[v] = {tile block (-1: none),
+// first list entry, entries, partial slot}; an XCD's range goes through the point
+// blocks from low to high, so that what runs there together reads the same rows.
 constexpr int kXcds = 8;
+// Bit of a list entry (mixed precision): the FP32 sums end with this point block.
+constexpr int kGroupEnd = 1 << 31;
 
 // The FP64 2-D contraction, its operands staged through LDS: each wave copies
 // the amplitude rows and weights of step st + D - 1 into slot (st + D - 1) % D
@@ -1385,42 +1338,46 @@ constexpr int kXcds = 8;
 // later steps in flight.  Slot layout (doubles): the 4 points' rows of tiles
 // I0..I0+3 (point-major, 64 each), of tiles J0..J0+NJ-1 (16 NJ each), then
 // u0 and u1 of the 4 points.  The epilogue's LDS reduction reuses the ring.
-template <int NOUT, int NJ, int D, bool DENSE>
+template <int NOUT, int NJ, int D>
 __global__ __launch_bounds__(256, 3) void k_contract2d_lds(const double* __restrict__ phi, int ldphi,
                                                           const double* __restrict__ u0,
                                                           const double* __restrict__ u1,
                                                           const int* __restrict__ cblocks,
                                                           const int* __restrict__ blist,
-                                                          const int* __restrict__ loff,
-                                                          const int2* __restrict__ order, int ngroups, int nsplit,
-                                                          double* part) {
+                                                          const int4* __restrict__ order, double* part) {
   constexpr int SA = 256, SB = 64 * NJ, SW = 8, SLOT = SA + SB + SW;  // doubles per slot
   constexpr int NI = 2 + NJ / 2 + 1;                                    // copy instructions per step
   static_assert(4 * SLOT * D >= 4 * NJ * 256, "the epilogue reduction fits in the ring");
   __shared__ __attribute__((aligned(16))) double ring[4 * SLOT * D];
   double* red = ring;
-  const int ncb = ngroups / 4, per = gridDim.x / kXcds;
-  const int v = (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
-  if (v >= ncb * nsplit) return;
-  const int cbi = order[v].x, split = order[v].y;
+  const int v = (blockIdx.x % kXcds) * (gridDim.x / kXcds) + blockIdx.x / kXcds;
+  const int4 job = order[v];
+  const int cbi = job.x;
+  if (cbi < 0) return;
   const int I0 = cblocks[4 * cbi], nI = cblocks[4 * cbi + 1], J0 = cblocks[4 * cbi + 2], nJ = cblocks[4 * cbi + 3];
   // the wave index as a scalar, so that the ring addresses stay in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int g = lane >> 4, c = lane & 15;
-  const long l0 = loff[cbi], cnt = loff[cbi + 1] - l0;
-  const int s0 = (int)(cnt * split / nsplit);
-  const int* bl = blist + l0 + s0;
-  const int nst = 4 * (int)(cnt * (split + 1) / nsplit - s0);
+  const int* bl = blist + job.y;
+  const int nst = 4 * job.z;
   double* my = ring + wave * SLOT * D;
   // step t covers this wave's points p .. p + 3, p = 4 wave + rows(t) with
-  // rows(t) = 64 s0 + 16 t dense, 64 blist[t / 4] + 16 (t % 4) screened
-  auto rows = [&](int t) { return DENSE ? 16L * t : 64L * bl[t >> 2] + 16 * (t & 3); };
+  // rows(t) = 64 bl[t / 4] + 16 (t % 4); copy runs through the steps in order,
+  // and each list entry is read one block ahead of its use
+  int blk = 0, ahead = nst > 0 ? bl[0] : 0;
+  auto rows = [&](int t) {
+    if ((t & 3) == 0) {
+      blk = ahead;
+      if (t + 4 < nst) ahead = bl[(t >> 2) + 1];
+    }
+    return 64L * (blk & ~kGroupEnd) + 16 * (t & 3);
+  };
   // copy lane roles: A pair k = 64 i + lane -> point k / 32, columns 2 (k % 32), +1;
   // weights: lanes 0, 1 u0 of points 0-1, 2-3, lanes 2, 3 u1 (unused with one output).
   // Each lane's sources at rows(t) = 0, so that a copy adds one row offset.
   const int ag = lane >> 5, acol = 16 * I0 + 2 * (lane & 31);
   const int bg = NJ == 2 ? lane >> 4 : lane >> 5, bcol = 16 * J0 + 2 * (NJ == 2 ? (lane & 15) : (lane & 31));
-  const long p0 = (DENSE ? 64L * s0 : 0L) + 4 * wave;
+  const long p0 = 4 * wave;
   const double* pa = phi + (p0 + ag) * ldphi + acol;
   const double* pb = phi + (p0 + bg) * ldphi + bcol;
   const double* pw = (lane < 2 ? u0 : u1) + p0 + 2 * (lane & 1);
@@ -1492,7 +1449,7 @@ __global__ __launch_bounds__(256, 3) void k_contract2d_lds(const double* __restr
     __syncthreads();
     for (int e = threadIdx.x; e < 4 * NJ * 256; e += 256) {
       const int r = e / (NJ * 256), t = (e >> 8) % NJ, rem = e & 255;
-      part[(((long)split * ngroups + 4 * cbi + r) * NOUT + o) * 1024 + t * 256 + rem] = red[e];
+      part[((4L * job.w + r) * NOUT + o) * 1024 + t * 256 + rem] = red[e];
     }
   }
 }
@@ -1501,49 +1458,53 @@ __global__ __launch_bounds__(256, 3) void k_contract2d_lds(const double* __restr
 // (register v of lane (c, g) holds row 4g + v), staged through the same kind of
 // per-wave LDS ring (slot: the 4 points' FP32 rows of tiles I0..I0+3, of tiles
 // J0..J0+NJ-1, then u0 and u1 of the 4 points in FP64; three copy instructions per
-// step).  Every 16 steps (64 points) a wave adds its FP32 sums into FP64 sums it
+// step).  At the marked list entries (at most 16 steps, 64 points of a wave, apart) a wave adds its FP32 sums into FP64 sums it
 // keeps in registers, so the waves never wait for each other before the epilogue;
 // the FP64 sums (64 doubles per lane) leave room for two waves per SIMD, and the
 // ring, with two work-groups per CU, is D steps deep.  The weights are rounded to
 // FP32 and multiply the B operand in FP32.
-template <int NOUT, int NJ, int D, bool DENSE>
+template <int NOUT, int NJ, int D>
 __global__ __launch_bounds__(256, 2) void k_contract2d_lds_f32(const float* __restrict__ phi, int ldphi,
                                                               const double* __restrict__ u0,
                                                               const double* __restrict__ u1,
                                                               const int* __restrict__ cblocks,
                                                               const int* __restrict__ blist,
-                                                              const int* __restrict__ loff,
-                                                              const int2* __restrict__ order, int ngroups,
-                                                              int nsplit, double* part) {
+                                                              const int4* __restrict__ order, double* part) {
   constexpr int SA = 256, SB = 64 * NJ;            // floats per slot: A and B rows
   constexpr int SLOT = (SA + SB) * 4 + 8 * 8;      // bytes per slot (+ 8 FP64 weights)
   constexpr int NI = 3;                            // copy instructions per step
   static_assert(4 * SLOT * D >= 4 * NJ * 256 * 8, "the epilogue reduction fits in the ring");
   __shared__ __attribute__((aligned(16))) char ring[4 * SLOT * D];
   double* red = reinterpret_cast<double*>(ring);
-  const int ncb = ngroups / 4, per = gridDim.x / kXcds;
-  const int v = (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
-  if (v >= ncb * nsplit) return;
-  const int cbi = order[v].x, split = order[v].y;
+  const int v = (blockIdx.x % kXcds) * (gridDim.x / kXcds) + blockIdx.x / kXcds;
+  const int4 job = order[v];
+  const int cbi = job.x;
+  if (cbi < 0) return;
   const int I0 = cblocks[4 * cbi], nI = cblocks[4 * cbi + 1], J0 = cblocks[4 * cbi + 2], nJ = cblocks[4 * cbi + 3];
   // the wave index as a scalar, so that the ring addresses stay in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int g = lane >> 4, c = lane & 15;
-  const long l0 = loff[cbi], cnt = loff[cbi + 1] - l0;
-  const int s0 = (int)(cnt * split / nsplit);
-  const int* bl = blist + l0 + s0;
-  const int nst = 4 * (int)(cnt * (split + 1) / nsplit - s0);
+  const int* bl = blist + job.y;
+  const int nst = 4 * job.z;
   char* my = ring + wave * SLOT * D;
   // step t covers this wave's points p .. p + 3, p = 4 wave + rows(t) with
-  // rows(t) = 64 s0 + 16 t dense, 64 blist[t / 4] + 16 (t % 4) screened
-  auto rows = [&](int t) { return DENSE ? 16L * t : 64L * bl[t >> 2] + 16 * (t & 3); };
+  // rows(t) = 64 bl[t / 4] + 16 (t % 4); copy runs through the steps in order,
+  // and each list entry is read one block ahead of its use
+  int blk = 0, ahead = nst > 0 ? bl[0] : 0;
+  auto rows = [&](int t) {
+    if ((t & 3) == 0) {
+      blk = ahead;
+      if (t + 4 < nst) ahead = bl[(t >> 2) + 1];
+    }
+    return 64L * (blk & ~kGroupEnd) + 16 * (t & 3);
+  };
   // copy lane roles: A: point lane / 16, 4 columns from 16 I0 + 4 (lane % 16);
   // B (the first 16 NJ lanes): point lane / (4 NJ), 4 columns from 16 J0 + 4 (lane % 4 NJ);
   // weights: lanes 0, 1 u0 of points 0-1, 2-3, lanes 2, 3 u1 (unused with one output).
   // Each lane's sources at rows(t) = 0, so that a copy adds one row offset.
   const int ag = lane >> 4, acol = 16 * I0 + 4 * (lane & 15);
   const int bg = lane / (4 * NJ), bcol = 16 * J0 + 4 * (lane % (4 * NJ));
-  const long p0 = (DENSE ? 64L * s0 : 0L) + 4 * wave;
+  const long p0 = 4 * wave;
   const float* pa = phi + (p0 + ag) * ldphi + acol;
   const float* pb = phi + (p0 + bg) * ldphi + bcol;
   const double* pw = (lane < 2 ? u0 : u1) + p0 + 2 * (lane & 1);
@@ -1570,7 +1531,9 @@ __global__ __launch_bounds__(256, 2) void k_contract2d_lds_f32(const float* __re
 #pragma unroll
   for (int k = 0; k < D - 1; ++k)
     if (k < nst) copy(k, k);
+  int entry = 0;
   for (int st = 0; st < nst; ++st) {
+    if ((st & 3) == 0) entry = bl[st >> 2];
     if (st + D - 1 < nst) {
       copy(st + D - 1, (st + D - 1) % D);
       __builtin_amdgcn_s_waitcnt(waitcnt_vm(NI * (D - 1)));
@@ -1597,7 +1560,7 @@ __global__ __launch_bounds__(256, 2) void k_contract2d_lds_f32(const float* __re
             acc[NOUT - 1][r][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(ca[r], b1, acc[NOUT - 1][r][t], 0, 0, 0);
         }
     }
-    if ((st & 15) == 15 || st + 1 == nst) {
+    if ((st & 3) == 3 && (entry & kGroupEnd)) {
 #pragma unroll
       for (int o = 0; o < NOUT; ++o)
 #pragma unroll
@@ -1630,7 +1593,7 @@ __global__ __launch_bounds__(256, 2) void k_contract2d_lds_f32(const float* __re
     __syncthreads();
     for (int e = threadIdx.x; e < 4 * NJ * 256; e += 256) {
       const int r = e / (NJ * 256), t = (e >> 8) % NJ, rem = e & 255;
-      part[(((long)split * ngroups + 4 * cbi + r) * NOUT + o) * 1024 + t * 256 + rem] = red[e];
+      part[((4L * job.w + r) * NOUT + o) * 1024 + t * 256 + rem] = red[e];
     }
   }
 }
@@ -1901,7 +1864,7 @@ __global__ void k_pfrag_full(const double* __restrict__ P, int nbf, int nt, doub
 }
 
 // T = Phi P (T[p][j] = sum_k phi_pk P_kj) with the FP64 MFMA, same operand
-// arrangement as k_density; T is written [npts_pad][ldphi].  W waves (16
+// arrangement as k_density_ring; T is written [npts_pad][ldphi].  W waves (16
 // points each) share each column tile's fragments in LDS, double-buffered: the
 // next tile's are copied by global_load_lds while the current tile's MFMAs run
 // in four accumulation chains; one wait and barrier per tile.
@@ -2689,8 +2652,9 @@ __device__ __forceinline__ flt4 mfma16x16x4f32(float a, float b, flt4 c) {
 // instead (k_scalars, which depends on nothing this kernel writes).
 __global__ __launch_bounds__(256) void k_contract_reduce(const double* __restrict__ part, int nsplit,
                                                          int ngroups, int nout,
-                                                         const int* __restrict__ groups, int nbf,
-                                                         double* out0, double* out1, ScalarArgs sa) {
+                                                         const int* __restrict__ groups,
+                                                         const int* __restrict__ slot0, int nbf, double* out0,
+                                                         double* out1, ScalarArgs sa) {
   if (sa.scalars && blockIdx.x == gridDim.x - 1) {
     scalars_block(sa);
     return;
@@ -2705,8 +2669,14 @@ __global__ __launch_bounds__(256) void k_contract_reduce(const double* __restric
   const int grp = live ? (int)((e >> 10) / nout) : 0;
   if (live && (idx >> 8) >= groups[3 * grp + 2]) live = false;  // tile beyond the group: not read
   if (live) {
-    const long stride = (long)ngroups * nout * 1024;
+    long stride = (long)ngroups * nout * 1024;
     const double* src = part + ((long)grp * nout + o) * 1024 + idx;
+    if (slot0) {
+      const int s0 = slot0[grp >> 2];
+      nsplit = slot0[(grp >> 2) + 1] - s0;
+      stride = 4096L * nout;
+      src = part + ((4L * s0 + (grp & 3)) * nout + o) * 1024 + idx;
+    }
     // eight splits' partials loaded per round (one memory latency), added in split order
     int sp = r;
     for (; sp + 16 * 7 < nsplit; sp += 16 * 8) {
@@ -2791,13 +2761,19 @@ struct ProfStat {
 
 // Tile blocks of the 2-D contraction for one block width NJ: {I0, nI, J0, nJ} per
 // block, its four reduction groups (I0 + r, J0, nJ) in the k_contract_reduce
-// layout, the 64-point block list of each block (all blocks, or with screening
-// those where its tiles are significant), and per virtual work-group id the
-// {tile block, split} it runs.
+// layout, the 64-point block lists of the blocks one after the other (where
+// their tiles count), per work-group {tile block, first and number of list
+// entries, partial slot}, and per tile block its first partial slot.
 struct TileBlocks {
-  int *cb = nullptr, *groups = nullptr, *list = nullptr, *loff = nullptr;
-  int2* order = nullptr;
-  int ncb = 0, nsplit = 0;
+  int *cb = nullptr, *groups = nullptr, *list = nullptr, *slot0 = nullptr;
+  int4* order = nullptr;
+  int ncb = 0, nwg = 0;
+};
+
+// A launch of k_density_ring<n>: entries [first, first + count) of dblocks / dtiles.
+struct DensityClass {
+  int n;
+  long first, count;
 };
 
 struct dg_handle {
@@ -2841,6 +2817,11 @@ struct dg_handle {
   // screening masks
   double screen = 0.0;
   unsigned* bmask = nullptr;
+  // density beyond 7 tiles: the point blocks by the number of tiles that count there
+  std::vector<DensityClass> dclass;
+  int *dblocks = nullptr, *dempty = nullptr;
+  uint4* dtiles = nullptr;
+  int nempty = 0;
   // reduced-precision mode
   float* phf = nullptr;  // FP32 amplitudes
   double* ej_part = nullptr;
@@ -2867,7 +2848,6 @@ struct dg_handle {
   int *ash_start = nullptr, *ash_list = nullptr;
   int* atom_order = nullptr;  // per atom, all atoms by distance
   unsigned* adj_tmask = nullptr;  // per 64-point block, the function tiles the force terms read
-  int *adj_list = nullptr, *adj_loff = nullptr;  // dE/dP: point blocks per one-output tile block
   // state
   bool has_density = false, has_hartree = false, has_xc = false, corrected = false;
   const double* last_P = nullptr;  // device density matrix of the last density evaluation
@@ -2886,11 +2866,12 @@ struct dg_handle {
                       mol_z, mol_fac, mol_qraw, atom_exc, atom_ej, qpart, uG, coef, mono, sh_amin};
     for (double* b : bufs)
       if (b) (void)hipFree(b);
-    int* ibufs[] = {sh_atom, sh_L, sh_nprim, sh_off, sh_cgf, blocks, ntask, ash_start, ash_list, atom_order, adj_list, adj_loff,
+    int* ibufs[] = {sh_atom, sh_L, sh_nprim, sh_off, sh_cgf, blocks, ntask, ash_start, ash_list, atom_order, dblocks, dempty,
                     atom_mol, mol_atom0, mol_shell0, mol_nbf, bchunks, mol_chunk0,
-                    tb[0].cb, tb[0].groups, tb[0].list, tb[0].loff, tb[1].cb, tb[1].groups, tb[1].list,
-                    tb[1].loff};
+                    tb[0].cb, tb[0].groups, tb[0].list, tb[0].slot0, tb[1].cb, tb[1].groups, tb[1].list,
+                    tb[1].slot0};
     if (bmask) (void)hipFree(bmask);
+    if (dtiles) (void)hipFree(dtiles);
     if (adj_tmask) (void)hipFree(adj_tmask);
     for (TileBlocks& t : tb)
       if (t.order) (void)hipFree(t.order);
@@ -2955,20 +2936,41 @@ int run(dg_handle* h, const char* name, F launch) {
 
 unsigned nblocks(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
-// Per 4 x 2 tile block {I0, nI, J0, nJ}, the 64-point blocks on which one of its
-// row tiles and one of its column tiles are significant (all blocks without
-// screening), and the list offsets.
-void tile_block_lists(const std::vector<unsigned>& mk, const std::vector<int>& cbs, std::vector<int>& list,
-                      std::vector<int>& off) {
+// Per tile block {I0, nI, J0, nJ}, the 64-point blocks on which one of its row
+// tiles and one of its column tiles count, and the list offsets.  split > 0
+// (mixed precision): kGroupEnd marks the ends of the FP32 sums, four blocks from
+// the start of each of split equal parts of the candidates, which are the blocks
+// that count (screened) or all blocks; so the grouping, and with it the rounding
+// of the FP32 sums, depends on neither the reach nor the work-groups.
+void tile_block_lists(const std::vector<unsigned>& mk, const std::vector<int>& cbs, long split, bool screened,
+                      std::vector<int>& list, std::vector<int>& off) {
   const int n = (int)cbs.size() / 4;
   off.assign(n + 1, 0);
   list.clear();
   for (int q = 0; q < n; ++q) {
     const unsigned ri = ((1u << cbs[4 * q + 1]) - 1u) << cbs[4 * q];
     const unsigned cj = ((1u << cbs[4 * q + 3]) - 1u) << cbs[4 * q + 2];
+    std::vector<int> at;  // their places among the candidates
     for (size_t b = 0; b < mk.size(); ++b)
-      if ((mk[b] & ri) && (mk[b] & cj)) list.push_back((int)b);
+      if ((mk[b] & ri) && (mk[b] & cj)) {
+        at.push_back(screened ? (int)at.size() : (int)b);
+        list.push_back((int)b);
+      }
     off[q + 1] = (int)list.size();
+    const long cnt = screened ? (long)at.size() : (long)mk.size();
+    long part = -1, group = -1, end = 0, begin = 0;
+    for (size_t i = 0; split > 0 && i < at.size(); ++i) {
+      while (at[i] >= end) {
+        ++part;
+        begin = cnt * part / split;
+        end = cnt * (part + 1) / split;
+        group = -1;
+      }
+      const long g = (at[i] - begin) / 4;
+      if (i > 0 && g != group) list[off[q] + i - 1] |= kGroupEnd;
+      group = g;
+    }
+    if (split > 0 && !at.empty()) list.back() |= kGroupEnd;
   }
 }
 
@@ -2980,27 +2982,6 @@ int sort_items(dg_handle* h) {
                        h->items, h->atoms, h->px, h->py, h->pz, h->knots, h->vbase, h->nrad, h->nang, h->max_tasks,
                        h->perm, h->task, h->ntask);
   });
-}
-
-template <int NT>
-void launch_density_nt(dg_handle* h) {
-  // Without screening, up to 400 functions: the fragments streamed through a
-  // ring, two work-groups per CU (the amplitude rows, 8 NT registers, leave room
-  // for two waves per SIMD).  With screening: small bases (NT <= 12) eight waves
-  // share double-buffered tiles; up to 400 functions one tile buffer and two
-  // work-groups per CU; beyond, double-buffered with one wave per SIMD.
-  // npts_pad is a multiple of 256.
-  constexpr int W = NT <= 12 ? 8 : 4;
-  constexpr int NBUF = (NT > 12 && NT <= 25) ? 1 : 2;
-  if constexpr (NT >= 8 && NT <= 25) {
-    if (!h->bmask) {
-      hipLaunchKernelGGL(k_density_ring<NT>, dim3(nblocks(h->npts_pad, 64)), dim3(256), 0, h->stream, h->phi,
-                         h->ldphi, h->pfrag, h->rho);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((k_density<NT, W, NBUF>), dim3(nblocks(h->npts_pad, 16 * W)), dim3(64 * W), 0, h->stream,
-                     h->phi, h->ldphi, h->pfrag, h->rho, h->bmask);
 }
 
 template <int NT>
@@ -3026,18 +3007,20 @@ int launch_density(dg_handle* h, const double* dP) {
       }
     });
   return run(h, "density", [&] {
-    switch (h->ntb) {
-#define DG_NT(N) \
-  case N:        \
-    launch_density_nt<N>(h); \
+    for (const DensityClass& k : h->dclass) {
+      const dim3 grid(k.count), block(256);
+      switch (k.n) {
+#define DG_N(N)                                                                                              \
+  case N:                                                                                                    \
+    hipLaunchKernelGGL(k_density_ring<N>, grid, block, 0, h->stream, h->phi, h->ldphi, h->pfrag, h->rho,     \
+                       h->dblocks + k.first, h->dtiles + 2 * k.first, h->ntb);                                      \
     break;
-      DG_NT(1) DG_NT(2) DG_NT(3) DG_NT(4) DG_NT(5) DG_NT(6) DG_NT(7) DG_NT(8) DG_NT(9) DG_NT(10) DG_NT(11)
-      DG_NT(12) DG_NT(13) DG_NT(14) DG_NT(15) DG_NT(16) DG_NT(17) DG_NT(18) DG_NT(19) DG_NT(20) DG_NT(21)
-      DG_NT(22) DG_NT(23) DG_NT(24) DG_NT(25) DG_NT(26) DG_NT(27) DG_NT(28) DG_NT(29) DG_NT(30) DG_NT(31)
-      DG_NT(32)
-#undef DG_NT
-      default:
-        break;
+        DG_N(4) DG_N(6) DG_N(8) DG_N(9) DG_N(10) DG_N(11) DG_N(12) DG_N(13) DG_N(14) DG_N(15) DG_N(16) DG_N(18)
+        DG_N(20) DG_N(22) DG_N(25) DG_N(28) DG_N(32)
+#undef DG_N
+        default:
+          break;
+      }
     }
   });
 }
@@ -3115,8 +3098,9 @@ int stage_density(dg_handle* h, const double* dP) {
   const long nfrag = 128L * h->ntb * (h->ntb + 1);
   if (h->ntb > 7)  // the persistent kernel forms its fragments itself
     DG_TRY(run(h, "pfrag", [&] {
-      hipLaunchKernelGGL(k_pfrag, dim3(nblocks(nfrag, 256)), dim3(256), 0, h->stream, dP, h->nbf, h->ntb,
-                         h->pfrag);
+      const unsigned nfb = nblocks(nfrag, 256);
+      hipLaunchKernelGGL(k_pfrag, dim3(nfb + nblocks(h->nempty, 4)), dim3(256), 0, h->stream, dP, h->nbf, h->ntb,
+                         h->pfrag, nfb, h->dempty, h->nempty, h->rho);
     }));
   DG_TRY(launch_density(h, dP));
   h->last_P = dP;
@@ -3312,40 +3296,25 @@ void launch_contract_small(dg_handle* h, const double* u0, const double* u1, int
 }
 
 // two outputs on 4 x 2 tile blocks, one output on 4 x 4 (the same 16 MFMAs per step);
-// list/loff (optional): point-block lists per tile block to use instead of the
-// handle's (the screened kernel then runs whatever the handle's screening)
 template <typename T, int NOUT>
-void launch_contract2d(dg_handle* h, const T* phi, const double* u0, const double* u1, const int* list = nullptr,
-                       const int* loff = nullptr) {
+void launch_contract2d(dg_handle* h, const T* phi, const double* u0, const double* u1) {
   constexpr int NJ = NOUT == 2 ? 2 : 4;
   const TileBlocks& t = h->tb[NOUT == 2 ? 0 : 1];
-  const int* bl = list ? list : t.list;
-  const int* bo = list ? loff : t.loff;
-  const bool dense = h->screen == 0.0 && !list;
-  const dim3 grid(round_up((long)t.ncb * t.nsplit, kXcds));
+  const dim3 grid(t.nwg);
   if constexpr (sizeof(T) == 8) {
     constexpr int D = NJ == 2 ? 4 : 3;  // ring slots: 3 work-groups per CU within 160 KB of LDS
-    if (dense)
-      hipLaunchKernelGGL((k_contract2d_lds<NOUT, NJ, D, true>), grid, dim3(256), 0, h->stream, phi, h->ldphi, u0, u1,
-                         t.cb, bl, bo, t.order, 4 * t.ncb, t.nsplit, h->cpart);
-    else
-      hipLaunchKernelGGL((k_contract2d_lds<NOUT, NJ, D, false>), grid, dim3(256), 0, h->stream, phi, h->ldphi, u0,
-                         u1, t.cb, bl, bo, t.order, 4 * t.ncb, t.nsplit, h->cpart);
+    hipLaunchKernelGGL((k_contract2d_lds<NOUT, NJ, D>), grid, dim3(256), 0, h->stream, phi, h->ldphi, u0, u1, t.cb,
+                       t.list, t.order, h->cpart);
   } else {
     constexpr int D = NJ == 2 ? 12 : 9;  // ring slots: 2 work-groups per CU within 160 KB of LDS
-    if (dense)
-      hipLaunchKernelGGL((k_contract2d_lds_f32<NOUT, NJ, D, true>), grid, dim3(256), 0, h->stream, phi, h->ldphi,
-                         u0, u1, t.cb, bl, bo, t.order, 4 * t.ncb, t.nsplit, h->cpart);
-    else
-      hipLaunchKernelGGL((k_contract2d_lds_f32<NOUT, NJ, D, false>), grid, dim3(256), 0, h->stream, phi, h->ldphi,
-                         u0, u1, t.cb, bl, bo, t.order, 4 * t.ncb, t.nsplit, h->cpart);
+    hipLaunchKernelGGL((k_contract2d_lds_f32<NOUT, NJ, D>), grid, dim3(256), 0, h->stream, phi, h->ldphi, u0, u1,
+                       t.cb, t.list, t.order, h->cpart);
   }
 }
 
 // sa (optional): the build's scalars, evaluated by one more work-group of the reduction
-// list/loff (optional, one output, 2-D path): point-block lists per tile block
 int stage_contract(dg_handle* h, const double* u0, const double* u1, double* out0, double* out1,
-                   const ScalarArgs* sa = nullptr, const int* list = nullptr, const int* loff = nullptr) {
+                   const ScalarArgs* sa = nullptr) {
   const int nout = u1 ? 2 : 1;
   const bool mx = h->precision == DG_PREC_MIXED;
   // up to 80 functions the dense all-tiles kernel (FP64, or FP32 in mixed mode)
@@ -3364,7 +3333,7 @@ int stage_contract(dg_handle* h, const double* u0, const double* u1, double* out
       if (nout == 2)
         launch_contract2d<double, 2>(h, h->phi, u0, u1);
       else
-        launch_contract2d<double, 1>(h, h->phi, u0, u0, list, loff);
+        launch_contract2d<double, 1>(h, h->phi, u0, u0);
     }
   }));
   const bool two_d = !small;
@@ -3374,8 +3343,8 @@ int stage_contract(dg_handle* h, const double* u0, const double* u1, double* out
   const unsigned nb = nblocks((long)ng * nout * 1024, 16) + (sa ? 1 : 0);
   return run(h, "contract_reduce", [&] {
     hipLaunchKernelGGL(k_contract_reduce, dim3(nb), dim3(256), 0, h->stream, h->cpart,
-                       small ? h->nsplit_small : tb.nsplit, ng, nout, two_d ? tb.groups : h->blocks, h->nbf,
-                       out0, out1, sa ? *sa : none);
+                       h->nsplit_small, ng, nout, two_d ? tb.groups : h->blocks, two_d ? tb.slot0 : nullptr,
+                       h->nbf, out0, out1, sa ? *sa : none);
   });
 }
 
@@ -3407,6 +3376,140 @@ int sync(dg_handle* h) {
 int copy_out(dg_handle* h, double* dst, const double* src, size_t n) {
   HIP_TRY(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, h->stream));
   return sync(h);
+}
+
+// The density's launches beyond 7 tiles: the blocks sorted by the number of
+// tiles that count there, a launch for every kernel size (kDensityTiles) that
+// at least kDensityClassMin blocks come to; fewer join the next larger one.
+constexpr int kDensityTiles[] = {4, 6, 8, 9, 10, 11, 12, 13, 14, 15, 16, 18, 20, 22, 25, 28, 32};
+constexpr long kDensityClassMin = 512;
+int density_classes(dg_handle* h, const std::vector<unsigned>& mk) {
+  const int nt = h->ntb;
+  std::vector<std::vector<int>> by(nt + 1);
+  for (size_t b = 0; b < mk.size(); ++b) by[__builtin_popcount(mk[b])].push_back((int)b);
+  const std::vector<int> empty = by[0];
+  by[0].clear();
+  std::vector<int> blocks;
+  std::vector<unsigned char> tiles;
+  std::vector<int> wait;  // blocks of fewer tiles, not yet in a launch
+  int done = 0;
+  for (int n : kDensityTiles) {
+    for (; done < std::min(n, nt); ++done) wait.insert(wait.end(), by[done + 1].begin(), by[done + 1].end());
+    if (wait.empty() || (n < nt && (long)wait.size() < kDensityClassMin)) continue;
+    h->dclass.push_back({n, (long)blocks.size(), (long)wait.size()});
+    for (int b : wait) {
+      unsigned char id[32];
+      std::memset(id, 255, 32);
+      for (int t = 0, r = 0; t < nt; ++t)
+        if ((mk[b] >> t) & 1u) id[r++] = (unsigned char)t;
+      tiles.insert(tiles.end(), id, id + 32);
+      blocks.push_back(b);
+    }
+    wait.clear();
+  }
+  std::reverse(h->dclass.begin(), h->dclass.end());
+  h->nempty = (int)empty.size();
+  DG_TRY(dalloc(&h->dblocks, blocks.size()));
+  DG_TRY(dalloc(&h->dtiles, tiles.size() / 16));
+  DG_TRY(dalloc(&h->dempty, empty.size()));
+  HIP_TRY(hipMemcpy(h->dblocks, blocks.data(), blocks.size() * 4, hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(h->dtiles, tiles.data(), tiles.size(), hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(h->dempty, empty.data(), empty.size() * 4, hipMemcpyHostToDevice));
+  return DG_OK;
+}
+
+// The tiles that count per 64-point block (k_block_mask) and, for the 2-D
+// contraction, the point blocks of every tile block and the order its
+// work-groups run in.  Without screening a tile counts where an amplitude
+// exceeds kAmpReach = 2^-106, the square of an FP64 rounding: a product with a
+// smaller amplitude lies as far below the last bit of a sum of order one as
+// that bit lies below the sum, so leaving it out changes no digit of rho, J or
+// XC.  The Gaussians of a 6-31G alkane end there at about 21 bohr, so that of
+// C30H62's tile pairs a third are left in the density and half in the
+// contraction; every grid also has shells beyond all its functions (8 % of
+// the blocks at 75 radial nodes).  Bases of at most 5 tiles keep the kernels
+// that walk every tile.
+int tile_reach(dg_handle* h, const std::vector<int> (&cbs)[2]) {
+  const long nblk = h->npts_pad / 64;
+  const bool two_d = h->ntb > 5;
+  if (h->screen == 0.0 && !two_d) return DG_OK;
+  DG_TRY(dalloc(&h->bmask, nblk));
+  DG_TRY(run(h, "block_mask", [&] {
+    hipLaunchKernelGGL(k_block_mask, dim3(nblk), dim3(64), 0, h->stream, h->phi, h->ldphi, h->ntb,
+                       h->screen > 0.0 ? h->screen : kAmpReach, h->bmask);
+  }));
+  if (!two_d) return DG_OK;
+  std::vector<unsigned> mk(nblk);
+  HIP_TRY(hipMemcpyAsync(mk.data(), h->bmask, nblk * 4, hipMemcpyDeviceToHost, h->stream));
+  DG_TRY(sync(h));
+  if (h->ntb > 7) DG_TRY(density_classes(h, mk));
+  size_t ncpart = 0;
+  for (int q = 0; q < 2; ++q) {
+    TileBlocks& t = h->tb[q];
+    const std::vector<int>& c = cbs[q];
+    std::vector<int> list, off;
+    const bool mx = h->precision == DG_PREC_MIXED;
+    const long parts = std::max(1L, std::min({512L, 6L * h->cus / t.ncb, nblk}));
+    tile_block_lists(mk, c, mx ? parts : 0, h->screen > 0.0, list, off);
+    // Work-groups of about equal cost: a step costs its MFMAs (one a tile pair and
+    // output) and as much as 13 more for its copies and barriers (with 3 instead,
+    // C10H22's contraction takes 455 us for 425).  Many small ones, because those
+    // that run together then read the same rows and the last round is short: 16
+    // rounds of the resident slots (3 FP64 / 2 FP32 work-groups per CU), as long as a
+    // work-group keeps some 20 point blocks to spread its partial sums over (C30H62,
+    // two outputs: 4 rounds 6.80 ms, 8 6.29, 16 5.88, 32 5.81 and 60 us more in the
+    // reduction; C10H22, which comes to 4: 2 rounds 517 us, 4 425, 8 438).
+    std::vector<long> cost(t.ncb, 0);
+    long total = 0;
+    for (int b = 0; b < t.ncb; ++b) {
+      for (int r = 0; r < c[4 * b + 1]; ++r)
+        for (int u = 0; u < c[4 * b + 3]; ++u) cost[b] += (c[4 * b] + r <= c[4 * b + 2] + u) ? 2 - q : 0;
+      cost[b] += 13;
+      total += cost[b] * (off[b + 1] - off[b]);
+    }
+    const long slots = (long)h->cus * (mx ? 2 : 3);
+    const long rounds = std::max(1L, std::min(16L, (long)list.size() / (20 * slots)));
+    const long each = std::max(1L, total / (rounds * slots));
+    std::vector<int4> job;
+    std::vector<int> slot0(t.ncb + 1, 0);
+    for (int b = 0; b < t.ncb; ++b) {
+      const long cnt = off[b + 1] - off[b];
+      const long ns = std::max(1L, std::min((cost[b] * cnt + each - 1) / each, cnt));
+      auto cut = [&](long k) {  // mixed precision: after the end of a group
+        long e = cnt * k / ns;
+        while (mx && e > 0 && e < cnt && !(list[off[b] + e - 1] & kGroupEnd)) ++e;
+        return (int)e;
+      };
+      for (long k = 0; k < ns; ++k)
+        job.push_back(make_int4(b, off[b] + cut(k), cut(k + 1) - cut(k), slot0[b] + (int)k));
+      slot0[b + 1] = slot0[b] + (int)ns;
+    }
+    ncpart = std::max(ncpart, job.size() * 4 * (q ? 1 : 2) * 1024);
+    // By first point block, cut into kXcds ranges of equal cost: an XCD's
+    // work-groups share the rows they read.  (Each range longest first, which the
+    // many work-groups make needless, takes C10H22 from 425 to 509 us.)
+    auto first = [&](const int4& x) { return x.z ? list[x.y] & ~kGroupEnd : 0; };
+    std::stable_sort(job.begin(), job.end(), [&](const int4& x, const int4& y) { return first(x) < first(y); });
+    std::vector<int> end(kXcds, (int)job.size());
+    long sum = 0;
+    for (int i = 0, x = 0; i < (int)job.size(); ++i) {
+      for (; x < kXcds - 1 && sum * kXcds >= total * (x + 1); ++x) end[x] = i;
+      sum += cost[job[i].x] * job[i].z;
+    }
+    int per = 1;
+    for (int x = 0; x < kXcds; ++x) per = std::max(per, end[x] - (x ? end[x - 1] : 0));
+    std::vector<int4> order((size_t)per * kXcds, make_int4(-1, 0, 0, 0));
+    for (int x = 0; x < kXcds; ++x)
+      std::copy(job.begin() + (x ? end[x - 1] : 0), job.begin() + end[x], order.begin() + (size_t)per * x);
+    t.nwg = (int)order.size();
+    DG_TRY(dalloc(&t.list, std::max<size_t>(list.size(), 1)));
+    DG_TRY(dalloc(&t.slot0, slot0.size()));
+    DG_TRY(dalloc(&t.order, order.size()));
+    HIP_TRY(hipMemcpy(t.list, list.data(), list.size() * 4, hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(t.slot0, slot0.data(), slot0.size() * 4, hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(t.order, order.data(), order.size() * sizeof(int4), hipMemcpyHostToDevice));
+  }
+  return dalloc(&h->cpart, ncpart);
 }
 
 // T = Phi P buffers (the adjoint's force terms and the density gradients), on first use.
@@ -3810,31 +3913,6 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
     // small contraction: exactly one round of resident work-groups (two per CU);
     // a partial second round measured slower, and so did fewer splits
     h->nsplit_small = (int)std::max(1L, std::min(2L * cus, h->npts_pad / 256));
-    // 2-D contraction: splits per tile block such that the work-groups make about
-    // three rounds of the resident slots (3 FP64 / 2 FP32 work-groups per CU); with
-    // the longest blocks first, the short ones even out the last round (C30H62: one
-    // round 14.3 ms, two 12.8, three 12.35, four 12.4)
-    const long slots = (long)cus * (h->precision == DG_PREC_MIXED ? 2 : 3);
-    for (int q = 0; q < 2; ++q) {
-      TileBlocks& t = h->tb[q];
-      const std::vector<int>& c = cbs[q];
-      t.nsplit = (int)std::max(1L, std::min(std::min(512L, 3 * slots / std::max(t.ncb, 1)), h->npts_pad / 64));
-      // virtual work-group order of the 2-D contraction: split-major, each XCD's range
-      // re-ordered by decreasing tile pairs of the block (stable)
-      const long nv = (long)t.ncb * t.nsplit, per = round_up(nv, kXcds) / kXcds;
-      std::vector<int> work(std::max(t.ncb, 1), 0);
-      for (int b = 0; b < t.ncb; ++b)
-        for (int r = 0; r < c[4 * b + 1]; ++r)
-          for (int u = 0; u < c[4 * b + 3]; ++u) work[b] += (c[4 * b] + r <= c[4 * b + 2] + u) ? 1 : 0;
-      std::vector<int2> order(std::max<long>(nv, 1));
-      for (long v = 0; v < nv; ++v)
-        order[v] = make_int2((int)(v % std::max(t.ncb, 1)), (int)(v / std::max(t.ncb, 1)));
-      for (long x0 = 0; x0 < nv; x0 += per)
-        std::stable_sort(order.begin() + x0, order.begin() + std::min(nv, x0 + per),
-                         [&](const int2& a, const int2& b) { return work[a.x] > work[b.x]; });
-      DG_TRY(dalloc(&t.order, order.size()));
-      HIP_TRY(hipMemcpy(t.order, order.data(), order.size() * sizeof(int2), hipMemcpyHostToDevice));
-    }
   }
 
   // allocations
@@ -3892,10 +3970,7 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
   DG_TRY(dalloc(&h->coef, h->nitems > 0 ? (size_t)h->natoms * (h->nrad + 1) * h->nlm * 4 : 1));
   DG_TRY(dalloc(&h->mono, mono.size()));
   DG_TRY(dalloc(&h->coef_grp, cgrp.size() / 4));
-  // partials: two outputs of the 4 x 2 blocks, one of the 4 x 4 blocks
-  DG_TRY(dalloc(&h->cpart, std::max({(size_t)h->nsplit_small * h->ngroups * 2 * 1024,
-                                      (size_t)h->tb[0].nsplit * h->tb[0].ncb * 4 * 2 * 1024,
-                                      (size_t)h->tb[1].nsplit * h->tb[1].ncb * 4 * 1024})));
+  if (h->ntb <= 5) DG_TRY(dalloc(&h->cpart, (size_t)h->nsplit_small * h->ngroups * 2 * 1024));
   for (int q = 0; q < 2; ++q) {
     DG_TRY(dalloc(&h->tb[q].cb, cbs[q].size()));
     DG_TRY(dalloc(&h->tb[q].groups, cbg[q].size()));
@@ -3980,27 +4055,7 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
     }));
   }
   DG_TRY(sort_items(h));
-  {
-    const long nblk = np / 64;
-    std::vector<unsigned> mk(nblk, 0xffffffffu);
-    if (h->screen > 0.0) {
-      DG_TRY(dalloc(&h->bmask, nblk));
-      DG_TRY(run(h, "block_mask", [&] {
-        hipLaunchKernelGGL(k_block_mask, dim3(nblk), dim3(64), 0, h->stream, h->phi, h->ldphi, h->ntb, h->screen,
-                           h->bmask);
-      }));
-      HIP_TRY(hipMemcpyAsync(mk.data(), h->bmask, nblk * 4, hipMemcpyDeviceToHost, h->stream));
-      DG_TRY(sync(h));
-    }
-    for (int q = 0; q < 2; ++q) {
-      std::vector<int> l2, o2;
-      tile_block_lists(mk, cbs[q], l2, o2);
-      DG_TRY(dalloc(&h->tb[q].list, std::max<size_t>(l2.size(), 1)));
-      DG_TRY(dalloc(&h->tb[q].loff, o2.size()));
-      HIP_TRY(hipMemcpy(h->tb[q].list, l2.data(), l2.size() * 4, hipMemcpyHostToDevice));
-      HIP_TRY(hipMemcpy(h->tb[q].loff, o2.data(), o2.size() * 4, hipMemcpyHostToDevice));
-    }
-  }
+  DG_TRY(tile_reach(h, cbs));
   DG_TRY(sync(h));
   guard.release();
   *out = h;
@@ -4266,29 +4321,9 @@ int dg_xc_adjoint(dg_handle* h, int hold_c, double* dEdP, double* grad) {
   }));
   if (dEdP) {
     // dE/dP = Phi^T diag(udp) Phi with the FP64 contraction in either precision mode.
-    // Unscreened handles on the 2-D path take, per tile block, only the point
-    // blocks where both its row and its column tiles are within reach
-    // (k_tile_mask; the terms left out are below e^-100 of an amplitude).
-    const bool lists = h->screen == 0.0 && h->ntb > 5 && h->ntb <= 32;
-    if (lists && !h->adj_list) {
-      DG_TRY(ensure_tile_mask(h));
-      const long nblk_m = h->npts_pad / 64;
-      std::vector<unsigned> mk(nblk_m);
-      std::vector<int> cb(4 * (size_t)h->tb[1].ncb), l2, o2;
-      HIP_TRY(hipMemcpyAsync(mk.data(), h->adj_tmask, nblk_m * 4, hipMemcpyDeviceToHost, h->stream));
-      HIP_TRY(hipMemcpyAsync(cb.data(), h->tb[1].cb, cb.size() * 4, hipMemcpyDeviceToHost, h->stream));
-      DG_TRY(sync(h));
-      tile_block_lists(mk, cb, l2, o2);
-      DG_TRY(dalloc(&h->adj_list, std::max<size_t>(l2.size(), 1)));
-      DG_TRY(dalloc(&h->adj_loff, o2.size()));
-      HIP_TRY(hipMemcpyAsync(h->adj_list, l2.data(), l2.size() * 4, hipMemcpyHostToDevice, h->stream));
-      HIP_TRY(hipMemcpyAsync(h->adj_loff, o2.data(), o2.size() * 4, hipMemcpyHostToDevice, h->stream));
-      DG_TRY(sync(h));
-    }
     const int saved = h->precision;
     h->precision = DG_PREC_FP64;
-    const int rc = stage_contract(h, h->adj_udp, nullptr, h->adj_dP, nullptr, nullptr, lists ? h->adj_list : nullptr,
-                                  lists ? h->adj_loff : nullptr);
+    const int rc = stage_contract(h, h->adj_udp, nullptr, h->adj_dP, nullptr);
     h->precision = saved;
     DG_TRY(rc);
     DG_TRY(copy_out(h, dEdP, h->adj_dP, (size_t)h->nbf * h->nbf));

@@ -67,10 +67,11 @@ typedef struct {
   int lmax;       /* spherical-harmonic cut-off of the Hartree expansion */
   int precision;  /* DG_PREC_FP64 or DG_PREC_MIXED */
   /* Amplitude screening (no counterpart in the reference, which sums every
-   * basis function at every point): 0 keeps every product; screen > 0 skips,
-   * in the density and in the Fock contractions, each 64-point block's 16-wide
-   * groups of basis functions whose |phi| stays at or below screen on the
-   * whole block.  Single-molecule handles only. */
+   * basis function at every point): screen > 0 skips, in the density and in
+   * the Fock contractions, each 64-point block's 16-wide groups of basis
+   * functions whose |phi| stays at or below screen on the whole block; 0 skips
+   * only those at or below 2^-106 (the square of an FP64 rounding, which no digit
+   * of the sums depends on).  Single-molecule handles only. */
   double screen;
 } dg_grid_params;
 
