@@ -391,7 +391,7 @@ int batch_alloc(dg_handle* h, const BatchSpec* bs, const std::vector<int>&) {
   DG_TRY(dalloc(&h->bchunks, cap));
   DG_TRY(dalloc(&h->mol_chunk0, nm + 1));
   if (h->cpart) {
-    HIP_TRY(hipFree(h->cpart));
+    dfree(h->cpart);
     h->cpart = nullptr;
   }
   DG_TRY(dalloc(&h->cpart, cap / 3 * 2 * 768));

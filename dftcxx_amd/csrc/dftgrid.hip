@@ -18,6 +18,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <list>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -1449,7 +1450,7 @@ __global__ __launch_bounds__(256, 3) void k_contract2d_lds(const double* __restr
     __syncthreads();
     for (int e = threadIdx.x; e < 4 * NJ * 256; e += 256) {
       const int r = e / (NJ * 256), t = (e >> 8) % NJ, rem = e & 255;
-      part[((4L * job.w + r) * NOUT + o) * 1024 + t * 256 + rem] = red[e];
+      part[((4L * job.w + r) * NOUT + o) * (NJ * 256) + t * 256 + rem] = red[e];
     }
   }
 }
@@ -1593,7 +1594,7 @@ __global__ __launch_bounds__(256, 2) void k_contract2d_lds_f32(const float* __re
     __syncthreads();
     for (int e = threadIdx.x; e < 4 * NJ * 256; e += 256) {
       const int r = e / (NJ * 256), t = (e >> 8) % NJ, rem = e & 255;
-      part[((4L * job.w + r) * NOUT + o) * 1024 + t * 256 + rem] = red[e];
+      part[((4L * job.w + r) * NOUT + o) * (NJ * 256) + t * 256 + rem] = red[e];
     }
   }
 }
@@ -2653,7 +2654,7 @@ __device__ __forceinline__ flt4 mfma16x16x4f32(float a, float b, flt4 c) {
 __global__ __launch_bounds__(256) void k_contract_reduce(const double* __restrict__ part, int nsplit,
                                                          int ngroups, int nout,
                                                          const int* __restrict__ groups,
-                                                         const int* __restrict__ slot0, int nbf, double* out0,
+                                                         const int* __restrict__ slot0, int nj, int nbf, double* out0,
                                                          double* out1, ScalarArgs sa) {
   if (sa.scalars && blockIdx.x == gridDim.x - 1) {
     scalars_block(sa);
@@ -2674,8 +2675,9 @@ __global__ __launch_bounds__(256) void k_contract_reduce(const double* __restric
     if (slot0) {
       const int s0 = slot0[grp >> 2];
       nsplit = slot0[(grp >> 2) + 1] - s0;
-      stride = 4096L * nout;
-      src = part + ((4L * s0 + (grp & 3)) * nout + o) * 1024 + idx;
+      const int tw = 256 * nj;  // a group's share of a slot
+      stride = 4L * tw * nout;
+      src = part + ((4L * s0 + (grp & 3)) * nout + o) * tw + idx;
     }
     // eight splits' partials loaded per round (one memory latency), added in split order
     int sp = r;
@@ -2734,10 +2736,94 @@ __global__ void k_mfma_probe(double* out) {
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
+// Device memory of handles and calls that have ended, kept for the next ones: a
+// program that makes a grid per geometry allocates the same sizes again and again,
+// and hipMalloc, hipFree and the mapping behind them take longer than the set-up's
+// kernels (C10H22 / 75 x 302: closing a handle 5.2 ms, the set-up's kernels 2).
+// At most kPoolMax per process, the longest kept leaving first, and all of it
+// before an allocation fails.  A block comes here only when the work that used it
+// is over (its owner's stream has been waited for), so any stream of the device
+// may have it next; what it holds then is not defined, as with hipMalloc.
+class DevicePool {
+ public:
+  hipError_t take(void** p, size_t bytes) {
+    bytes = std::max<size_t>((bytes + 511) / 512 * 512, 512);
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    {
+      std::lock_guard<std::mutex> lock(m_);
+      auto best = kept_.end();
+      for (auto it = kept_.begin(); it != kept_.end(); ++it)
+        if (it->dev == dev && it->bytes >= bytes && it->bytes <= bytes + bytes / 8 &&
+            (best == kept_.end() || it->bytes < best->bytes))
+          best = it;
+      if (best != kept_.end()) {
+        *p = best->p;
+        used_[best->p] = *best;
+        held_ -= best->bytes;
+        kept_.erase(best);
+        return hipSuccess;
+      }
+    }
+    e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      std::lock_guard<std::mutex> lock(m_);
+      while (!kept_.empty()) drop_oldest();
+      e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) return e;
+    std::lock_guard<std::mutex> lock(m_);
+    used_[*p] = Block{*p, bytes, dev};
+    return hipSuccess;
+  }
+  void give(void* p) {
+    if (!p) return;
+    std::lock_guard<std::mutex> lock(m_);
+    auto it = used_.find(p);
+    if (it == used_.end()) return;
+    const Block b = it->second;
+    used_.erase(it);
+    if (b.bytes > kPoolMax) {
+      (void)hipFree(p);
+      return;
+    }
+    while (held_ + b.bytes > kPoolMax) drop_oldest();
+    kept_.push_back(b);
+    held_ += b.bytes;
+  }
+
+ private:
+  struct Block {
+    void* p;
+    size_t bytes;
+    int dev;
+  };
+  void drop_oldest() {
+    held_ -= kept_.front().bytes;
+    (void)hipFree(kept_.front().p);
+    kept_.pop_front();
+  }
+  static constexpr size_t kPoolMax = (size_t)2 << 30;  // under 1 % of the device's memory
+  std::mutex m_;
+  std::list<Block> kept_;  // oldest first
+  std::map<void*, Block> used_;
+  size_t held_ = 0;
+};
+
+DevicePool& pool() {
+  static DevicePool* p = new DevicePool;  // not destroyed: handles may outlive static objects
+  return *p;
+}
+
+// Returns a buffer no pending work uses.
+void dfree(void* p) { pool().give(p); }
+
 template <typename T>
 int dalloc(T** p, size_t n) {
   if (n == 0) n = 1;
-  hipError_t e = hipMalloc((void**)p, n * sizeof(T));
+  hipError_t e = pool().take((void**)p, n * sizeof(T));
   if (e != hipSuccess) {
     *p = nullptr;
     return fail(DG_ERR_ALLOC, std::string("hipMalloc of ") + std::to_string(n * sizeof(T)) +
@@ -2858,6 +2944,8 @@ struct dg_handle {
   std::map<std::string, ProfStat> stats;
 
   ~dg_handle() {
+    // the buffers go to the next owner: nothing of this handle may still run
+    if (stream && hipStreamSynchronize(stream) != hipSuccess) (void)hipDeviceSynchronize();
     double* bufs[] = {atoms, invR,  rad,   wrad,   leb,   px,     py,    pz,   w,     wb,
                       phi,   pr_alpha, pr_cn0, pr_cn1, P, pfrag, rho,  uxc,   exd,   uJ,
                       V,     vcell, vpart, q,      qc,    exc_part, scalars, ylm, minvT, shc,
@@ -2865,28 +2953,28 @@ struct dg_handle {
                       adj_ub, adj_ab, adj_udp, adj_T, adj_frag, adj_part, adj_mot, adj_lam, adj_out, adj_dP,
                       mol_z, mol_fac, mol_qraw, atom_exc, atom_ej, qpart, uG, coef, mono, sh_amin};
     for (double* b : bufs)
-      if (b) (void)hipFree(b);
+      if (b) dfree(b);
     int* ibufs[] = {sh_atom, sh_L, sh_nprim, sh_off, sh_cgf, blocks, ntask, ash_start, ash_list, atom_order, dblocks, dempty,
                     atom_mol, mol_atom0, mol_shell0, mol_nbf, bchunks, mol_chunk0,
                     tb[0].cb, tb[0].groups, tb[0].list, tb[0].slot0, tb[1].cb, tb[1].groups, tb[1].list,
                     tb[1].slot0};
-    if (bmask) (void)hipFree(bmask);
-    if (dtiles) (void)hipFree(dtiles);
-    if (adj_tmask) (void)hipFree(adj_tmask);
+    if (bmask) dfree(bmask);
+    if (dtiles) dfree(dtiles);
+    if (adj_tmask) dfree(adj_tmask);
     for (TileBlocks& t : tb)
-      if (t.order) (void)hipFree(t.order);
-    if (vbase) (void)hipFree(vbase);
-    if (perm) (void)hipFree(perm);
-    if (items) (void)hipFree(items);
-    if (task) (void)hipFree(task);
-    if (coef_grp) (void)hipFree(coef_grp);
-    if (mol_poff) (void)hipFree(mol_poff);
+      if (t.order) dfree(t.order);
+    if (vbase) dfree(vbase);
+    if (perm) dfree(perm);
+    if (items) dfree(items);
+    if (task) dfree(task);
+    if (coef_grp) dfree(coef_grp);
+    if (mol_poff) dfree(mol_poff);
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (graph) (void)hipGraphDestroy(graph);
-    if (phf) (void)hipFree(phf);
-    if (ej_part) (void)hipFree(ej_part);
+    if (phf) dfree(phf);
+    if (ej_part) dfree(ej_part);
     for (int* b : ibufs)
-      if (b) (void)hipFree(b);
+      if (b) dfree(b);
     for (auto& e : pending) {
       (void)hipEventDestroy(e.e0);
       (void)hipEventDestroy(e.e1);
@@ -3344,7 +3432,7 @@ int stage_contract(dg_handle* h, const double* u0, const double* u1, double* out
   return run(h, "contract_reduce", [&] {
     hipLaunchKernelGGL(k_contract_reduce, dim3(nb), dim3(256), 0, h->stream, h->cpart,
                        h->nsplit_small, ng, nout, two_d ? tb.groups : h->blocks, two_d ? tb.slot0 : nullptr,
-                       h->nbf, out0, out1, sa ? *sa : none);
+                       nout == 2 ? 2 : 4, h->nbf, out0, out1, sa ? *sa : none);
   });
 }
 
@@ -3484,7 +3572,7 @@ int tile_reach(dg_handle* h, const std::vector<int> (&cbs)[2]) {
         job.push_back(make_int4(b, off[b] + cut(k), cut(k + 1) - cut(k), slot0[b] + (int)k));
       slot0[b + 1] = slot0[b] + (int)ns;
     }
-    ncpart = std::max(ncpart, job.size() * 4 * (q ? 1 : 2) * 1024);
+    ncpart = std::max(ncpart, job.size() * 4096);  // 4 NJ NOUT tiles a slot, 16 either way
     // By first point block, cut into kXcds ranges of equal cost: an XCD's
     // work-groups share the rows they read.  (Each range longest first, which the
     // many work-groups make needless, takes C10H22 from 425 to 509 us.)
@@ -3803,15 +3891,18 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
   for (int t = 0; t < h->nrad; ++t) knots[t] = rad[h->nrad - 1 - t];
   for (int t = 1; t < h->nrad; ++t) invh[t] = 1.0 / (knots[t] - knots[t - 1]);
   const std::vector<double> Sspl = dg::spline_slope_matrix(knots);  // [t][t'] row-major
+  std::vector<double> St(Sspl.size());                              // [t'][t]
+  for (int t = 0; t < h->nrad; ++t)
+    for (int tp = 0; tp < h->nrad; ++tp) St[(size_t)tp * h->nrad + t] = Sspl[(size_t)t * h->nrad + tp];
   std::vector<double> KD(minvT.size(), 0.0);
   for (int l = 0; l <= h->lmax; ++l)
     for (int k = 0; k < n2; ++k) {
       const double* ku = &minvT[((size_t)l * n2 + k) * h->nrad];  // ku[i], i = radial node
       double* kd = &KD[((size_t)l * n2 + k) * h->nrad];
-      for (int t = 0; t < h->nrad; ++t) {
-        double acc = 0.0;
-        for (int tp = 0; tp < h->nrad; ++tp) acc += Sspl[(size_t)t * h->nrad + tp] * ku[h->nrad - 1 - tp];
-        kd[t] = acc;
+      for (int tp = 0; tp < h->nrad; ++tp) {
+        const double v = ku[h->nrad - 1 - tp];
+        const double* st = &St[(size_t)tp * h->nrad];
+        for (int t = 0; t < h->nrad; ++t) kd[t] += st[t] * v;
       }
     }
   // spherical-harmonic recurrence constants per (l, m >= 0): {N_lm c_lm (the table
@@ -3977,7 +4068,7 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
   }
   DG_TRY(dalloc(&h->ej_part, h->npts_pad / 256));
   if (h->precision == DG_PREC_MIXED) {
-    HIP_TRY(hipMalloc((void**)&h->phf, (size_t)(np + 1) * h->ldphi * sizeof(float)));
+    DG_TRY(dalloc(&h->phf, (size_t)(np + 1) * h->ldphi));
   }
   DG_TRY(dalloc(&h->J, (size_t)h->packed));
   DG_TRY(dalloc(&h->XC, (size_t)h->packed));
@@ -4376,7 +4467,7 @@ int dg_get_amplitude_gradients(dg_handle* h, double* dphi) {
     });
     if (rc == DG_OK) rc = copy_out(h, dphi + p0 * 3 * h->nbf, buf, (size_t)n * 3 * h->nbf);
   }
-  (void)hipFree(buf);
+  dfree(buf);
   return rc;
 }
 
@@ -4396,7 +4487,7 @@ int dg_get_density_gradients(dg_handle* h, double* grad) {
                        h->zsum, nullptr, buf);
   });
   if (rc == DG_OK) rc = copy_out(h, grad, buf, (size_t)3 * h->npts);
-  (void)hipFree(buf);
+  dfree(buf);
   return rc;
 }
 
@@ -4416,7 +4507,7 @@ int dg_density_at_points(const dg_molecule* mol, const dg_basis* basis, long npt
     hipStream_t st = nullptr;
     ~Bufs() {
       if (st) (void)hipStreamSynchronize(st);
-      for (void* b : p) (void)hipFree(b);
+      for (void* b : p) dfree(b);
       if (st) (void)hipStreamDestroy(st);
     }
   } B;
@@ -4502,7 +4593,7 @@ int dg_mfma_probe(const double* a, const double* b, double* d) {
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipMemcpy(d, buf + 128, 256 * 8, hipMemcpyDeviceToHost);
-  (void)hipFree(buf);
+  dfree(buf);
   if (e != hipSuccess) return fail(DG_ERR_HIP, std::string("dg_mfma_probe: ") + hipGetErrorString(e));
   return DG_OK;
 }
@@ -4510,16 +4601,15 @@ int dg_mfma_probe(const double* a, const double* b, double* d) {
 int dg_mfma_probe_f32(const float* a, const float* b, float* d) {
   if (!a || !b || !d) return fail(DG_ERR_INVALID, "dg_mfma_probe_f32: null argument");
   float* buf = nullptr;
-  hipError_t e = hipMalloc((void**)&buf, (64 + 64 + 256) * sizeof(float));
-  if (e != hipSuccess) return fail(DG_ERR_ALLOC, "dg_mfma_probe_f32: hipMalloc failed");
-  e = hipMemcpy(buf, a, 64 * 4, hipMemcpyHostToDevice);
+  DG_TRY(dalloc(&buf, 64 + 64 + 256));
+  hipError_t e = hipMemcpy(buf, a, 64 * 4, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(buf + 64, b, 64 * 4, hipMemcpyHostToDevice);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_mfma_raw_f32, dim3(1), dim3(64), 0, 0, buf, buf + 64, buf + 128);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipMemcpy(d, buf + 128, 256 * 4, hipMemcpyDeviceToHost);
-  (void)hipFree(buf);
+  dfree(buf);
   if (e != hipSuccess) return fail(DG_ERR_HIP, std::string("dg_mfma_probe_f32: ") + hipGetErrorString(e));
   return DG_OK;
 }
@@ -4532,7 +4622,7 @@ int dg_selftest_mfma(int* ok) {
   hipLaunchKernelGGL(k_mfma_probe, dim3(1), dim3(64), 0, 0, d);
   std::vector<double> out(256);
   hipError_t e = hipMemcpy(out.data(), d, 256 * 8, hipMemcpyDeviceToHost);
-  (void)hipFree(d);
+  dfree(d);
   if (e != hipSuccess) return fail(DG_ERR_HIP, std::string("dg_selftest_mfma: ") + hipGetErrorString(e));
   int good = 1;
   for (int lane = 0; lane < 64; ++lane)

@@ -147,28 +147,32 @@ bool invert_matrix(int n, std::vector<double>& a) {
       for (int j = 0; j < n; ++j) std::swap(A(k, j), A(p, j));
       std::swap(perm[k], perm[p]);
     }
+    int end = n;  // past the row's last value
+    while (end > k + 1 && A(k, end - 1) == 0.0) --end;
     for (int i = k + 1; i < n; ++i) {
       A(i, k) /= A(k, k);
       const double f = A(i, k);
       if (f != 0.0)
-        for (int j = k + 1; j < n; ++j) A(i, j) -= f * A(k, j);
+        for (int j = k + 1; j < end; ++j) A(i, j) -= f * A(k, j);
     }
   }
-  // solve LU x = e_perm for every unit vector
-  std::vector<double> inv((size_t)n * n, 0.0), col(n);
-  for (int c = 0; c < n; ++c) {
-    for (int i = 0; i < n; ++i) col[i] = (perm[i] == c) ? 1.0 : 0.0;
-    for (int i = 0; i < n; ++i) {
-      double s = col[i];
-      for (int j = 0; j < i; ++j) s -= A(i, j) * col[j];
-      col[i] = s;
-    }
-    for (int i = n - 1; i >= 0; --i) {
-      double s = col[i];
-      for (int j = i + 1; j < n; ++j) s -= A(i, j) * col[j];
-      col[i] = s / A(i, i);
-    }
-    for (int i = 0; i < n; ++i) inv[(size_t)i * n + c] = col[i];
+  // solve LU X = P for all unit vectors together, row after row; the factors of a
+  // banded matrix are mostly zeros, which are passed over
+  std::vector<double> inv((size_t)n * n, 0.0);
+  auto take = [&](int i, int j) {  // row i -= A(i, j) row j
+    const double f = A(i, j);
+    if (f == 0.0) return;
+    double* x = &inv[(size_t)i * n];
+    const double* y = &inv[(size_t)j * n];
+    for (int c = 0; c < n; ++c) x[c] -= f * y[c];
+  };
+  for (int i = 0; i < n; ++i) {
+    inv[(size_t)i * n + perm[i]] = 1.0;
+    for (int j = 0; j < i; ++j) take(i, j);
+  }
+  for (int i = n - 1; i >= 0; --i) {
+    for (int j = i + 1; j < n; ++j) take(i, j);
+    for (int c = 0; c < n; ++c) inv[(size_t)i * n + c] /= A(i, i);
   }
   a.swap(inv);
   return true;
