@@ -1917,16 +1917,10 @@ __global__ __launch_bounds__(64 * W) void k_tmat(const double* __restrict__ phi,
 // is the order consumed; chunks of kDensityChunk units copied two ahead into
 // three LDS slots (48 KB: two work-groups of W = 4 waves per CU), one wait and
 // barrier per chunk.  Same chains and sums as k_tmat, so the same T.
-// With tmask (bit b of tmask[block]: tile b matters at the block's 64 points,
-// k_tile_mask), the block forms and writes only the column tiles in its mask
-// and sums only over the reduction tiles in it (the others' amplitudes are
-// below e^-100 there); the ring's copies, waits and barriers run unchanged.
 template <int NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_tmat_ring(
-    const double* __restrict__ phi, int ldphi, const double* __restrict__ frag, double* tmat,
-    const unsigned* __restrict__ tmask) {
+    const double* __restrict__ phi, int ldphi, const double* __restrict__ frag, double* tmat) {
   constexpr int C = kDensityChunk, U = NT * NT, NCH = (U + C - 1) / C;
-  const unsigned tm = tmask ? tmask[blockIdx.x] : ~0u;
   __shared__ double ring[3][C * 256];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int g = lane >> 4, c = lane & 15;
@@ -1949,30 +1943,111 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   };
 #pragma unroll
   for (int b = 0; b < NT; ++b) {
-    if ((tm >> b) & 1u) {
-      dbl4 d0 = {0.0, 0.0, 0.0, 0.0}, d1 = d0, d2 = d0, d3 = d0;
+    dbl4 d0 = {0.0, 0.0, 0.0, 0.0}, d1 = d0, d2 = d0, d3 = d0;
 #pragma unroll
-      for (int k = 0; k < NT; ++k) {
-        const int u = b * NT + k;
-        ring_step(u);
-        if ((tm >> k) & 1u) {
-          const double* cur = ring[(u / C) % 3] + (u - stream_start<C, U>(u / C)) * 256;
-          d0 = mfma16x16x4(cur[lane], f[4 * k], d0);
-          d1 = mfma16x16x4(cur[64 + lane], f[4 * k + 1], d1);
-          d2 = mfma16x16x4(cur[128 + lane], f[4 * k + 2], d2);
-          d3 = mfma16x16x4(cur[192 + lane], f[4 * k + 3], d3);
-        }
-      }
-      double* out = tmat + (p0 + c) * ldphi + 16 * b + g;
-      out[0] = (d0[0] + d1[0]) + (d2[0] + d3[0]);
-      out[4] = (d0[1] + d1[1]) + (d2[1] + d3[1]);
-      out[8] = (d0[2] + d1[2]) + (d2[2] + d3[2]);
-      out[12] = (d0[3] + d1[3]) + (d2[3] + d3[3]);
-    } else {
-#pragma unroll
-      for (int k = 0; k < NT; ++k) ring_step(b * NT + k);
+    for (int k = 0; k < NT; ++k) {
+      const int u = b * NT + k;
+      ring_step(u);
+      const double* cur = ring[(u / C) % 3] + (u - stream_start<C, U>(u / C)) * 256;
+      d0 = mfma16x16x4(cur[lane], f[4 * k], d0);
+      d1 = mfma16x16x4(cur[64 + lane], f[4 * k + 1], d1);
+      d2 = mfma16x16x4(cur[128 + lane], f[4 * k + 2], d2);
+      d3 = mfma16x16x4(cur[192 + lane], f[4 * k + 3], d3);
     }
+    double* out = tmat + (p0 + c) * ldphi + 16 * b + g;
+    out[0] = (d0[0] + d1[0]) + (d2[0] + d3[0]);
+    out[4] = (d0[1] + d1[1]) + (d2[1] + d3[1]);
+    out[8] = (d0[2] + d1[2]) + (d2[2] + d3[2]);
+    out[12] = (d0[3] + d1[3]) + (d2[3] + d3[3]);
   }
+}
+
+// T = Phi P where only the tiles that count on a block are wanted (the force
+// terms): a block of N tiles a work-group, the fragments gathered by tile as in
+// k_density_ring, both ways.  A column tile's N units come in chunks of CL, the
+// last of them filled up; the column tiles are a loop, the reduction is unrolled.
+// A tile's result is stored after the next chunk's wait, so that no wait is for a
+// store just issued.  Tiles that do not count are left as they are.
+// Bound by the FP64 MFMAs and, below some 10 tiles, by T's way to HBM and back;
+// C30H62's T 6.7 -> 4.7 ms against walking all tiles and skipping those out of reach.
+template <int N>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N <= 25 ? 2 : 1))) void
+k_tmat_tiles(const double* __restrict__ phi, int ldphi, const double* __restrict__ frag, double* tmat,
+             const int* __restrict__ blocks, const uint4* __restrict__ tiles, int nt) {
+  constexpr int CPR = (N + kDensityChunk - 1) / kDensityChunk, CL = 2 * ((N + 2 * CPR - 1) / (2 * CPR));
+  __shared__ double ring[3][CL * 256];
+  __shared__ int ids[32];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int g = lane >> 4, c = lane & 15;
+  const uint4 ta = tiles[2 * (long)blockIdx.x], tb = tiles[2 * (long)blockIdx.x + 1];
+  const unsigned tw[8] = {ta.x, ta.y, ta.z, ta.w, tb.x, tb.y, tb.z, tb.w};
+  if (threadIdx.x < 32) ids[threadIdx.x] = ((const unsigned char*)(tiles + 2 * (long)blockIdx.x))[threadIdx.x];
+  const long p0 = 64L * blocks[blockIdx.x] + wave * 16;
+  bare_barrier();
+  const double* row = phi + (p0 + c) * ldphi + 4 * g;
+  double f[4 * N];
+  int live = 0;
+#pragma unroll
+  for (int r = 0; r < N; ++r) {
+    const int t = (int)((tw[r >> 2] >> (8 * (r & 3))) & 255u);
+    const double* x = row + 16 * min(t, nt - 1);
+    live += t < nt ? 1 : 0;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) f[4 * r + v] = t < nt ? x[v] : 0.0;
+  }
+  const int nch = live * CPR;
+  const double* src = frag + (wave & 1) * 128 + lane * 2;
+  int cb = 0, cm = 0;  // the next chunk to copy: column tile, chunk of it
+  auto copy = [&](int slot) {
+    const int mine = ids[min(cm * CL + 2 * (lane & 3) + (wave >> 1), N - 1)];
+    const int col = __builtin_amdgcn_readfirstlane(ids[cb]) * nt;
+#pragma unroll
+    for (int q = 0; q < CL / 2; ++q) {
+      const int at = col + min(__builtin_amdgcn_readlane(mine, q), nt - 1);
+      __builtin_amdgcn_global_load_lds((const void*)(src + 256L * at),
+                                       (__attribute__((address_space(3))) void*)(&ring[slot][(wave + 4 * q) * 128]),
+                                       16, 0, 0);
+    }
+    if (++cm == CPR) {
+      cm = 0;
+      ++cb;
+    }
+  };
+  copy(0);
+  if (nch > 1) copy(1);
+  int j = 0, slot = 0;
+  dbl4 done = {0.0, 0.0, 0.0, 0.0};
+  auto store = [&](int b) {
+    double* out = tmat + (p0 + c) * ldphi + 16 * __builtin_amdgcn_readfirstlane(ids[b]) + g;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) out[4 * v] = done[v];
+  };
+  for (int b = 0; b < live; ++b) {
+    dbl4 d0 = {0.0, 0.0, 0.0, 0.0}, d1 = d0;
+#pragma unroll
+    for (int m = 0; m < CPR; ++m, ++j) {
+      if (j + 1 < nch)
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(CL / 2));
+      else
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+      bare_barrier();
+      if (m == 0 && b > 0) store(b - 1);
+      if (j + 2 < nch) copy(slot == 0 ? 2 : slot - 1);
+      const double* cur = &ring[slot][lane];
+      slot = slot == 2 ? 0 : slot + 1;
+#pragma unroll
+      for (int k = CL * m; k < N && k < CL * (m + 1); ++k) {
+        const double* a = cur + (k - CL * m) * 256;
+        d0 = mfma16x16x4(a[0], f[4 * k], d0);
+        d1 = mfma16x16x4(a[64], f[4 * k + 1], d1);
+        d0 = mfma16x16x4(a[128], f[4 * k + 2], d0);
+        d1 = mfma16x16x4(a[192], f[4 * k + 3], d1);
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) done[v] = d0[v] + d1[v];
+  }
+  store(live - 1);
 }
 
 // Value and gradient of component `comp` of a shell with radial sums
@@ -2010,55 +2085,24 @@ __device__ __forceinline__ void shell_grad(int L, int comp, double r0, double d0
 // primitive's exp(-alpha r^2) at least e^-100).
 constexpr double kShellReach = 100.0;
 
-// Function tiles the force terms read, per 64-point block: bit t of mask[blk]
-// is set when a shell with a function in tile t (16 functions) passes the
-// shell test at one of the block's points, with a 1 % margin on kShellReach so
-// that every shell k_force_basis takes is covered.  Four threads per point,
-// each taking every fourth shell; the bits are OR-ed over the block.
-__global__ __launch_bounds__(256) void k_tile_mask(const double* __restrict__ atoms, int nshell,
-                                                   const int* __restrict__ sh_atom, const int* __restrict__ sh_L,
-                                                   const int* __restrict__ sh_cgf, const double* __restrict__ sh_amin,
-                                                   long npts, const double* __restrict__ px,
-                                                   const double* __restrict__ py, const double* __restrict__ pz,
-                                                   unsigned* mask) {
-  __shared__ unsigned red[4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const long p = (long)blockIdx.x * 64 + lane;
-  unsigned m = 0;
-  if (p < npts) {
-    const double x = px[p], y = py[p], z = pz[p];
-    for (int s = wave; s < nshell; s += 4) {
-      const int a = sh_atom[s];
-      const double dx = x - atoms[4 * a], dy = y - atoms[4 * a + 1], dz = z - atoms[4 * a + 2];
-      const double r2 = dx * dx + dy * dy + dz * dz;
-      if (sh_amin[s] * r2 <= 1.01 * kShellReach) {
-        const int L = sh_L[s], i0 = sh_cgf[s], i1 = i0 + (L + 1) * (L + 2) / 2 - 1;
-        for (int t = i0 >> 4; t <= (i1 >> 4); ++t) m |= 1u << t;
-      }
-    }
-  }
-  for (int o = 32; o > 0; o >>= 1) m |= (unsigned)__shfl_xor((int)m, o);
-  if (lane == 0) red[wave] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) mask[blockIdx.x] = red[0] | red[1] | red[2] | red[3];
-}
-
 // Basis-centre and grid-motion terms of dE_xc/dR, one wave per 64 points.
 // For point p and atom A: g_A(p) = ub_p sum_{i on A} T_pi grad phi_i(r_p).
 // part[(A*3+d)*nblk + blk] = -4 sum_{p in blk} g_A(p)  (functions move with A)
 // mot[d*npts + p]          = +4 sum_A g_A(p)         (the point moves with its atom)
 // Shells are visited atom by atom through ash_start/ash_list (shells of atom
-// A are ash_list[ash_start[A] .. ash_start[A+1])).
+// A are ash_list[ash_start[A] .. ash_start[A+1])).  mask (may be null): the
+// function tiles that count per block, the only ones T is formed for.
 __global__ __launch_bounds__(64) void k_force_basis(
     const double* __restrict__ atoms, int natoms, const int* __restrict__ ash_start,
     const int* __restrict__ ash_list, const int* __restrict__ sh_L, const int* __restrict__ sh_nprim,
     const int* __restrict__ sh_off, const int* __restrict__ sh_cgf, const double* __restrict__ sh_amin,
     const double* __restrict__ alpha, const double* __restrict__ cn0, const double* __restrict__ cn1, long npts,
     const double* __restrict__ px, const double* __restrict__ py, const double* __restrict__ pz,
-    int ldphi, const double* __restrict__ tmat, const double* __restrict__ ub, long nblk, double* part,
-    double* mot) {
+    int ldphi, const double* __restrict__ tmat, const double* __restrict__ ub, long nblk,
+    const unsigned* __restrict__ mask, double* part, double* mot) {
   const long p = (long)blockIdx.x * 64 + threadIdx.x;
   const bool valid = p < npts;
+  const unsigned tiles = mask ? mask[blockIdx.x] : ~0u;
   const double x = valid ? px[p] : 0.0, y = valid ? py[p] : 0.0, z = valid ? pz[p] : 0.0;
   const double u = valid ? ub[p] : 0.0;
   const double* trow = tmat + (valid ? p : 0) * ldphi;
@@ -2072,6 +2116,8 @@ __global__ __launch_bounds__(64) void k_force_basis(
         const int s = ash_list[t];
         // every primitive's exp(-alpha r2) below e^-kShellReach (1e-43): the shell's
         // terms are below the rounding of the sums they would enter, and it is skipped
+        const int L = sh_L[s], nc = (L + 1) * (L + 2) / 2, i0 = sh_cgf[s];
+        if (!(((tiles >> (i0 >> 4)) | (tiles >> ((i0 + nc - 1) >> 4))) & 1u)) continue;
         if (sh_amin[s] * r2 > kShellReach) continue;
         double r0 = 0.0, d0 = 0.0, r1 = 0.0, d1 = 0.0;
         for (int k = 0; k < sh_nprim[s]; ++k) {
@@ -2080,16 +2126,16 @@ __global__ __launch_bounds__(64) void k_force_basis(
           const double m2a = -2.0 * alpha[q];
           r0 += cn0[q] * e;
           d0 += cn0[q] * m2a * e;
-          if (sh_L[s] == 2) {  // the xy, xz, yz functions' own norm
+          if (L == 2) {  // the xy, xz, yz functions' own norm
             r1 += cn1[q] * e;
             d1 += cn1[q] * m2a * e;
           }
         }
-        const int L = sh_L[s], nc = (L + 1) * (L + 2) / 2;
         for (int c = 0; c < nc; ++c) {
+          if (!((tiles >> ((i0 + c) >> 4)) & 1u)) continue;  // its T is not formed
           double gr[3];
           shell_grad(L, c, r0, d0, r1, d1, dx, dy, dz, gr);
-          const double tv = u * trow[sh_cgf[s] + c];
+          const double tv = u * trow[i0 + c];
           g[0] += tv * gr[0];
           g[1] += tv * gr[1];
           g[2] += tv * gr[2];
@@ -2856,10 +2902,19 @@ struct TileBlocks {
   int ncb = 0, nwg = 0;
 };
 
-// A launch of k_density_ring<n>: entries [first, first + count) of dblocks / dtiles.
-struct DensityClass {
-  int n;
-  long first, count;
+// The point blocks by the number of function tiles that count there: launches of
+// the kernels for n tiles over entries [first, first + count) of block / tile, the
+// blocks without any, and per block the tiles as bits.
+struct BlockClasses {
+  struct Launch {
+    int n;
+    long first, count;
+  };
+  std::vector<Launch> launch;
+  int *block = nullptr, *empty = nullptr;
+  uint4* tile = nullptr;
+  unsigned* mask = nullptr;
+  int nempty = 0;
 };
 
 struct dg_handle {
@@ -2902,12 +2957,8 @@ struct dg_handle {
   int4* coef_grp = nullptr;
   // screening masks
   double screen = 0.0;
-  unsigned* bmask = nullptr;
-  // density beyond 7 tiles: the point blocks by the number of tiles that count there
-  std::vector<DensityClass> dclass;
-  int *dblocks = nullptr, *dempty = nullptr;
-  uint4* dtiles = nullptr;
-  int nempty = 0;
+  BlockClasses reach;      // at screen, or at kAmpReach without
+  BlockClasses adj_reach;  // screened handles: at kAmpReach, for the force terms (on their first use)
   // reduced-precision mode
   float* phf = nullptr;  // FP32 amplitudes
   double* ej_part = nullptr;
@@ -2933,7 +2984,6 @@ struct dg_handle {
   double *adj_part = nullptr, *adj_mot = nullptr, *adj_lam = nullptr, *adj_out = nullptr, *adj_dP = nullptr;
   int *ash_start = nullptr, *ash_list = nullptr;
   int* atom_order = nullptr;  // per atom, all atoms by distance
-  unsigned* adj_tmask = nullptr;  // per 64-point block, the function tiles the force terms read
   // state
   bool has_density = false, has_hartree = false, has_xc = false, corrected = false;
   const double* last_P = nullptr;  // device density matrix of the last density evaluation
@@ -2954,13 +3004,15 @@ struct dg_handle {
                       mol_z, mol_fac, mol_qraw, atom_exc, atom_ej, qpart, uG, coef, mono, sh_amin};
     for (double* b : bufs)
       if (b) dfree(b);
-    int* ibufs[] = {sh_atom, sh_L, sh_nprim, sh_off, sh_cgf, blocks, ntask, ash_start, ash_list, atom_order, dblocks, dempty,
+    int* ibufs[] = {sh_atom, sh_L, sh_nprim, sh_off, sh_cgf, blocks, ntask, ash_start, ash_list, atom_order,
+                    reach.block, reach.empty, adj_reach.block, adj_reach.empty,
                     atom_mol, mol_atom0, mol_shell0, mol_nbf, bchunks, mol_chunk0,
                     tb[0].cb, tb[0].groups, tb[0].list, tb[0].slot0, tb[1].cb, tb[1].groups, tb[1].list,
                     tb[1].slot0};
-    if (bmask) dfree(bmask);
-    if (dtiles) dfree(dtiles);
-    if (adj_tmask) dfree(adj_tmask);
+    for (BlockClasses* r : {&reach, &adj_reach}) {
+      dfree(r->tile);
+      dfree(r->mask);
+    }
     for (TileBlocks& t : tb)
       if (t.order) dfree(t.order);
     if (vbase) dfree(vbase);
@@ -3077,7 +3129,7 @@ void launch_density_pl_nt(dg_handle* h, const double* dP) {
   const long nblk = h->npts_pad / 64;
   const unsigned G = (unsigned)std::min<long>(nblk, 1024);
   hipLaunchKernelGGL(k_density_pl<NT>, dim3(G), dim3(256), 0, h->stream, h->phi, h->ldphi, dP, h->nbf, nblk, h->rho,
-                     h->bmask);
+                     h->reach.mask);
 }
 
 int launch_density(dg_handle* h, const double* dP) {
@@ -3095,13 +3147,13 @@ int launch_density(dg_handle* h, const double* dP) {
       }
     });
   return run(h, "density", [&] {
-    for (const DensityClass& k : h->dclass) {
+    for (const BlockClasses::Launch& k : h->reach.launch) {
       const dim3 grid(k.count), block(256);
       switch (k.n) {
 #define DG_N(N)                                                                                              \
   case N:                                                                                                    \
     hipLaunchKernelGGL(k_density_ring<N>, grid, block, 0, h->stream, h->phi, h->ldphi, h->pfrag, h->rho,     \
-                       h->dblocks + k.first, h->dtiles + 2 * k.first, h->ntb);                                      \
+                       h->reach.block + k.first, h->reach.tile + 2 * k.first, h->ntb);                                      \
     break;
         DG_N(4) DG_N(6) DG_N(8) DG_N(9) DG_N(10) DG_N(11) DG_N(12) DG_N(13) DG_N(14) DG_N(15) DG_N(16) DG_N(18)
         DG_N(20) DG_N(22) DG_N(25) DG_N(28) DG_N(32)
@@ -3113,15 +3165,11 @@ int launch_density(dg_handle* h, const double* dP) {
   });
 }
 
-// tmask: the tiles that matter per 64-point block (k_tile_mask), or null for
-// all; only the ring kernel uses it, the others form every tile.
 template <int NT>
-void launch_tmat_nt(hipStream_t st, long npts_pad, const double* phi, int ldphi, const double* frag, double* tmat,
-                    const unsigned* tmask) {
+void launch_tmat_nt(hipStream_t st, long npts_pad, const double* phi, int ldphi, const double* frag, double* tmat) {
   // 8 to 25 tiles: the fragments streamed through a ring, two work-groups per CU
   if constexpr (NT >= 8 && NT <= 25) {
-    hipLaunchKernelGGL(k_tmat_ring<NT>, dim3(nblocks(npts_pad, 64)), dim3(256), 0, st, phi, ldphi, frag, tmat,
-                       tmask);
+    hipLaunchKernelGGL(k_tmat_ring<NT>, dim3(nblocks(npts_pad, 64)), dim3(256), 0, st, phi, ldphi, frag, tmat);
     return;
   }
   // eight waves (two per SIMD) when the rows come in 128s and the amplitude
@@ -3135,14 +3183,13 @@ void launch_tmat_nt(hipStream_t st, long npts_pad, const double* phi, int ldphi,
   hipLaunchKernelGGL((k_tmat<NT, 4>), dim3(nblocks(npts_pad, 64)), dim3(256), 0, st, phi, ldphi, frag, tmat);
 }
 
-// T = Phi P on npts_pad (a multiple of 64) rows, from full P fragments of nt tiles;
-// with tmask, tiles outside a block's mask may be left unformed.
+// T = Phi P on npts_pad (a multiple of 64) rows, from full P fragments of nt tiles.
 void launch_tmat_rows(int nt, hipStream_t st, long npts_pad, const double* phi, int ldphi, const double* frag,
-                      double* tmat, const unsigned* tmask = nullptr) {
+                      double* tmat) {
   switch (nt) {
 #define DG_NT(N)                                                         \
   case N:                                                                \
-    launch_tmat_nt<N>(st, npts_pad, phi, ldphi, frag, tmat, tmask); \
+    launch_tmat_nt<N>(st, npts_pad, phi, ldphi, frag, tmat); \
     break;
     DG_NT(1) DG_NT(2) DG_NT(3) DG_NT(4) DG_NT(5) DG_NT(6) DG_NT(7) DG_NT(8) DG_NT(9) DG_NT(10) DG_NT(11)
     DG_NT(12) DG_NT(13) DG_NT(14) DG_NT(15) DG_NT(16) DG_NT(17) DG_NT(18) DG_NT(19) DG_NT(20) DG_NT(21)
@@ -3154,31 +3201,47 @@ void launch_tmat_rows(int nt, hipStream_t st, long npts_pad, const double* phi, 
   }
 }
 
-// T = Phi P for the force terms (P = the last density matrix, full fragments).
-// The function tiles within reach of each 64-point block (k_tile_mask), on
-// first use; none beyond 32 tiles (the masks are 32-bit).
-int ensure_tile_mask(dg_handle* h) {
-  if (h->adj_tmask || h->ntb > 32) return DG_OK;
-  const long nblk = h->npts_pad / 64;
-  DG_TRY(dalloc(&h->adj_tmask, nblk));
-  return run(h, "adj_tile_mask", [&] {
-    hipLaunchKernelGGL(k_tile_mask, dim3(nblk), dim3(256), 0, h->stream, h->atoms, h->nshell, h->sh_atom, h->sh_L,
-                       h->sh_cgf, h->sh_amin, h->npts, h->px, h->py, h->pz, h->adj_tmask);
-  });
+int block_reach(dg_handle* h, double limit, std::vector<unsigned>& mk, BlockClasses& r);
+
+// The function tiles the force terms take per point block (mask null: all).
+// Screened handles take them at the reach of unscreened ones: their forces leave
+// out no more than those.
+int force_reach(dg_handle* h, const BlockClasses** r) {
+  const bool own = h->screen > 0.0 && h->ntb > 7;
+  *r = own ? &h->adj_reach : &h->reach;
+  if (!own || h->adj_reach.mask) return DG_OK;
+  std::vector<unsigned> mk(h->npts_pad / 64);
+  return block_reach(h, kAmpReach, mk, h->adj_reach);
 }
 
-// T = Phi P for the last density matrix.  masked (the force terms): only the
-// tiles k_force_basis reads are formed (k_tile_mask).
-int launch_tmat(dg_handle* h, bool masked = false) {
-  if (masked) DG_TRY(ensure_tile_mask(h));
+// T = Phi P for the last density matrix (full fragments); with r, only the tiles in
+// its blocks' masks are formed.
+int launch_tmat(dg_handle* h, const BlockClasses* r = nullptr) {
   DG_TRY(run(h, "adj_pfrag", [&] {
     const long nf = 256L * h->ntb * h->ntb;
     hipLaunchKernelGGL(k_pfrag_full, dim3(nblocks(nf, 256)), dim3(256), 0, h->stream, h->last_P, h->nbf, h->ntb,
                        h->adj_frag);
   }));
-  const unsigned* tmask = masked ? h->adj_tmask : nullptr;
   return run(h, "adj_tmat", [&] {
-    launch_tmat_rows(h->ntb, h->stream, h->npts_pad, h->phi, h->ldphi, h->adj_frag, h->adj_T, tmask);
+    if (!r) {
+      launch_tmat_rows(h->ntb, h->stream, h->npts_pad, h->phi, h->ldphi, h->adj_frag, h->adj_T);
+      return;
+    }
+    for (const BlockClasses::Launch& k : r->launch) {
+      const dim3 grid(k.count), block(256);
+      switch (k.n) {
+#define DG_N(N)                                                                                              \
+  case N:                                                                                                    \
+    hipLaunchKernelGGL(k_tmat_tiles<N>, grid, block, 0, h->stream, h->phi, h->ldphi, h->adj_frag, h->adj_T,  \
+                       r->block + k.first, r->tile + 2 * k.first, h->ntb);                                   \
+    break;
+        DG_N(4) DG_N(6) DG_N(8) DG_N(9) DG_N(10) DG_N(11) DG_N(12) DG_N(13) DG_N(14) DG_N(15) DG_N(16) DG_N(18)
+        DG_N(20) DG_N(22) DG_N(25) DG_N(28) DG_N(32)
+#undef DG_N
+        default:
+          break;
+      }
+    }
   });
 }
 
@@ -3187,8 +3250,8 @@ int stage_density(dg_handle* h, const double* dP) {
   if (h->ntb > 7)  // the persistent kernel forms its fragments itself
     DG_TRY(run(h, "pfrag", [&] {
       const unsigned nfb = nblocks(nfrag, 256);
-      hipLaunchKernelGGL(k_pfrag, dim3(nfb + nblocks(h->nempty, 4)), dim3(256), 0, h->stream, dP, h->nbf, h->ntb,
-                         h->pfrag, nfb, h->dempty, h->nempty, h->rho);
+      hipLaunchKernelGGL(k_pfrag, dim3(nfb + nblocks(h->reach.nempty, 4)), dim3(256), 0, h->stream, dP, h->nbf, h->ntb,
+                         h->pfrag, nfb, h->reach.empty, h->reach.nempty, h->rho);
     }));
   DG_TRY(launch_density(h, dP));
   h->last_P = dP;
@@ -3471,8 +3534,7 @@ int copy_out(dg_handle* h, double* dst, const double* src, size_t n) {
 // at least kDensityClassMin blocks come to; fewer join the next larger one.
 constexpr int kDensityTiles[] = {4, 6, 8, 9, 10, 11, 12, 13, 14, 15, 16, 18, 20, 22, 25, 28, 32};
 constexpr long kDensityClassMin = 512;
-int density_classes(dg_handle* h, const std::vector<unsigned>& mk) {
-  const int nt = h->ntb;
+int block_classes(const std::vector<unsigned>& mk, int nt, BlockClasses& r) {
   std::vector<std::vector<int>> by(nt + 1);
   for (size_t b = 0; b < mk.size(); ++b) by[__builtin_popcount(mk[b])].push_back((int)b);
   const std::vector<int> empty = by[0];
@@ -3484,26 +3546,39 @@ int density_classes(dg_handle* h, const std::vector<unsigned>& mk) {
   for (int n : kDensityTiles) {
     for (; done < std::min(n, nt); ++done) wait.insert(wait.end(), by[done + 1].begin(), by[done + 1].end());
     if (wait.empty() || (n < nt && (long)wait.size() < kDensityClassMin)) continue;
-    h->dclass.push_back({n, (long)blocks.size(), (long)wait.size()});
+    r.launch.push_back({n, (long)blocks.size(), (long)wait.size()});
     for (int b : wait) {
       unsigned char id[32];
       std::memset(id, 255, 32);
-      for (int t = 0, r = 0; t < nt; ++t)
-        if ((mk[b] >> t) & 1u) id[r++] = (unsigned char)t;
+      for (int t = 0, at = 0; t < nt; ++t)
+        if ((mk[b] >> t) & 1u) id[at++] = (unsigned char)t;
       tiles.insert(tiles.end(), id, id + 32);
       blocks.push_back(b);
     }
     wait.clear();
   }
-  std::reverse(h->dclass.begin(), h->dclass.end());
-  h->nempty = (int)empty.size();
-  DG_TRY(dalloc(&h->dblocks, blocks.size()));
-  DG_TRY(dalloc(&h->dtiles, tiles.size() / 16));
-  DG_TRY(dalloc(&h->dempty, empty.size()));
-  HIP_TRY(hipMemcpy(h->dblocks, blocks.data(), blocks.size() * 4, hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(h->dtiles, tiles.data(), tiles.size(), hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(h->dempty, empty.data(), empty.size() * 4, hipMemcpyHostToDevice));
+  std::reverse(r.launch.begin(), r.launch.end());
+  r.nempty = (int)empty.size();
+  DG_TRY(dalloc(&r.block, blocks.size()));
+  DG_TRY(dalloc(&r.tile, tiles.size() / 16));
+  DG_TRY(dalloc(&r.empty, empty.size()));
+  HIP_TRY(hipMemcpy(r.block, blocks.data(), blocks.size() * 4, hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(r.tile, tiles.data(), tiles.size(), hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(r.empty, empty.data(), empty.size() * 4, hipMemcpyHostToDevice));
   return DG_OK;
+}
+
+// The tiles with an amplitude beyond limit, per 64-point block, and, past 7 tiles,
+// the blocks by their number.
+int block_reach(dg_handle* h, double limit, std::vector<unsigned>& mk, BlockClasses& r) {
+  const long nblk = h->npts_pad / 64;
+  DG_TRY(dalloc(&r.mask, nblk));
+  DG_TRY(run(h, "block_mask", [&] {
+    hipLaunchKernelGGL(k_block_mask, dim3(nblk), dim3(64), 0, h->stream, h->phi, h->ldphi, h->ntb, limit, r.mask);
+  }));
+  HIP_TRY(hipMemcpyAsync(mk.data(), r.mask, nblk * 4, hipMemcpyDeviceToHost, h->stream));
+  DG_TRY(sync(h));
+  return h->ntb > 7 ? block_classes(mk, h->ntb, r) : DG_OK;
 }
 
 // The tiles that count per 64-point block (k_block_mask) and, for the 2-D
@@ -3521,16 +3596,9 @@ int tile_reach(dg_handle* h, const std::vector<int> (&cbs)[2]) {
   const long nblk = h->npts_pad / 64;
   const bool two_d = h->ntb > 5;
   if (h->screen == 0.0 && !two_d) return DG_OK;
-  DG_TRY(dalloc(&h->bmask, nblk));
-  DG_TRY(run(h, "block_mask", [&] {
-    hipLaunchKernelGGL(k_block_mask, dim3(nblk), dim3(64), 0, h->stream, h->phi, h->ldphi, h->ntb,
-                       h->screen > 0.0 ? h->screen : kAmpReach, h->bmask);
-  }));
-  if (!two_d) return DG_OK;
   std::vector<unsigned> mk(nblk);
-  HIP_TRY(hipMemcpyAsync(mk.data(), h->bmask, nblk * 4, hipMemcpyDeviceToHost, h->stream));
-  DG_TRY(sync(h));
-  if (h->ntb > 7) DG_TRY(density_classes(h, mk));
+  DG_TRY(block_reach(h, h->screen > 0.0 ? h->screen : kAmpReach, mk, h->reach));
+  if (!two_d) return DG_OK;
   size_t ncpart = 0;
   for (int q = 0; q < 2; ++q) {
     TileBlocks& t = h->tb[q];
@@ -4420,11 +4488,14 @@ int dg_xc_adjoint(dg_handle* h, int hold_c, double* dEdP, double* grad) {
     DG_TRY(copy_out(h, dEdP, h->adj_dP, (size_t)h->nbf * h->nbf));
   }
   if (grad) {
-    DG_TRY(launch_tmat(h, true));
+    const BlockClasses* r = nullptr;
+    if (h->ntb > 7) DG_TRY(force_reach(h, &r));
+    DG_TRY(launch_tmat(h, r));
     DG_TRY(run(h, "adj_force_basis", [&] {
       hipLaunchKernelGGL(k_force_basis, dim3(nblk), dim3(64), 0, h->stream, h->atoms, na, h->ash_start, h->ash_list,
                          h->sh_L, h->sh_nprim, h->sh_off, h->sh_cgf, h->sh_amin, h->pr_alpha, h->pr_cn0, h->pr_cn1,
-                         h->npts, h->px, h->py, h->pz, h->ldphi, h->adj_T, h->adj_ub, nblk, h->adj_part, h->adj_mot);
+                         h->npts, h->px, h->py, h->pz, h->ldphi, h->adj_T, h->adj_ub, nblk, r ? r->mask : nullptr,
+                         h->adj_part, h->adj_mot);
     }));
     HIP_TRY(hipMemsetAsync(h->adj_out + 6 * na, 0, sizeof(double), h->stream));
     DG_TRY(run(h, "adj_force_becke", [&] {
