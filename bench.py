@@ -20,6 +20,7 @@ Usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload NAME]
 """
 import argparse
 import json
+import math
 import os
 import sys
 import time
@@ -53,20 +54,50 @@ def traffic_key(label, names):
 CPU_SAMPLE_MAX_POINTS = 300000
 
 
+def tile_pair_share(mol, xyz):
+    """Share of the pairs of 16-function tiles that count on the 64-point blocks of
+    the points, where the library's default reach (2^-106) leaves tiles out: bases of
+    more than 80 functions.  A shell counts where its most diffuse primitive,
+    exp(-alpha r^2), is above the reach."""
+    import numpy as np
+    import torch
+
+    nt = (mol.nbf() + 15) // 16
+    if nt <= 5:
+        return 1.0
+    s = mol.shells()
+    limit = 106 * math.log(2.0)
+    R = torch.as_tensor(mol.xyz, device="cuda")
+    x = torch.as_tensor(xyz, device="cuda")
+    x = x[:len(x) // 64 * 64]
+    live = torch.zeros(len(x) // 64, nt, dtype=torch.bool, device="cuda")
+    i = 0
+    for k, L in enumerate(s["L"]):
+        a = float(np.min(s["alpha"][s["offset"][k]:s["offset"][k] + s["nprim"][k]]))
+        near = ((x - R[int(s["atom"][k])]).square().sum(1) * a <= limit).view(-1, 64).any(1)
+        n = (int(L) + 1) * (int(L) + 2) // 2
+        for t in range(i // 16, (i + n - 1) // 16 + 1):
+            live[:, t] |= near
+        i += n
+    n = live.sum(1).double()
+    return float((n * (n + 1)).mean()) / (nt * (nt + 1))
+
+
 def kernel_work(name, mol_info):
     """(algorithmic flops of one launch, the unit that bounds it) of a build kernel,
     or (None, None) for kernels without a flop model.
 
     One convention throughout: the symmetric products count only the pairs
-    i <= j (the work the result needs), 2 flops per multiply-add; the Hartree
-    cross term counts 10 flops per (point, atom, lm) spline + harmonic term."""
+    i <= j (the work the result needs) of the function tiles that count at a point,
+    2 flops per multiply-add; the Hartree cross term counts 10 flops per (point,
+    atom, lm) spline + harmonic term."""
     npts, nbf, nat, nlm = mol_info["npts"], mol_info["nbf"], mol_info["natoms"], mol_info["nlm"]
     if name == "hartree_cross":  # FP64 vector ALU: the kernel issues no MFMA
         return HARTREE_FLOPS_PER_TERM * npts * (nat - 1) * nlm / mol_info["cross_launches"], "valu_fp64"
     if name == "contract":  # J and XC, FP64 (or FP32 in mixed mode) MFMA
-        return 2 * 2.0 * npts * nbf * (nbf + 1) / 2, "mfma"
+        return mol_info.get("pair_share", 1.0) * 2 * 2.0 * npts * nbf * (nbf + 1) / 2, "mfma"
     if name == "density":
-        return 2.0 * npts * nbf * (nbf + 1) / 2 + 2.0 * npts * nbf, "mfma"
+        return mol_info.get("pair_share", 1.0) * (2.0 * npts * nbf * (nbf + 1) / 2 + 2.0 * npts * nbf), "mfma"
     return None, None
 
 
@@ -330,7 +361,9 @@ def main():
         total = sum(ms for ms, _ in prof.values())
         out["kernels_ms_per_step"] = {k: ms / nprof for k, (ms, _) in sorted(prof.items())}
         info = {"npts": npts, "nbf": nbf, "natoms": mol.natoms, "nlm": (lmax + 1) ** 2,
+                "pair_share": tile_pair_share(mol, grid.get_positions()),
                 "cross_launches": max(1, prof.get("hartree_cross", (0, nprof))[1] // nprof)}
+        out["tile_pair_share"] = info["pair_share"]
         dom = max(prof.items(), key=lambda kv: kv[1][0])[0]
         ms, cnt = prof[dom]
         avg_s = ms / cnt / 1e3
