@@ -255,9 +255,9 @@ __global__ __launch_bounds__(64) void k_block_mask(const double* __restrict__ ph
   const double* row = phi + p * ldphi;
   unsigned bits = 0u;
   for (int T = 0; T < ntb; ++T) {
-    double m = 0.0;
-    for (int i = 0; i < 16; ++i) m = fmax(m, fabs(row[16 * T + i]));
-    if (m > screen) bits |= 1u << T;
+    bool on = false;  // NaN counts: it has to show in the results
+    for (int i = 0; i < 16; ++i) on |= !(fabs(row[16 * T + i]) <= screen);
+    if (on) bits |= 1u << T;
   }
   for (int o = 32; o > 0; o >>= 1) bits |= (unsigned)__shfl_xor((int)bits, o);
   if (threadIdx.x == 0) mask[blockIdx.x] = bits;
