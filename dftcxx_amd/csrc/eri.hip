@@ -447,7 +447,7 @@ __global__ __launch_bounds__(256) void k_eri_partial(const double* __restrict__ 
   const int ncol = (npair + 63) / 64, cb = (int)blockIdx.x - npair;
   const long IJ0 = 64L * (cb % ncol), IJ = IJ0 + (tid & 63), ch = cb / ncol;
   const long k0 = ch * chunk, k1 = std::min<long>(k0 + chunk, npair);
-  if (k1 <= IJ0 + 1) return;  // no row below the diagonal: k_eri_unpack skips the chunk too
+  if (k1 <= IJ0) return;  // below the chunks k_eri_unpack takes for these pairs, (IJ + 1) / chunk and up
   double s = 0.0;
   if (IJ < npair) {
     long KL = k0 + (tid >> 6);
