@@ -2878,6 +2878,13 @@ int dalloc(T** p, size_t n) {
   return DG_OK;
 }
 
+// As dalloc, but leaves a buffer that is there: set-up on first use can be taken up
+// again after an allocation failed in the middle of it.
+template <typename T>
+int dalloc_once(T** p, size_t n) {
+  return *p ? DG_OK : dalloc(p, n);
+}
+
 long round_up(long x, long m) { return (x + m - 1) / m * m; }
 
 }  // namespace
@@ -2915,6 +2922,11 @@ struct BlockClasses {
   uint4* tile = nullptr;
   unsigned* mask = nullptr;
   int nempty = 0;
+
+  void release() {
+    for (void* p : {(void*)block, (void*)empty, (void*)tile, (void*)mask}) dfree(p);
+    *this = BlockClasses();
+  }
 };
 
 struct dg_handle {
@@ -2984,6 +2996,7 @@ struct dg_handle {
   double *adj_part = nullptr, *adj_mot = nullptr, *adj_lam = nullptr, *adj_out = nullptr, *adj_dP = nullptr;
   int *ash_start = nullptr, *ash_list = nullptr;
   int* atom_order = nullptr;  // per atom, all atoms by distance
+  bool adj_lists = false;     // ash_start, ash_list and atom_order are filled
   // state
   bool has_density = false, has_hartree = false, has_xc = false, corrected = false;
   const double* last_P = nullptr;  // device density matrix of the last density evaluation
@@ -3005,14 +3018,11 @@ struct dg_handle {
     for (double* b : bufs)
       if (b) dfree(b);
     int* ibufs[] = {sh_atom, sh_L, sh_nprim, sh_off, sh_cgf, blocks, ntask, ash_start, ash_list, atom_order,
-                    reach.block, reach.empty, adj_reach.block, adj_reach.empty,
                     atom_mol, mol_atom0, mol_shell0, mol_nbf, bchunks, mol_chunk0,
                     tb[0].cb, tb[0].groups, tb[0].list, tb[0].slot0, tb[1].cb, tb[1].groups, tb[1].list,
                     tb[1].slot0};
-    for (BlockClasses* r : {&reach, &adj_reach}) {
-      dfree(r->tile);
-      dfree(r->mask);
-    }
+    reach.release();
+    adj_reach.release();
     for (TileBlocks& t : tb)
       if (t.order) dfree(t.order);
     if (vbase) dfree(vbase);
@@ -3211,7 +3221,15 @@ int force_reach(dg_handle* h, const BlockClasses** r) {
   *r = own ? &h->adj_reach : &h->reach;
   if (!own || h->adj_reach.mask) return DG_OK;
   std::vector<unsigned> mk(h->npts_pad / 64);
-  return block_reach(h, kAmpReach, mk, h->adj_reach);
+  BlockClasses made;  // the handle's only once it is whole
+  const int rc = block_reach(h, kAmpReach, mk, made);
+  if (rc == DG_OK) {
+    h->adj_reach = made;
+  } else {
+    (void)hipStreamSynchronize(h->stream);
+    made.release();
+  }
+  return rc;
 }
 
 // T = Phi P for the last density matrix (full fragments); with r, only the tiles in
@@ -3670,9 +3688,8 @@ int tile_reach(dg_handle* h, const std::vector<int> (&cbs)[2]) {
 
 // T = Phi P buffers (the adjoint's force terms and the density gradients), on first use.
 int ensure_tmat_bufs(dg_handle* h) {
-  if (!h->adj_T) DG_TRY(dalloc(&h->adj_T, (size_t)h->npts_pad * h->ldphi));
-  if (!h->adj_frag) DG_TRY(dalloc(&h->adj_frag, (size_t)256 * h->ntb * h->ntb));
-  return DG_OK;
+  DG_TRY(dalloc_once(&h->adj_T, (size_t)h->npts_pad * h->ldphi));
+  return dalloc_once(&h->adj_frag, (size_t)256 * h->ntb * h->ntb);
 }
 
 // ---------------------------------------------------------------------------
@@ -4436,16 +4453,14 @@ int dg_xc_adjoint(dg_handle* h, int hold_c, double* dEdP, double* grad) {
   const int na = h->natoms;
   if (grad && na > 65535)
     return fail(DG_ERR_UNSUPPORTED, "dg_xc_adjoint: forces for at most 65535 atoms");
-  if (!h->adj_ub) {
-    for (double** b : {&h->adj_ub, &h->adj_ab, &h->adj_udp}) DG_TRY(dalloc(b, np));
-    DG_TRY(dalloc(&h->adj_lam, np / 256 + 1));
-    DG_TRY(dalloc(&h->adj_dP, (size_t)h->nbf * h->nbf));
-    DG_TRY(dalloc(&h->adj_out, (size_t)6 * na + 1));
-  }
+  for (double** b : {&h->adj_ub, &h->adj_ab, &h->adj_udp}) DG_TRY(dalloc_once(b, np));
+  DG_TRY(dalloc_once(&h->adj_lam, np / 256 + 1));
+  DG_TRY(dalloc_once(&h->adj_dP, (size_t)h->nbf * h->nbf));
+  DG_TRY(dalloc_once(&h->adj_out, (size_t)6 * na + 1));
   if (grad) DG_TRY(ensure_tmat_bufs(h));
-  if (grad && !h->adj_part) {
-    DG_TRY(dalloc(&h->adj_part, (size_t)3 * na * nblk));
-    DG_TRY(dalloc(&h->adj_mot, (size_t)3 * h->npts));
+  if (grad && !h->adj_lists) {
+    DG_TRY(dalloc_once(&h->adj_part, (size_t)3 * na * nblk));
+    DG_TRY(dalloc_once(&h->adj_mot, (size_t)3 * h->npts));
     // shells grouped by centre atom
     std::vector<int> at(h->nshell), start(na + 1, 0), list;
     HIP_TRY(hipMemcpyAsync(at.data(), h->sh_atom, h->nshell * 4, hipMemcpyDeviceToHost, h->stream));
@@ -4456,16 +4471,17 @@ int dg_xc_adjoint(dg_handle* h, int hold_c, double* dEdP, double* grad) {
         if (at[s] == a) list.push_back(s);
     }
     start[na] = (int)list.size();
-    DG_TRY(dalloc(&h->atom_order, (size_t)na * na));
+    DG_TRY(dalloc_once(&h->atom_order, (size_t)na * na));
     DG_TRY(run(h, "adj_atom_order", [&] {
       hipLaunchKernelGGL(k_atom_order, dim3(nblocks((long)na * na, 256)), dim3(256), 0, h->stream, h->atoms, na,
                          h->atom_order);
     }));
-    DG_TRY(dalloc(&h->ash_start, na + 1));
-    DG_TRY(dalloc(&h->ash_list, std::max<size_t>(list.size(), 1)));
+    DG_TRY(dalloc_once(&h->ash_start, na + 1));
+    DG_TRY(dalloc_once(&h->ash_list, std::max<size_t>(list.size(), 1)));
     HIP_TRY(hipMemcpyAsync(h->ash_start, start.data(), (na + 1) * 4, hipMemcpyHostToDevice, h->stream));
     HIP_TRY(hipMemcpyAsync(h->ash_list, list.data(), list.size() * 4, hipMemcpyHostToDevice, h->stream));
     DG_TRY(sync(h));
+    h->adj_lists = true;
   }
   // Lambda = sum w v rho (uxc = w v), then the per-point factors
   const long nparts = np / 256;
