@@ -18,7 +18,6 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
-#include <list>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -26,6 +25,7 @@
 #include <vector>
 
 #include "../../include/dftgrid.h"
+#include "device_pool.h"
 #include "grid_tables.h"
 #include "unroll.h"
 
@@ -2786,80 +2786,24 @@ __global__ void k_mfma_probe(double* out) {
 // program that makes a grid per geometry allocates the same sizes again and again,
 // and hipMalloc, hipFree and the mapping behind them take longer than the set-up's
 // kernels (C10H22 / 75 x 302: closing a handle 5.2 ms, the set-up's kernels 2).
-// At most kPoolMax per process, the longest kept leaving first, and all of it
-// before an allocation fails.  A block comes here only when the work that used it
-// is over (its owner's stream has been waited for), so any stream of the device
-// may have it next; what it holds then is not defined, as with hipMalloc.
-class DevicePool {
- public:
-  hipError_t take(void** p, size_t bytes) {
-    bytes = std::max<size_t>((bytes + 511) / 512 * 512, 512);
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    {
-      std::lock_guard<std::mutex> lock(m_);
-      auto best = kept_.end();
-      for (auto it = kept_.begin(); it != kept_.end(); ++it)
-        if (it->dev == dev && it->bytes >= bytes && it->bytes <= bytes + bytes / 8 &&
-            (best == kept_.end() || it->bytes < best->bytes))
-          best = it;
-      if (best != kept_.end()) {
-        *p = best->p;
-        used_[best->p] = *best;
-        held_ -= best->bytes;
-        kept_.erase(best);
-        return hipSuccess;
-      }
-    }
-    e = hipMalloc(p, bytes);
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      std::lock_guard<std::mutex> lock(m_);
-      while (!kept_.empty()) drop_oldest();
-      e = hipMalloc(p, bytes);
-    }
-    if (e != hipSuccess) return e;
-    std::lock_guard<std::mutex> lock(m_);
-    used_[*p] = Block{*p, bytes, dev};
-    return hipSuccess;
+// At most 2 GiB per process, under 1 % of the device's memory, and all of it goes back
+// before an allocation of the library fails.  A block comes here only when the work
+// that used it is over, so any stream of the device may have it next; what it holds
+// then is not defined, as with hipMalloc.
+struct HipMemory {
+  static constexpr int kNoMemory = hipErrorOutOfMemory;
+  static int device(int* d) { return hipGetDevice(d); }
+  static int alloc(void** p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();  // reported here, not by the next launch's check
+    return e;
   }
-  void give(void* p) {
-    if (!p) return;
-    std::lock_guard<std::mutex> lock(m_);
-    auto it = used_.find(p);
-    if (it == used_.end()) return;
-    const Block b = it->second;
-    used_.erase(it);
-    if (b.bytes > kPoolMax) {
-      (void)hipFree(p);
-      return;
-    }
-    while (held_ + b.bytes > kPoolMax) drop_oldest();
-    kept_.push_back(b);
-    held_ += b.bytes;
-  }
-
- private:
-  struct Block {
-    void* p;
-    size_t bytes;
-    int dev;
-  };
-  void drop_oldest() {
-    held_ -= kept_.front().bytes;
-    (void)hipFree(kept_.front().p);
-    kept_.pop_front();
-  }
-  static constexpr size_t kPoolMax = (size_t)2 << 30;  // under 1 % of the device's memory
-  std::mutex m_;
-  std::list<Block> kept_;  // oldest first
-  std::map<void*, Block> used_;
-  size_t held_ = 0;
+  static void release(void* p) { (void)hipFree(p); }
 };
 
-DevicePool& pool() {
-  static DevicePool* p = new DevicePool;  // not destroyed: handles may outlive static objects
+dg::DevicePool<HipMemory>& pool() {
+  // not destroyed: handles may outlive static objects
+  static auto* p = new dg::DevicePool<HipMemory>((size_t)2 << 30);
   return *p;
 }
 
@@ -2869,12 +2813,10 @@ void dfree(void* p) { pool().give(p); }
 template <typename T>
 int dalloc(T** p, size_t n) {
   if (n == 0) n = 1;
-  hipError_t e = pool().take((void**)p, n * sizeof(T));
-  if (e != hipSuccess) {
-    *p = nullptr;
+  const hipError_t e = (hipError_t)pool().take((void**)p, n * sizeof(T));
+  if (e != hipSuccess)
     return fail(DG_ERR_ALLOC, std::string("hipMalloc of ") + std::to_string(n * sizeof(T)) +
                                   " bytes failed: " + hipGetErrorString(e));
-  }
   return DG_OK;
 }
 
