@@ -2807,6 +2807,12 @@ dg::DevicePool<HipMemory>& pool() {
   return *p;
 }
 
+}  // namespace
+
+int dg::device_malloc(void** p, size_t bytes) { return pool().raw(p, bytes); }
+
+namespace {
+
 // Returns a buffer no pending work uses.
 void dfree(void* p) { pool().give(p); }
 
@@ -4188,6 +4194,12 @@ int dg_destroy(dg_handle* h) {
   if (!h) return DG_OK;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   delete h;
+  return DG_OK;
+}
+
+int dg_release_memory(void) {
+  g_last_error.clear();
+  pool().release_kept();
   return DG_OK;
 }
 

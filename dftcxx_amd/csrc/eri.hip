@@ -572,7 +572,7 @@ int dg_eri_create(const dg_molecule* mol, const dg_basis* basis, dg_eri** out) {
   e->nints = (long)e->npair * (e->npair + 1) / 2;
   if (e->nints > (1L << 36)) return fail(DG_ERR_UNSUPPORTED, "dg_eri_create: more than 2^36 integrals");
   ERI_HIP(hipStreamCreate(&e->stream));
-  ERI_HIP(hipMalloc((void**)&e->ints, sizeof(double) * std::max<long>(e->nints, 1)));
+  ERI_HIP((hipError_t)dg::device_malloc((void**)&e->ints, sizeof(double) * std::max<long>(e->nints, 1)));
   std::vector<int> pij(2 * (size_t)e->npair);
   for (int i = 0, IJ = 0; i < n; ++i)
     for (int j = 0; j <= i; ++j, ++IJ) {
@@ -671,7 +671,7 @@ int dg_eri_create(const dg_molecule* mol, const dg_basis* basis, dg_eri** out) {
   put(o_off, off.data(), off.size() * 4);
   put(o_pl, pl.data(), pl.size() * 4);
   put(o_pd, pd.data(), pd.size() * 4);
-  ERI_HIP(hipMalloc((void**)&e->work, c.size));
+  ERI_HIP((hipError_t)dg::device_malloc((void**)&e->work, c.size));
   char* w = e->work;
   double* tab = (double*)(w + o_tab);
   e->pij = (int*)(w + o_pij);

@@ -2,6 +2,7 @@
 #ifndef DFTGRID_GRID_TABLES_H
 #define DFTGRID_GRID_TABLES_H
 
+#include <cstddef>
 #include <string>
 #include <vector>
 
@@ -54,6 +55,11 @@ SplineSystem spline_system(const std::vector<double>& x);
 // x of the spline through the values y (src/cspline.cpp:66-127 applied to the
 // unit vectors; the slope system is linear in y).
 std::vector<double> spline_slope_matrix(const std::vector<double>& x);
+
+// hipMalloc for memory that its owner frees with hipFree: the memory of closed handles
+// kept by the library goes back to the device first if there is no room.  Returns the
+// hipError_t.
+int device_malloc(void** p, size_t bytes);
 
 }  // namespace dg
 

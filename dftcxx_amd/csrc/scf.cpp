@@ -734,7 +734,7 @@ class DFT : public HostSCF {
       device_iteration(false);
       return;
     }
-    if (hipMalloc((void**)&dP_, sizeof(double) * (3 * (size_t)n_ * n_ + 4)) != hipSuccess)
+    if (dg::device_malloc((void**)&dP_, sizeof(double) * (3 * (size_t)n_ * n_ + 4)) != hipSuccess)
       throw std::runtime_error("hipMalloc failed");
     // pinned staging for P, J, XC and the scalars (page-locked copies each iteration)
     if (hipHostMalloc((void**)&hbuf_, sizeof(double) * (3 * (size_t)n_ * n_ + 4), hipHostMallocDefault) !=

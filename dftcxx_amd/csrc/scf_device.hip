@@ -20,6 +20,7 @@
 #include <stdexcept>
 #include <string>
 
+#include "grid_tables.h"
 #include "scf_device.h"
 
 namespace {
@@ -438,8 +439,8 @@ DeviceStep::DeviceStep(int n, int nocc, hipStream_t stream) : n_(n), nocc_(nocc)
   // H, X, F (also P'), F', Pn, P2 (also X P'), P, J, XC, scalars(4), energy(5 of 8),
   // energy partial sums (2 kEnergyParts), Gershgorin bounds (2 n)
   const size_t total = 9 * nn + 12 + 2 * kEnergyParts + 2 * (size_t)n;
-  check(hipMalloc((void**)&buf_, sizeof(double) * total), "hipMalloc of the SCF buffers");
-  check(hipMalloc((void**)&ctl_, sizeof(Sp2Ctl)), "hipMalloc of the SCF control block");
+  check((hipError_t)dg::device_malloc((void**)&buf_, sizeof(double) * total), "hipMalloc of the SCF buffers");
+  check((hipError_t)dg::device_malloc((void**)&ctl_, sizeof(Sp2Ctl)), "hipMalloc of the SCF control block");
   check(hipHostMalloc((void**)&host_, sizeof(double) * 8 + sizeof(Sp2Ctl), hipHostMallocDefault),
         "hipHostMalloc of the SCF staging");
   H_ = buf_;
@@ -569,8 +570,10 @@ BatchStep::BatchStep(int nmol, const int* nbf, const long* off, const int* nocc,
     if (nbf[m] > kBatchN) throw std::runtime_error("batched device step: more than 32 functions in a molecule");
   const size_t np = (size_t)packed_;
   // H, X, P, J, XC, scalars (4/mol), energies (5/mol), enuc
-  check(hipMalloc((void**)&buf_, sizeof(double) * (5 * np + 10 * (size_t)nmol)), "hipMalloc of the batch SCF");
-  check(hipMalloc((void**)&ibuf_, sizeof(long) * (nmol + 1) + sizeof(int) * 3 * (size_t)nmol + nmol),
+  check((hipError_t)dg::device_malloc((void**)&buf_, sizeof(double) * (5 * np + 10 * (size_t)nmol)),
+        "hipMalloc of the batch SCF");
+  check((hipError_t)dg::device_malloc((void**)&ibuf_,
+                                      sizeof(long) * (nmol + 1) + sizeof(int) * 3 * (size_t)nmol + nmol),
         "hipMalloc of the batch SCF");
   check(hipHostMalloc((void**)&host_, sizeof(double) * 5 * (size_t)nmol + sizeof(int) * (size_t)nmol,
                       hipHostMallocDefault),

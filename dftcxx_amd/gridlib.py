@@ -37,7 +37,7 @@ EXPORTS = (
     "dg_input_basis", "dg_input_grid", "dg_input_value", "dg_get_amplitude_gradients",
     "dg_get_density_gradients", "dg_density_at_points", "dg_density_at_points_noalloc", "dg_build_fock_device",
     "dg_build_xc_device", "dg_eri_create", "dg_eri_destroy", "dg_eri_count", "dg_eri_get", "dg_eri_coulomb_device",
-    "dg_eri_coulomb",
+    "dg_eri_coulomb", "dg_release_memory",
 )
 
 
@@ -512,6 +512,12 @@ class Batch:
 
     def profile_read(self):
         return _profile_read(self.h)
+
+
+def release_memory():
+    """Gives the device memory kept from closed grids (at most 2 GiB) back to the device,
+    for other allocators of the process."""
+    _check(lib().dg_release_memory())
 
 
 def one_electron(mol):
