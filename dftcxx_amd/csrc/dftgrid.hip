@@ -2816,6 +2816,13 @@ namespace {
 // Returns a buffer no pending work uses.
 void dfree(void* p) { pool().give(p); }
 
+// Returns a call's buffer after its work on st ended with status rc: a failed call has
+// not waited for what it had launched.
+void dfree_call(void* p, int rc, hipStream_t st) {
+  if (rc != 0) (void)hipStreamSynchronize(st);
+  dfree(p);
+}
+
 template <typename T>
 int dalloc(T** p, size_t n) {
   if (n == 0) n = 1;
@@ -2955,8 +2962,15 @@ struct dg_handle {
   std::map<std::string, ProfStat> stats;
 
   ~dg_handle() {
-    // the buffers go to the next owner: nothing of this handle may still run
-    if (stream && hipStreamSynchronize(stream) != hipSuccess) (void)hipDeviceSynchronize();
+    // The buffers go to the next owner, so nothing that uses them may still run, on any
+    // stream: a graph captured from a build may be replaying on another than the
+    // handle's (hipFree, where they went before there was a pool, waits for the device).
+    if (stream) {
+      int cur = device;
+      const bool other = hipGetDevice(&cur) == hipSuccess && cur != device && hipSetDevice(device) == hipSuccess;
+      if (hipDeviceSynchronize() != hipSuccess) (void)hipStreamSynchronize(stream);
+      if (other) (void)hipSetDevice(cur);
+    }
     double* bufs[] = {atoms, invR,  rad,   wrad,   leb,   px,     py,    pz,   w,     wb,
                       phi,   pr_alpha, pr_cn0, pr_cn1, P, pfrag, rho,  uxc,   exd,   uJ,
                       V,     vcell, vpart, q,      qc,    exc_part, scalars, ylm, minvT, shc,
@@ -4192,7 +4206,6 @@ int dg_create(const dg_molecule* mol, const dg_basis* basis, const dg_grid_param
 
 int dg_destroy(dg_handle* h) {
   if (!h) return DG_OK;
-  if (h->stream) (void)hipStreamSynchronize(h->stream);
   delete h;
   return DG_OK;
 }
@@ -4508,7 +4521,7 @@ int dg_get_amplitude_gradients(dg_handle* h, double* dphi) {
     });
     if (rc == DG_OK) rc = copy_out(h, dphi + p0 * 3 * h->nbf, buf, (size_t)n * 3 * h->nbf);
   }
-  dfree(buf);
+  dfree_call(buf, rc, h->stream);
   return rc;
 }
 
@@ -4528,7 +4541,7 @@ int dg_get_density_gradients(dg_handle* h, double* grad) {
                        h->zsum, nullptr, buf);
   });
   if (rc == DG_OK) rc = copy_out(h, grad, buf, (size_t)3 * h->npts);
-  dfree(buf);
+  dfree_call(buf, rc, h->stream);
   return rc;
 }
 
@@ -4634,7 +4647,7 @@ int dg_mfma_probe(const double* a, const double* b, double* d) {
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipMemcpy(d, buf + 128, 256 * 8, hipMemcpyDeviceToHost);
-  dfree(buf);
+  dfree_call(buf, e, nullptr);
   if (e != hipSuccess) return fail(DG_ERR_HIP, std::string("dg_mfma_probe: ") + hipGetErrorString(e));
   return DG_OK;
 }
@@ -4650,7 +4663,7 @@ int dg_mfma_probe_f32(const float* a, const float* b, float* d) {
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipMemcpy(d, buf + 128, 256 * 4, hipMemcpyDeviceToHost);
-  dfree(buf);
+  dfree_call(buf, e, nullptr);
   if (e != hipSuccess) return fail(DG_ERR_HIP, std::string("dg_mfma_probe_f32: ") + hipGetErrorString(e));
   return DG_OK;
 }
@@ -4663,7 +4676,7 @@ int dg_selftest_mfma(int* ok) {
   hipLaunchKernelGGL(k_mfma_probe, dim3(1), dim3(64), 0, 0, d);
   std::vector<double> out(256);
   hipError_t e = hipMemcpy(out.data(), d, 256 * 8, hipMemcpyDeviceToHost);
-  dfree(d);
+  dfree_call(d, e, nullptr);
   if (e != hipSuccess) return fail(DG_ERR_HIP, std::string("dg_selftest_mfma: ") + hipGetErrorString(e));
   int good = 1;
   for (int lane = 0; lane < 64; ++lane)
