@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "../../include/dftgrid.h"
+#include "atom_order.h"
 #include "device_pool.h"
 #include "grid_tables.h"
 #include "unroll.h"
@@ -2342,18 +2343,7 @@ __global__ __launch_bounds__(256) void k_atom_order(const double* __restrict__ a
   const long e = (long)blockIdx.x * 256 + threadIdx.x;
   if (e >= (long)natoms * natoms) return;
   const int a = (int)(e / natoms), m = (int)(e % natoms);
-  auto d2 = [&](int k) {
-    const double dx = atoms[4 * k] - atoms[4 * a], dy = atoms[4 * k + 1] - atoms[4 * a + 1],
-                 dz = atoms[4 * k + 2] - atoms[4 * a + 2];
-    return dx * dx + dy * dy + dz * dz;
-  };
-  const double d = d2(m);
-  int rank = 0;
-  for (int k = 0; k < natoms; ++k) {
-    const double x = d2(k);
-    rank += (x < d || (x == d && k < m)) ? 1 : 0;
-  }
-  order[(long)a * natoms + rank] = m;
+  order[(long)a * natoms + dg::distance_place(atoms, natoms, a, m)] = m;
 }
 
 // Bound by the FP64 vector unit: per point, the cell functions (phase 1) and one ratio
