@@ -247,17 +247,17 @@ __global__ void k_phi(const double* __restrict__ atoms, int nshell, const int* _
 }
 
 // Tile mask: bit T of mask[b] is set when some |phi| of basis tile T (16
-// functions) exceeds screen on the 64-point block b.  One wave per block.
-constexpr double kAmpReach = 0x1p-106;
-
+// functions) exceeds its limit on the 64-point block b, screen or, where given, the
+// function's own (amplitude_limit).  One wave per block.
 __global__ __launch_bounds__(64) void k_block_mask(const double* __restrict__ phi, int ldphi, int ntb,
-                                                   double screen, unsigned* mask) {
+                                                   double screen, const double* __restrict__ limit,
+                                                   unsigned* mask) {
   const long p = (long)blockIdx.x * 64 + threadIdx.x;
   const double* row = phi + p * ldphi;
   unsigned bits = 0u;
   for (int T = 0; T < ntb; ++T) {
     bool on = false;  // NaN counts: it has to show in the results
-    for (int i = 0; i < 16; ++i) on |= !(fabs(row[16 * T + i]) <= screen);
+    for (int i = 0; i < 16; ++i) on |= !(fabs(row[16 * T + i]) <= (limit ? limit[16 * T + i] : screen));
     if (on) bits |= 1u << T;
   }
   for (int o = 32; o > 0; o >>= 1) bits |= (unsigned)__shfl_xor((int)bits, o);
@@ -2893,6 +2893,7 @@ struct dg_handle {
   double* phi = nullptr;
   int *sh_atom = nullptr, *sh_L = nullptr, *sh_nprim = nullptr, *sh_off = nullptr, *sh_cgf = nullptr;
   double* sh_amin = nullptr;  // per shell, its smallest exponent
+  double* amp_lim = nullptr;  // per function, the amplitude below which it is out of reach
   double *pr_alpha = nullptr, *pr_cn0 = nullptr, *pr_cn1 = nullptr;
   double *P = nullptr, *pfrag = nullptr, *rho = nullptr, *uxc = nullptr, *exd = nullptr;
   double *uJ = nullptr, *V = nullptr, *vcell = nullptr, *vpart = nullptr;
@@ -2914,8 +2915,8 @@ struct dg_handle {
   int4* coef_grp = nullptr;
   // screening masks
   double screen = 0.0;
-  BlockClasses reach;      // at screen, or at kAmpReach without
-  BlockClasses adj_reach;  // screened handles: at kAmpReach, for the force terms (on their first use)
+  BlockClasses reach;      // at screen, or at amp_lim without
+  BlockClasses adj_reach;  // screened handles: at amp_lim, for the force terms (on their first use)
   // reduced-precision mode
   float* phf = nullptr;  // FP32 amplitudes
   double* ej_part = nullptr;
@@ -2966,7 +2967,7 @@ struct dg_handle {
                       V,     vcell, vpart, q,      qc,    exc_part, scalars, ylm, minvT, shc,
                       knots, invh,  KD,    rho_lm, U,     tab,  cpart, J,   XC,
                       adj_ub, adj_ab, adj_udp, adj_T, adj_frag, adj_part, adj_mot, adj_lam, adj_out, adj_dP,
-                      mol_z, mol_fac, mol_qraw, atom_exc, atom_ej, qpart, uG, coef, mono, sh_amin};
+                      mol_z, mol_fac, mol_qraw, atom_exc, atom_ej, qpart, uG, coef, mono, sh_amin, amp_lim};
     for (double* b : bufs)
       if (b) dfree(b);
     int* ibufs[] = {sh_atom, sh_L, sh_nprim, sh_off, sh_cgf, blocks, ntask, ash_start, ash_list, atom_order,
@@ -3163,7 +3164,7 @@ void launch_tmat_rows(int nt, hipStream_t st, long npts_pad, const double* phi, 
   }
 }
 
-int block_reach(dg_handle* h, double limit, std::vector<unsigned>& mk, BlockClasses& r);
+int block_reach(dg_handle* h, double screen, std::vector<unsigned>& mk, BlockClasses& r);
 
 // The function tiles the force terms take per point block (mask null: all).
 // Screened handles take them at the reach of unscreened ones: their forces leave
@@ -3174,7 +3175,7 @@ int force_reach(dg_handle* h, const BlockClasses** r) {
   if (!own || h->adj_reach.mask) return DG_OK;
   std::vector<unsigned> mk(h->npts_pad / 64);
   BlockClasses made;  // the handle's only once it is whole
-  const int rc = block_reach(h, kAmpReach, mk, made);
+  const int rc = block_reach(h, 0.0, mk, made);
   if (rc == DG_OK) {
     h->adj_reach = made;
   } else {
@@ -3499,6 +3500,20 @@ int copy_out(dg_handle* h, double* dst, const double* src, size_t n) {
   return sync(h);
 }
 
+// The amplitude at or below which a function of shell s is out of reach without
+// screening, from a bound M of its largest amplitude (c: its primitives' c N).  Functions
+// of ordinary size, M >= 2^-10, are cut at 2^-106; smaller ones at the same distance
+// below their own size, so that a basis scaled down (and P scaled up) keeps its digits.
+double amplitude_limit(const dg_basis* b, int s, const double* c) {
+  double m = 0.0;  // r^L exp(-a r^2) is largest at r^2 = L / 2a
+  for (int k = 0; k < b->nprim[s]; ++k) {
+    const int i = b->offset[s] + k;
+    const double u = b->L[s] / (2.0 * 2.718281828459045 * b->alpha[i]);
+    m += std::fabs(c[i]) * (b->L[s] == 0 ? 1.0 : b->L[s] == 1 ? std::sqrt(u) : u);
+  }
+  return 0x1p-106 * std::min(1.0, 0x1p10 * m);  // (m not a number: 2^-106)
+}
+
 // The density's launches beyond 7 tiles: the blocks sorted by the number of
 // tiles that count there, a launch for every kernel size (kDensityTiles) that
 // at least kDensityClassMin blocks come to; fewer join the next larger one.
@@ -3538,13 +3553,14 @@ int block_classes(const std::vector<unsigned>& mk, int nt, BlockClasses& r) {
   return DG_OK;
 }
 
-// The tiles with an amplitude beyond limit, per 64-point block, and, past 7 tiles,
-// the blocks by their number.
-int block_reach(dg_handle* h, double limit, std::vector<unsigned>& mk, BlockClasses& r) {
+// The tiles with an amplitude beyond screen (0: beyond its function's reach), per
+// 64-point block, and, past 7 tiles, the blocks by their number.
+int block_reach(dg_handle* h, double screen, std::vector<unsigned>& mk, BlockClasses& r) {
   const long nblk = h->npts_pad / 64;
   DG_TRY(dalloc(&r.mask, nblk));
   DG_TRY(run(h, "block_mask", [&] {
-    hipLaunchKernelGGL(k_block_mask, dim3(nblk), dim3(64), 0, h->stream, h->phi, h->ldphi, h->ntb, limit, r.mask);
+    hipLaunchKernelGGL(k_block_mask, dim3(nblk), dim3(64), 0, h->stream, h->phi, h->ldphi, h->ntb, screen,
+                       screen > 0.0 ? nullptr : h->amp_lim, r.mask);
   }));
   HIP_TRY(hipMemcpyAsync(mk.data(), r.mask, nblk * 4, hipMemcpyDeviceToHost, h->stream));
   DG_TRY(sync(h));
@@ -3553,9 +3569,9 @@ int block_reach(dg_handle* h, double limit, std::vector<unsigned>& mk, BlockClas
 
 // The tiles that count per 64-point block (k_block_mask) and, for the 2-D
 // contraction, the point blocks of every tile block and the order its
-// work-groups run in.  Without screening a tile counts where an amplitude
-// exceeds kAmpReach = 2^-106, the square of an FP64 rounding: a product with a
-// smaller amplitude lies as far below the last bit of a sum of order one as
+// work-groups run in.  Without screening a tile counts where an amplitude exceeds
+// its limit (amplitude_limit), about 2^-106, the square of an FP64 rounding: a product
+// with a smaller amplitude lies as far below the last bit of a sum of order one as
 // that bit lies below the sum, so leaving it out changes no digit of rho, J or
 // XC.  The Gaussians of a 6-31G alkane end there at about 21 bohr, so that of
 // C30H62's tile pairs a third are left in the density and half in the
@@ -3567,7 +3583,7 @@ int tile_reach(dg_handle* h, const std::vector<int> (&cbs)[2]) {
   const bool two_d = h->ntb > 5;
   if (h->screen == 0.0 && !two_d) return DG_OK;
   std::vector<unsigned> mk(nblk);
-  DG_TRY(block_reach(h, h->screen > 0.0 ? h->screen : kAmpReach, mk, h->reach));
+  DG_TRY(block_reach(h, h->screen, mk, h->reach));
   if (!two_d) return DG_OK;
   size_t ncpart = 0;
   for (int q = 0; q < 2; ++q) {
@@ -3894,6 +3910,11 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
       cn1[i] = c * dg::gto_norm(a, L == 2 ? 1 : L, L == 2 ? 1 : 0, 0);
     }
   }
+  std::vector<double> amp_lim(16 * (size_t)h->ntb, 0.0);
+  for (int s = 0; s < h->nshell && !bs; ++s)
+    for (int c = 0; c < (basis->L[s] + 1) * (basis->L[s] + 2) / 2; ++c)
+      amp_lim[cgf_off[s] + c] =
+          amplitude_limit(basis, s, basis->L[s] == 2 && (c == 1 || c == 2 || c == 4) ? cn1.data() : cn0.data());
   std::vector<double> atoms(4 * h->natoms), invR((size_t)h->natoms * h->natoms, 0.0);
   for (int a = 0; a < h->natoms; ++a) {
     for (int d = 0; d < 3; ++d) atoms[4 * a + d] = mol->xyz[3 * a + d];
@@ -4061,6 +4082,7 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
   DG_TRY(dalloc(&h->sh_off, h->nshell));
   DG_TRY(dalloc(&h->sh_cgf, h->nshell));
   DG_TRY(dalloc(&h->sh_amin, h->nshell));
+  DG_TRY(dalloc(&h->amp_lim, amp_lim.size()));
   DG_TRY(dalloc(&h->pr_alpha, nprim_tot));
   DG_TRY(dalloc(&h->pr_cn0, nprim_tot));
   DG_TRY(dalloc(&h->pr_cn1, nprim_tot));
@@ -4126,6 +4148,7 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
   HIP_TRY(up(h->sh_off, basis->offset, h->nshell * 4));
   HIP_TRY(up(h->sh_cgf, cgf_off.data(), h->nshell * 4));
   HIP_TRY(up(h->sh_amin, amin.data(), h->nshell * 8));
+  HIP_TRY(up(h->amp_lim, amp_lim.data(), amp_lim.size() * 8));
   HIP_TRY(up(h->pr_alpha, alpha.data(), nprim_tot * 8));
   HIP_TRY(up(h->pr_cn0, cn0.data(), nprim_tot * 8));
   HIP_TRY(up(h->pr_cn1, cn1.data(), nprim_tot * 8));
