@@ -248,9 +248,13 @@ __global__ void k_phi(const double* __restrict__ atoms, int nshell, const int* _
 
 // Tile mask: bit T of mask[b] is set when some |phi| of basis tile T (16
 // functions) exceeds its limit on the 64-point block b, screen or, where given, the
-// function's own (amplitude_limit).  One wave per block.
+// function's own (amplitude_limit).  One wave per block.  By its functions' own limits
+// a tile counts in any case on a last block of fewer than 64 points: few points may all
+// lie in a nodal plane of a tile's only functions within reach, where the force terms
+// take gradients that do not vanish.  (64 neighbours of an angular rule lie in no plane,
+// so on whole blocks a gradient within reach comes with an amplitude.)
 __global__ __launch_bounds__(64) void k_block_mask(const double* __restrict__ phi, int ldphi, int ntb,
-                                                   double screen, const double* __restrict__ limit,
+                                                   double screen, const double* __restrict__ limit, long npts,
                                                    unsigned* mask) {
   const long p = (long)blockIdx.x * 64 + threadIdx.x;
   const double* row = phi + p * ldphi;
@@ -261,6 +265,7 @@ __global__ __launch_bounds__(64) void k_block_mask(const double* __restrict__ ph
     if (on) bits |= 1u << T;
   }
   for (int o = 32; o > 0; o >>= 1) bits |= (unsigned)__shfl_xor((int)bits, o);
+  if (limit && p - threadIdx.x == npts / 64 * 64 && npts % 64 != 0) bits = ~0u >> (32 - ntb);
   if (threadIdx.x == 0) mask[blockIdx.x] = bits;
 }
 
@@ -3560,7 +3565,7 @@ int block_reach(dg_handle* h, double screen, std::vector<unsigned>& mk, BlockCla
   DG_TRY(dalloc(&r.mask, nblk));
   DG_TRY(run(h, "block_mask", [&] {
     hipLaunchKernelGGL(k_block_mask, dim3(nblk), dim3(64), 0, h->stream, h->phi, h->ldphi, h->ntb, screen,
-                       screen > 0.0 ? nullptr : h->amp_lim, r.mask);
+                       screen > 0.0 ? nullptr : h->amp_lim, h->npts, r.mask);
   }));
   HIP_TRY(hipMemcpyAsync(mk.data(), r.mask, nblk * 4, hipMemcpyDeviceToHost, h->stream));
   DG_TRY(sync(h));
