@@ -2372,7 +2372,8 @@ __global__ __launch_bounds__(64) void k_force_becke(const double* __restrict__ a
                                                     const double* __restrict__ ab, long nblk,
                                                     double* part, double* mot, int* overflow) {
   // the point's cell functions above the skip level: atom and P_n (|r - R_n| is
-  // recomputed where needed: 10 bytes per entry keep ten work-groups per CU)
+  // recomputed where needed: 10 bytes per entry and the sums keep nine work-groups per
+  // CU at 92 atoms)
   __shared__ unsigned short act_n[kBeckeActive * 64];
   __shared__ double act_P[kBeckeActive * 64];
   // the work-group's sums per atom (lane 63 adds, in program order), added to part at
@@ -2526,6 +2527,7 @@ __global__ __launch_bounds__(64) void k_force_becke(const double* __restrict__ a
       }
   }
   for (int e = lane; e < 3 * natoms; e += 64) bsum[e] = 0.0;
+  __syncthreads();  // lane 63 adds to what the other lanes cleared
   double own_acc[3] = {0.0, 0.0, 0.0};
   // Every pair (active n, atom m != n) enters twice with the same
   // rho = ratio(mu_nm), f = P_n rho / R_nm and g = f mu / R_nm: into dP_n/dR_m as
