@@ -247,25 +247,23 @@ __global__ void k_phi(const double* __restrict__ atoms, int nshell, const int* _
 }
 
 // Tile mask: bit T of mask[b] is set when some |phi| of basis tile T (16
-// functions) exceeds its limit on the 64-point block b, screen or, where given, the
-// function's own (amplitude_limit).  One wave per block.  By its functions' own limits
-// a tile counts in any case on a last block of fewer than 64 points: few points may all
+// functions) exceeds limit on the 64-point block b.  One wave per block.  With whole, a
+// tile counts in any case on a last block of fewer than 64 points: few points may all
 // lie in a nodal plane of a tile's only functions within reach, where the force terms
 // take gradients that do not vanish.  (64 neighbours of an angular rule lie in no plane,
 // so on whole blocks a gradient within reach comes with an amplitude.)
 __global__ __launch_bounds__(64) void k_block_mask(const double* __restrict__ phi, int ldphi, int ntb,
-                                                   double screen, const double* __restrict__ limit, long npts,
-                                                   unsigned* mask) {
+                                                   double limit, long npts, bool whole, unsigned* mask) {
   const long p = (long)blockIdx.x * 64 + threadIdx.x;
   const double* row = phi + p * ldphi;
   unsigned bits = 0u;
   for (int T = 0; T < ntb; ++T) {
     bool on = false;  // NaN counts: it has to show in the results
-    for (int i = 0; i < 16; ++i) on |= !(fabs(row[16 * T + i]) <= (limit ? limit[16 * T + i] : screen));
+    for (int i = 0; i < 16; ++i) on |= !(fabs(row[16 * T + i]) <= limit);
     if (on) bits |= 1u << T;
   }
   for (int o = 32; o > 0; o >>= 1) bits |= (unsigned)__shfl_xor((int)bits, o);
-  if (limit && p - threadIdx.x == npts / 64 * 64 && npts % 64 != 0) bits = ~0u >> (32 - ntb);
+  if (whole && p - threadIdx.x == npts / 64 * 64 && npts % 64 != 0) bits = ~0u >> (32 - ntb);
   if (threadIdx.x == 0) mask[blockIdx.x] = bits;
 }
 
@@ -2900,7 +2898,6 @@ struct dg_handle {
   double* phi = nullptr;
   int *sh_atom = nullptr, *sh_L = nullptr, *sh_nprim = nullptr, *sh_off = nullptr, *sh_cgf = nullptr;
   double* sh_amin = nullptr;  // per shell, its smallest exponent
-  double* amp_lim = nullptr;  // per function, the amplitude below which it is out of reach
   double *pr_alpha = nullptr, *pr_cn0 = nullptr, *pr_cn1 = nullptr;
   double *P = nullptr, *pfrag = nullptr, *rho = nullptr, *uxc = nullptr, *exd = nullptr;
   double *uJ = nullptr, *V = nullptr, *vcell = nullptr, *vpart = nullptr;
@@ -2922,8 +2919,9 @@ struct dg_handle {
   int4* coef_grp = nullptr;
   // screening masks
   double screen = 0.0;
-  BlockClasses reach;      // at screen, or at amp_lim without
-  BlockClasses adj_reach;  // screened handles: at amp_lim, for the force terms (on their first use)
+  double amp_reach = 0.0;  // the amplitude at or below which unscreened work leaves a tile out
+  BlockClasses reach;      // at screen, or at amp_reach without
+  BlockClasses adj_reach;  // screened handles: at amp_reach, for the force terms (on their first use)
   // reduced-precision mode
   float* phf = nullptr;  // FP32 amplitudes
   double* ej_part = nullptr;
@@ -2974,7 +2972,7 @@ struct dg_handle {
                       V,     vcell, vpart, q,      qc,    exc_part, scalars, ylm, minvT, shc,
                       knots, invh,  KD,    rho_lm, U,     tab,  cpart, J,   XC,
                       adj_ub, adj_ab, adj_udp, adj_T, adj_frag, adj_part, adj_mot, adj_lam, adj_out, adj_dP,
-                      mol_z, mol_fac, mol_qraw, atom_exc, atom_ej, qpart, uG, coef, mono, sh_amin, amp_lim};
+                      mol_z, mol_fac, mol_qraw, atom_exc, atom_ej, qpart, uG, coef, mono, sh_amin};
     for (double* b : bufs)
       if (b) dfree(b);
     int* ibufs[] = {sh_atom, sh_L, sh_nprim, sh_off, sh_cgf, blocks, ntask, ash_start, ash_list, atom_order,
@@ -3507,18 +3505,23 @@ int copy_out(dg_handle* h, double* dst, const double* src, size_t n) {
   return sync(h);
 }
 
-// The amplitude at or below which a function of shell s is out of reach without
-// screening, from a bound M of its largest amplitude (c: its primitives' c N).  Functions
-// of ordinary size, M >= 2^-10, are cut at 2^-106; smaller ones at the same distance
-// below their own size, so that a basis scaled down (and P scaled up) keeps its digits.
-double amplitude_limit(const dg_basis* b, int s, const double* c) {
-  double m = 0.0;  // r^L exp(-a r^2) is largest at r^2 = L / 2a
-  for (int k = 0; k < b->nprim[s]; ++k) {
-    const int i = b->offset[s] + k;
-    const double u = b->L[s] / (2.0 * 2.718281828459045 * b->alpha[i]);
-    m += std::fabs(c[i]) * (b->L[s] == 0 ? 1.0 : b->L[s] == 1 ? std::sqrt(u) : u);
-  }
-  return 0x1p-106 * std::min(1.0, 0x1p10 * m);  // (m not a number: 2^-106)
+// The amplitude at or below which a function is out of reach without screening: 2^-106
+// where every function is of ordinary size, that is, a bound M of its largest amplitude is
+// at least 2^-10; with smaller ones (but for those that are 0) 2^-96 of the smallest M,
+// so that a basis scaled down, and P scaled up, keeps its digits.  cn0, cn1: c N of the
+// primitives.
+double amplitude_reach(const dg_basis* b, const double* cn0, const double* cn1) {
+  double smallest = 0x1p-10;
+  for (int s = 0; s < b->nshell; ++s)
+    for (const double* c : {cn0, cn1}) {
+      double m = 0.0;  // r^L exp(-a r^2) is largest at r^2 = L / 2a
+      for (int i = b->offset[s]; i < b->offset[s] + b->nprim[s]; ++i) {
+        const double u = b->L[s] / (2.0 * 2.718281828459045 * b->alpha[i]);
+        m += std::fabs(c[i]) * (b->L[s] == 0 ? 1.0 : b->L[s] == 1 ? std::sqrt(u) : u);
+      }
+      if (m > 0.0 && m < smallest) smallest = m;
+    }
+  return 0x1p-96 * smallest;
 }
 
 // The density's launches beyond 7 tiles: the blocks sorted by the number of
@@ -3560,14 +3563,14 @@ int block_classes(const std::vector<unsigned>& mk, int nt, BlockClasses& r) {
   return DG_OK;
 }
 
-// The tiles with an amplitude beyond screen (0: beyond its function's reach), per
-// 64-point block, and, past 7 tiles, the blocks by their number.
+// The tiles with an amplitude beyond screen (0: within reach), per 64-point block, and,
+// past 7 tiles, the blocks by their number.
 int block_reach(dg_handle* h, double screen, std::vector<unsigned>& mk, BlockClasses& r) {
   const long nblk = h->npts_pad / 64;
   DG_TRY(dalloc(&r.mask, nblk));
   DG_TRY(run(h, "block_mask", [&] {
-    hipLaunchKernelGGL(k_block_mask, dim3(nblk), dim3(64), 0, h->stream, h->phi, h->ldphi, h->ntb, screen,
-                       screen > 0.0 ? nullptr : h->amp_lim, h->npts, r.mask);
+    hipLaunchKernelGGL(k_block_mask, dim3(nblk), dim3(64), 0, h->stream, h->phi, h->ldphi, h->ntb,
+                       screen > 0.0 ? screen : h->amp_reach, h->npts, screen == 0.0, r.mask);
   }));
   HIP_TRY(hipMemcpyAsync(mk.data(), r.mask, nblk * 4, hipMemcpyDeviceToHost, h->stream));
   DG_TRY(sync(h));
@@ -3577,7 +3580,7 @@ int block_reach(dg_handle* h, double screen, std::vector<unsigned>& mk, BlockCla
 // The tiles that count per 64-point block (k_block_mask) and, for the 2-D
 // contraction, the point blocks of every tile block and the order its
 // work-groups run in.  Without screening a tile counts where an amplitude exceeds
-// its limit (amplitude_limit), about 2^-106, the square of an FP64 rounding: a product
+// amplitude_reach, 2^-106 for any usual basis, the square of an FP64 rounding: a product
 // with a smaller amplitude lies as far below the last bit of a sum of order one as
 // that bit lies below the sum, so leaving it out changes no digit of rho, J or
 // XC.  The Gaussians of a 6-31G alkane end there at about 21 bohr, so that of
@@ -3917,11 +3920,7 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
       cn1[i] = c * dg::gto_norm(a, L == 2 ? 1 : L, L == 2 ? 1 : 0, 0);
     }
   }
-  std::vector<double> amp_lim(16 * (size_t)h->ntb, 0.0);
-  for (int s = 0; s < h->nshell && !bs; ++s)
-    for (int c = 0; c < (basis->L[s] + 1) * (basis->L[s] + 2) / 2; ++c)
-      amp_lim[cgf_off[s] + c] =
-          amplitude_limit(basis, s, basis->L[s] == 2 && (c == 1 || c == 2 || c == 4) ? cn1.data() : cn0.data());
+  h->amp_reach = amplitude_reach(basis, cn0.data(), cn1.data());
   std::vector<double> atoms(4 * h->natoms), invR((size_t)h->natoms * h->natoms, 0.0);
   for (int a = 0; a < h->natoms; ++a) {
     for (int d = 0; d < 3; ++d) atoms[4 * a + d] = mol->xyz[3 * a + d];
@@ -4089,7 +4088,6 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
   DG_TRY(dalloc(&h->sh_off, h->nshell));
   DG_TRY(dalloc(&h->sh_cgf, h->nshell));
   DG_TRY(dalloc(&h->sh_amin, h->nshell));
-  DG_TRY(dalloc(&h->amp_lim, amp_lim.size()));
   DG_TRY(dalloc(&h->pr_alpha, nprim_tot));
   DG_TRY(dalloc(&h->pr_cn0, nprim_tot));
   DG_TRY(dalloc(&h->pr_cn1, nprim_tot));
@@ -4155,7 +4153,6 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
   HIP_TRY(up(h->sh_off, basis->offset, h->nshell * 4));
   HIP_TRY(up(h->sh_cgf, cgf_off.data(), h->nshell * 4));
   HIP_TRY(up(h->sh_amin, amin.data(), h->nshell * 8));
-  HIP_TRY(up(h->amp_lim, amp_lim.data(), amp_lim.size() * 8));
   HIP_TRY(up(h->pr_alpha, alpha.data(), nprim_tot * 8));
   HIP_TRY(up(h->pr_cn0, cn0.data(), nprim_tot * 8));
   HIP_TRY(up(h->pr_cn1, cn1.data(), nprim_tot * 8));

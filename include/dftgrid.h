@@ -70,9 +70,9 @@ typedef struct {
    * basis function at every point): screen > 0 skips, in the density and in
    * the Fock contractions, each 64-point block's 16-wide groups of basis
    * functions whose |phi| stays at or below screen on the whole block; 0 skips,
-   * in bases of more than 80 functions, only those at or below 2^-106 (for functions
-   * whose largest amplitude M is under 2^-10, 2^-96 M): products of the square of an
-   * FP64 rounding, which no digit of a sum with terms of order one depends on.  What
+   * in bases of more than 80 functions, only those at or below 2^-106 (2^-96 M, where
+   * the smallest of the functions' largest amplitudes M is under 2^-10): products of the
+   * square of an FP64 rounding, which no digit of a sum with terms of order one depends on.  What
    * consists of such products alone comes out as 0: the density far outside the
    * molecule, elements between functions that meet nowhere above that level.
    * Single-molecule handles only. */
