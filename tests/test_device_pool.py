@@ -101,11 +101,11 @@ int main() {
     CHECK(!p.take(&a, 512) && !p.take(&b, 512));
     p.give(a);
     no_host = true;
-    CHECK(p.take(&c, 512) == Device::kNoMemory && !c && p.take(&c, 4096) == Device::kNoMemory && !c);
-    p.give(b);
+    CHECK(p.take(&c, 4096) == Device::kNoMemory && !c && Device::live == 2);
+    CHECK(!p.take(&c, 512) && c == a);  // a block that is known needs none
+    p.give(b), p.give(c), p.give(c);
     no_host = false;
-    CHECK(Device::live == 1 && !p.take(&c, 512) && c == a);
-    p.give(c), p.release_kept();
+    CHECK(Device::live == 2 && p.release_kept());
     CHECK(Device::live == 0);
   }
   {  // many kept blocks: 1e5 takes beside 1e5 others, in well under the time of 1e10 steps
