@@ -292,56 +292,6 @@ int batch_mol_of_atom(const dg_handle* h, int k) {
   return m;
 }
 
-// Points of a cross-potential item of at most about len points: whole shells, one
-// at least.
-int cross_item_pts(const dg_handle* h, int len) { return std::max(1, len / h->nang) * h->nang; }
-
-// Work list of the cross-atom potentials: for every atom k, every other cell of its
-// molecule in equal runs of at most cross_item_pts(len) points, k ascending.
-std::vector<CrossItem> cross_items(const dg_handle* h, int len) {
-  std::vector<CrossItem> items;
-  const int cap = cross_item_pts(h, len) / h->nang, runs = (h->nrad + cap - 1) / cap;
-  for (int k = 0; k < h->natoms; ++k) {
-    int a0 = 0, a1 = h->natoms;
-    if (h->nmol) {
-      const int m = batch_mol_of_atom(h, k);
-      a0 = h->h_mol_atom0[m];
-      a1 = h->h_mol_atom0[m + 1];
-    }
-    for (int a = a0; a < a1; ++a)
-      for (int r = 0; r < runs && a != k; ++r) {
-        const int p = h->nrad * r / runs, q = h->nrad * (r + 1) / runs;
-        items.push_back({k, a, p, q - p});
-      }
-  }
-  return items;
-}
-
-// Points per item: 4096 where that makes four items per CU, else halved down to 512.
-// Longer items group better (C30H62: 7 % of the lanes idle at 4096, 11 at 2048) and a
-// work-group costs its launch; shorter ones spread a small molecule over the chip
-// (cross kernel, us at 4096 / 2048 / 1024 / 512: H2O 50 x 110 30 / 25 / 20 / 20, ethane
-// 20 x 146 35 / 29 / 22 / 20, benzene 85 / 80 / 87 / 127, C10H22 417 / 431 / 466 / 736).
-int cross_item_len(const dg_handle* h) {
-  int len = 4096;
-  while (len > 512 && cross_items(h, len).size() < 4 * 256) len /= 2;
-  return len;
-}
-
-int set_items(dg_handle* h, int len) {
-  const std::vector<CrossItem> items = cross_items(h, len);
-  const int pts = cross_item_pts(h, len), maxt = cross_max_tasks(pts, h->nrad);
-  if (items.size() > h->items_cap || items.size() * maxt > h->task_cap)
-    return fail(DG_ERR_INVALID, "cross-potential item list exceeds its buffer");
-  if (!items.empty())
-    HIP_TRY(hipMemcpy(h->items, items.data(), items.size() * sizeof(CrossItem), hipMemcpyHostToDevice));
-  h->nitems = (int)items.size();
-  h->item_pts = pts;
-  h->max_tasks = maxt;
-  h->item_len = len;
-  return sort_items(h);
-}
-
 std::vector<int> batch_chunks(const dg_handle* h, int len, std::vector<int>* first) {
   std::vector<int> ch;
   first->assign(h->nmol + 1, 0);
@@ -418,7 +368,7 @@ int batch_setup(dg_handle* h) {
   HIP_TRY(hipMemcpy(h->mol_poff, h->h_mol_poff.data(), (nm + 1) * 8, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(h->mol_z, mz.data(), nm * 8, hipMemcpyHostToDevice));
   DG_TRY(set_bchunks(h, h->bchunk_len));
-  DG_TRY(set_items(h, h->item_len));
+  DG_TRY(sort_cross(h));
   const size_t lds = (size_t)h->max_mol_atoms * 64 * 8;
   if (lds > 160 * 1024) return fail(DG_ERR_UNSUPPORTED, "dg_batch_create: too many atoms in a molecule");
   HIP_TRY(hipFuncSetAttribute((const void*)k_becke_batch, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -654,8 +604,8 @@ int dg_batch_autotune(dg_batch* b, int* chunk_len, int* item_len, double* best_m
   const bool prof = h->prof;
   h->prof = false;
   drop_graph(h);
-  double best_c = 1e30, best_i = 1e30;
-  int bc = h->bchunk_len, bi = h->item_len;
+  double best_c = 1e30, hartree = 0.0;
+  int bc = h->bchunk_len;
   for (int len : kChunkCandidates) {
     DG_TRY(set_bchunks(h, len));
     double ms = 0.0;
@@ -666,22 +616,13 @@ int dg_batch_autotune(dg_batch* b, int* chunk_len, int* item_len, double* best_m
     }
   }
   DG_TRY(set_bchunks(h, bc));
-  for (int len : kItemCandidates) {
-    DG_TRY(set_items(h, len));
-    double ms = 0.0;
-    DG_TRY(time_ms(h, 3, [&] { return stage_hartree(h); }, &ms));
-    if (ms < best_i) {
-      best_i = ms;
-      bi = len;
-    }
-  }
-  DG_TRY(set_items(h, bi));
+  DG_TRY(time_ms(h, 3, [&] { return stage_hartree(h); }, &hartree));
   h->prof = prof;
   if (chunk_len) *chunk_len = bc;
-  if (item_len) *item_len = bi;
+  if (item_len) *item_len = kCrossWaves * kTaskPts;
   if (best_ms) {
     best_ms[0] = best_c;
-    best_ms[1] = best_i;
+    best_ms[1] = hartree;
   }
   return sync(h);
 }

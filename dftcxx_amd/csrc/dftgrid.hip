@@ -967,6 +967,7 @@ struct CoefArgs {
   const double* invh;  // 1/(x_t - x_{t-1})
   const double* mono;
   const int4* grp;
+  const unsigned char* used;  // [natoms][nrad+1]: some point lies in the interval
   int nrad, nlm, lmax;
   long total;  // natoms (nrad+1) nlm
   double* coef;
@@ -976,6 +977,7 @@ __device__ __forceinline__ void cross_coef(const CoefArgs& A, long e) {
   if (e >= A.total) return;
   const int q = (int)(e % A.nlm);
   const long ks = e / A.nlm;
+  if (!A.used[ks]) return;
   const int key = (int)(ks % (A.nrad + 1)), k = (int)(ks / (A.nrad + 1));
   const int4 g = A.grp[q];
   const int m = g.x, i = g.y, L1 = A.lmax + 1, n = A.nrad;
@@ -1015,94 +1017,185 @@ __global__ __launch_bounds__(256) void k_vcell_coef(const double* __restrict__ U
     cross_coef(C, (long)(blockIdx.x - nvb) * 256 + threadIdx.x);
 }
 
-// Work items: runs of whole shells (the nang points of one radius) of one cell other
-// than k.
-struct CrossItem {
-  int k;       // atom whose expansion is evaluated
-  int cell;    // atom whose shells these are
-  int i0;      // first radial index
-  int nshell;
+// The points outside cell k, by spline interval of their distance to atom k, cut into
+// tasks of at most kTaskPts points of one interval: counts per chunk of `chunk` points
+// and key, their scan over the chunks and the keys, then the points by key and their
+// tasks.  All other cells are sorted together, so that on any angular grid the tasks are
+// full but for one an interval (with 500-point runs of one cell's shells, 50-point shells
+// left more than half of the lanes idle).  The order inside an interval does not matter: a
+// point's potential does not depend on its slot.
+constexpr int kTaskPts = 128;  // two per lane of one wave
+struct CrossTask {
+  long slot;  // first in perm
+  int k;
+  unsigned last_key;  // points - 1 | interval key << 7 (keys up to 3777, see dg_create)
+};
+struct CrossSort {
+  const double *atoms, *rad, *leb, *knots;
+  const long* vbase;
+  const int *atom_mol, *mol_atom0;  // null for one molecule
+  const int* chunk0;  // [natoms+1] first chunk
+  int natoms, nrad, nang, chunk;
+  long cell;
+  double inv_nang, inv_nrad;
+  double* vpart;        // its room holds the points' keys between the passes
+  int* cnt;             // [chunks][nrad+1] points, then slots before the chunk's
+  int2* group;          // [natoms][nrad+1] {first slot, points}
+  int* ntask;           // [natoms] tasks of an atom, then [1] of all
+  unsigned char* used;  // [natoms][nrad+1]
+  unsigned* perm;       // point of a slot; atom k's from vbase[k] + its molecule's first point
+  CrossTask* task;
 };
 
-constexpr int kMaxItem = 4096;    // points of an item (their potentials sit in LDS)
-constexpr int kCrossThreads = 512;
-constexpr int kTaskPts = 128;     // points of a task: two per lane of one wave
+// One work-group's chunk of atom k's points.
+struct SortChunk {
+  int k, c;
+  long p0, n;          // the molecule's first point; points outside cell k
+  long base;           // first slot
+  unsigned short* key; // of the n points
+  __device__ __forceinline__ explicit SortChunk(const CrossSort& S) {
+    k = 0;  // the last atom whose first chunk is at or before this one
+    for (int hi = S.natoms; hi - k > 1;) {
+      const int mid = (k + hi) >> 1;
+      if (S.chunk0[mid] <= (int)blockIdx.x)
+        k = mid;
+      else
+        hi = mid;
+    }
+    c = (int)blockIdx.x - S.chunk0[k];
+    const int m = S.atom_mol ? S.atom_mol[k] : 0;
+    const int a0 = S.atom_mol ? S.mol_atom0[m] : 0, a1 = S.atom_mol ? S.mol_atom0[m + 1] : S.natoms;
+    p0 = a0 * S.cell;
+    n = (a1 - a0 - 1) * S.cell;
+    base = S.vbase[k] + p0;
+    key = reinterpret_cast<unsigned short*>(S.vpart + base);
+  }
+  // its points: u in [begin, end) of those outside cell k, and their place in the grid
+  __device__ __forceinline__ long begin(const CrossSort& S) const { return (long)c * S.chunk; }
+  __device__ __forceinline__ long end(const CrossSort& S) const { return min(n, (long)(c + 1) * S.chunk); }
+  __device__ __forceinline__ long point(const CrossSort& S, long u) const {
+    return p0 + u < k * S.cell ? p0 + u : p0 + u + S.cell;
+  }
+};
 
-// Upper bound of an item's tasks: full tasks of its points and one partial task per
-// spline interval it touches.
-__host__ __device__ inline int cross_max_tasks(int item_pts, int nrad) {
-  return item_pts / kTaskPts + (item_pts < nrad + 1 ? item_pts : nrad + 1) + 1;
+// The squares of the knots sit in LDS and stand for the knots: no square root.
+__global__ __launch_bounds__(256) void k_cross_count(CrossSort S) {
+  extern __shared__ double lds_dbl[];
+  const SortChunk C(S);
+  const int nk = S.nrad + 1;
+  double* k2 = lds_dbl;
+  int* cnt = reinterpret_cast<int*>(k2 + S.nrad);
+  for (int i = threadIdx.x; i < nk; i += 256) {
+    cnt[i] = 0;
+    if (i < S.nrad) k2[i] = S.knots[i] * S.knots[i];
+  }
+  __syncthreads();
+  const double ax = S.atoms[4 * C.k], ay = S.atoms[4 * C.k + 1], az = S.atoms[4 * C.k + 2];
+  const long end = C.end(S);
+  for (long u0 = C.begin(S) + threadIdx.x; u0 < end; u0 += 4 * 256) {
+    int key[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int p = (int)C.point(S, min(u0 + 256 * q, end - 1));
+      const int ai = (int)(((double)p + 0.5) * S.inv_nang), a = (int)(((double)ai + 0.5) * S.inv_nrad);
+      double x, y, z;
+      grid_xyz(S.atoms, S.rad, S.leb, a, ai - a * S.nrad, p - ai * S.nang, x, y, z);
+      x -= ax;
+      y -= ay;
+      z -= az;
+      key[q] = spline_key(x * x + y * y + z * z, k2, S.nrad);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (u0 + 256 * q < end) {
+        C.key[u0 + 256 * q] = (unsigned short)key[q];
+        atomicAdd(&cnt[key[q]], 1);
+      }
+  }
+  __syncthreads();
+  int* out = S.cnt + (long)blockIdx.x * nk;
+  for (int i = threadIdx.x; i < nk; i += 256) out[i] = cnt[i];
 }
 
-// Groups every item's points by spline interval (counting sort in LDS) and cuts the
-// groups into tasks of at most kTaskPts points, one wave each:
-//   perm[vbase[k] + p_begin + s]   offset (from p_begin) of the item's s-th point,
-//   task[item maxt + t]            first s | (points - 1) << 12 | interval key << 19
-// (keys up to nrad + 1 <= 3777, see dg_create's bound on the radial grid).
-// The order inside a group does not matter: a point's potential does not depend on
-// its slot.
-__global__ __launch_bounds__(kCrossThreads) void k_sort_items(
-    const CrossItem* __restrict__ items, const double* __restrict__ atoms, const double* __restrict__ px,
-    const double* __restrict__ py, const double* __restrict__ pz, const double* __restrict__ knots,
-    const long* __restrict__ vbase, int nrad, int nang, int maxt, unsigned short* perm, unsigned* task, int* ntask) {
-  __shared__ unsigned short out[kMaxItem];
-  extern __shared__ int lds_int[];
-  int* cnt = lds_int;             // [nrad + 1] points per key
-  int* base = cnt + nrad + 1;     // [nrad + 1] first slot
-  int* tbase = base + nrad + 1;   // [nrad + 1] first task
-  const CrossItem it = items[blockIdx.x];
-  const long pb = ((long)it.cell * nrad + it.i0) * nang;
-  const int len = it.nshell * nang;
-  for (int i = threadIdx.x; i <= nrad; i += kCrossThreads) cnt[i] = 0;
-  __syncthreads();
-  const double ax = atoms[4 * it.k], ay = atoms[4 * it.k + 1], az = atoms[4 * it.k + 2];
-  int key[kMaxItem / kCrossThreads], rank[kMaxItem / kCrossThreads];
+__global__ __launch_bounds__(64) void k_cross_scan(CrossSort S) {
+  const int k = blockIdx.x, nk = S.nrad + 1, nchunk = S.chunk0[k + 1] - S.chunk0[k];
+  int slot = 0, task = 0;
+  for (int i0 = 0; i0 < nk; i0 += 64) {
+    const int i = i0 + threadIdx.x;
+    int* x = S.cnt + (long)S.chunk0[k] * nk + i;
+    int n = 0;
+    for (int c0 = 0; i < nk && c0 < nchunk; c0 += 16) {  // 16 loads in flight
+      int v[16];
 #pragma unroll
-  for (int u = 0; u < kMaxItem / kCrossThreads; ++u) {
-    const int i = threadIdx.x + kCrossThreads * u;
-    key[u] = rank[u] = 0;
-    if (i < len) {
-      const double dx = px[pb + i] - ax, dy = py[pb + i] - ay, dz = pz[pb + i] - az;
-      key[u] = spline_key(sqrt(dx * dx + dy * dy + dz * dz), knots, nrad);
-      rank[u] = atomicAdd(&cnt[key[u]], 1);
-    }
-  }
-  __syncthreads();
-  if (threadIdx.x < 64) {  // exclusive scans over the keys, 64 at a time
-    int s = 0, t = 0;
-    for (int i0 = 0; i0 <= nrad; i0 += 64) {
-      const int i = i0 + threadIdx.x, c = i <= nrad ? cnt[i] : 0, w = (c + kTaskPts - 1) / kTaskPts;
-      int cs = c, ws = w;
-      for (int o = 1; o < 64; o <<= 1) {
-        const int a = __shfl_up(cs, o), b = __shfl_up(ws, o);
-        if ((int)threadIdx.x >= o) {
-          cs += a;
-          ws += b;
-        }
-      }
-      if (i <= nrad) {
-        base[i] = s + cs - c;
-        tbase[i] = t + ws - w;
-      }
-      s += __shfl(cs, 63);
-      t += __shfl(ws, 63);
-    }
-    if (threadIdx.x == 0) ntask[blockIdx.x] = t;
-  }
-  __syncthreads();
+      for (int c = 0; c < 16; ++c) v[c] = c0 + c < nchunk ? x[(long)(c0 + c) * nk] : 0;
 #pragma unroll
-  for (int u = 0; u < kMaxItem / kCrossThreads; ++u) {
-    const int i = threadIdx.x + kCrossThreads * u;
-    if (i < len) out[base[key[u]] + rank[u]] = (unsigned short)i;
+      for (int c = 0; c < 16; ++c) {
+        if (c0 + c < nchunk) x[(long)(c0 + c) * nk] = n;
+        n += v[c];
+      }
+    }
+    int ns = n, nt = (n + kTaskPts - 1) / kTaskPts;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int a = __shfl_up(ns, o), b = __shfl_up(nt, o);
+      if ((int)threadIdx.x >= o) {
+        ns += a;
+        nt += b;
+      }
+    }
+    if (i < nk) {
+      S.group[(long)k * nk + i] = make_int2(slot + ns - n, n);
+      S.used[(long)k * nk + i] = n > 0;
+    }
+    slot += __shfl(ns, 63);
+    task += __shfl(nt, 63);
   }
-  unsigned* tk = task + (long)blockIdx.x * maxt;
-  for (int i = threadIdx.x; i <= nrad; i += kCrossThreads)
-    for (int c = 0; kTaskPts * c < cnt[i]; ++c)
-      tk[tbase[i] + c] = (unsigned)(base[i] + kTaskPts * c) |
-                         (unsigned)(min(kTaskPts, cnt[i] - kTaskPts * c) - 1) << 12 | (unsigned)i << 19;
+  if (threadIdx.x == 0) S.ntask[k] = task;
+}
+
+__global__ __launch_bounds__(256) void k_cross_tasks(CrossSort S) {
+  extern __shared__ int lds_int[];  // the chunk's next slot of each key
+  const SortChunk C(S);
+  const int nk = S.nrad + 1;
+  const int2* group = S.group + (long)C.k * nk;
+  for (int i = threadIdx.x; i < nk; i += 256) lds_int[i] = group[i].x + S.cnt[(long)blockIdx.x * nk + i];
   __syncthreads();
-  unsigned short* pm = perm + vbase[it.k] + pb;
-  for (int i = threadIdx.x; i < len; i += kCrossThreads) pm[i] = out[i];
+  const long end = C.end(S);
+  for (long u0 = C.begin(S) + threadIdx.x; u0 < end; u0 += 4 * 256) {
+    int key[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) key[q] = C.key[min(u0 + 256 * q, end - 1)];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (u0 + 256 * q < end)
+        S.perm[C.base + atomicAdd(&lds_int[key[q]], 1)] = (unsigned)C.point(S, u0 + 256 * q);
+  }
+  if (C.c > 0 || threadIdx.x >= 64) return;
+  int before = 0, all = 0;  // tasks of the atoms before k, of all atoms
+  for (int j = threadIdx.x; j < S.natoms; j += 64) {
+    const int m = S.ntask[j];
+    before += j < C.k ? m : 0;
+    all += m;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    before += __shfl_xor(before, o);
+    all += __shfl_xor(all, o);
+  }
+  if (threadIdx.x == 0) S.ntask[S.natoms] = all;  // the same from every atom
+  CrossTask* out = S.task + before;
+  for (int i0 = 0; i0 < nk; i0 += 64) {  // a key a lane
+    const int i = i0 + threadIdx.x;
+    const int2 g = i < nk ? group[i] : make_int2(0, 0);
+    const int m = (g.y + kTaskPts - 1) / kTaskPts;
+    int s = m;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int a = __shfl_up(s, o);
+      if ((int)threadIdx.x >= o) s += a;
+    }
+    for (int t = 0; t < m; ++t)
+      out[s - m + t] = CrossTask{C.base + g.x + t * kTaskPts, C.k,
+                                 (unsigned)(min(kTaskPts, g.y - t * kTaskPts) - 1) | (unsigned)i << 7};
+    out += __shfl(s, 63);
+  }
 }
 
 struct CrossArgs {
@@ -1111,14 +1204,13 @@ struct CrossArgs {
   const double* atoms;
   const double* knots;  // ascending, nrad
   const double* coef;   // see cross_coef
-  const CrossItem* items;
-  const unsigned short* perm;
-  const unsigned* task;
-  const int* ntask;
+  const unsigned* perm;
+  const CrossTask* task;
   double* vpart;        // partial potentials, atom k's at vpart + vbase[k] + p
   const long* vbase;
-  int nrad, nang, maxt;
-  float inv_nang;
+  const int* ntasks;
+  int task0, nrad, nang;
+  double inv_nang, inv_nrad;
 };
 
 // s += v c with a wave-uniform c read as a scalar operand (left to itself the compiler
@@ -1195,37 +1287,63 @@ __device__ __forceinline__ void cross_eval(const double* coef, const double (&x)
   });
 }
 
-// Potential of atom k's expansion at the points of one item.  A wave takes tasks of
-// up to kTaskPts points that share their spline interval, so the interval's
-// coefficients are wave-uniform: they come through the scalar cache and enter the
-// multiply-adds as scalar operands, with no LDS or vector-register traffic.
+// (x, y, z) to its unit vector; r and 1/r from the hardware reciprocal square root
+// (about 2^-26) and two coupled Newton steps.
+__device__ __forceinline__ void to_unit(double& x, double& y, double& z, double& r, double& ri) {
+  const double r2 = x * x + y * y + z * z;
+  double h = __builtin_amdgcn_rsq(r2);
+  r = r2 * h;
+  h *= 0.5;
+  double d = __fma_rn(-r, h, 0.5);
+  r = __fma_rn(r, d, r);
+  h = __fma_rn(h, d, h);
+  d = __fma_rn(-r, h, 0.5);
+  r = __fma_rn(r, d, r);
+  ri = 2.0 * __fma_rn(h, d, h);
+  x *= ri;
+  y *= ri;
+  z *= ri;
+}
+
+// Potential of atom k's expansion at the points of one task, one wave each.  The points
+// share their spline interval, so the interval's coefficients are wave-uniform: they come
+// through the scalar cache and enter the multiply-adds as scalar operands, with no LDS or
+// vector-register traffic.  Bound by the FP64 multiply-adds, 4 (lmax+1)^2 a point, where
+// the tasks fill the chip.
+// With items of up to 4096 points of one other cell, their potentials collected in LDS
+// and written in point order, the kernel took (us, before -> after) H2O 50 x 110 18.5 -> 9.0,
+// 26 atoms 60 x 50 lmax 10 107 -> 56, C10H22 75 x 302 447 -> 380, C30H62 3230 -> 2980, 256
+// small molecules at 60 x 50 lmax 10 690 -> 453, at 75 x 302 2125 -> 1877.  Tasks of 64
+// points: the same on H2O, 1 to 8 % slower elsewhere.
+constexpr int kCrossWaves = 4;
+constexpr int kCrossLaunch = 1 << 25;  // tasks: under 2^32 threads a launch
 template <int LMAX>
-__global__ __launch_bounds__(kCrossThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_hartree_cross(
+__global__ __launch_bounds__(64 * kCrossWaves) __attribute__((amdgpu_waves_per_eu(8))) void k_hartree_cross(
     CrossArgs A) {
-  extern __shared__ double vbuf[];  // potentials by offset in the item
-  const CrossItem it = A.items[blockIdx.x];
-  const long vb = A.vbase[it.k] + ((long)it.cell * A.nrad + it.i0) * A.nang;
-  const unsigned short* pm = A.perm + vb;
-  const unsigned* tk = A.task + (long)blockIdx.x * A.maxt;
-  const int nt = A.ntask[blockIdx.x];
-  const int lane = threadIdx.x & 63;
-  const double* rad = A.rad + it.i0;
-  const double* coef = A.coef + (long)it.k * (A.nrad + 1) * (4 * (LMAX + 1) * (LMAX + 1));
-  const double Dx = A.atoms[4 * it.cell] - A.atoms[4 * it.k], Dy = A.atoms[4 * it.cell + 1] - A.atoms[4 * it.k + 1],
-               Dz = A.atoms[4 * it.cell + 2] - A.atoms[4 * it.k + 2];
-  auto points = [&](auto Q, int s, int last, int key) {
+  __shared__ double park[kCrossWaves * kTaskPts];  // 1/r of the points, out of the registers' way
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int w = A.task0 + kCrossWaves * blockIdx.x + wave;
+  if (w >= *A.ntasks) return;
+  const CrossTask T = A.task[w];
+  const int k = T.k, last = T.last_key & 127, key = T.last_key >> 7;
+  const unsigned* pm = A.perm + T.slot;
+  const long vb = A.vbase[k];
+  constexpr int N = 4 * (LMAX + 1) * (LMAX + 1);
+  const double* coef = A.coef + ((long)k * (A.nrad + 1) + key) * N;
+  const double x0 = A.knots[max(key - 1, 0)], Ax = A.atoms[4 * k], Ay = A.atoms[4 * k + 1], Az = A.atoms[4 * k + 2];
+  double* mine = park + kTaskPts * wave + lane;
+  auto points = [&](auto Q) {
     double x[Q], y[Q], z[Q], t[Q], v[Q];
-    int e[Q];
-    const double x0 = A.knots[max(key - 1, 0)];
+    int p[Q];
     static_for<0, Q>([&](auto q) {
-      e[q] = pm[s + min(lane + 64 * q, last)];
-      // shell of the item and angular point: e < 4096, exact in FP32 with the half-step offset
-      const int sl = (int)(((float)e[q] + 0.5f) * A.inv_nang);
-      const int j = e[q] - sl * A.nang;
-      const double rs = rad[sl];
-      x[q] = __fma_rn(A.leb[4 * j], rs, Dx);
-      y[q] = __fma_rn(A.leb[4 * j + 1], rs, Dy);
-      z[q] = __fma_rn(A.leb[4 * j + 2], rs, Dz);
+      p[q] = (int)pm[min(lane + 64 * q, last)];  // (lanes past the end repeat the last point)
+      // p = (a nrad + i) nang + j
+      const int ai = (int)(((double)p[q] + 0.5) * A.inv_nang), a = (int)(((double)ai + 0.5) * A.inv_nrad);
+      const int j = p[q] - ai * A.nang;
+      const double rs = A.rad[ai - a * A.nrad];
+      x[q] = __fma_rn(A.leb[4 * j], rs, A.atoms[4 * a] - Ax);
+      y[q] = __fma_rn(A.leb[4 * j + 1], rs, A.atoms[4 * a + 1] - Ay);
+      z[q] = __fma_rn(A.leb[4 * j + 2], rs, A.atoms[4 * a + 2] - Az);
       // r and 1/r from the hardware reciprocal square root (about 2^-26) and two
       // coupled Newton steps
       const double r2 = x[q] * x[q] + y[q] * y[q] + z[q] * z[q];
@@ -1241,24 +1359,17 @@ __global__ __launch_bounds__(kCrossThreads) __attribute__((amdgpu_waves_per_eu(8
       y[q] *= ri;
       z[q] *= ri;
       t[q] = r - x0;
-      vbuf[e[q]] = ri;  // waits in the point's own slot (lanes past the end repeat the last point)
+      mine[64 * q] = ri;
     });
-    cross_eval<LMAX, Q>(coef + key * (4 * (LMAX + 1) * (LMAX + 1)), x, y, z, t, v);
+    cross_eval<LMAX, Q>(coef, x, y, z, t, v);
     static_for<0, Q>([&](auto q) {
-      if (lane + 64 * q <= last) vbuf[e[q]] *= v[q];
+      if (lane + 64 * q <= last) A.vpart[vb + p[q]] = mine[64 * q] * v[q];
     });
   };
-  for (int t = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); t < nt; t += kCrossThreads / 64) {
-    const unsigned T = __builtin_amdgcn_readfirstlane(tk[t]);
-    const int s = T & 4095, last = (T >> 12) & 127, key = T >> 19;
-    if (last >= 64)
-      points(std::integral_constant<int, 2>{}, s, last, key);
-    else
-      points(std::integral_constant<int, 1>{}, s, last, key);
-  }
-  __syncthreads();
-  const int len = it.nshell * A.nang;
-  for (int e = threadIdx.x; e < len; e += kCrossThreads) A.vpart[vb + e] = vbuf[e];
+  if (last >= 64)
+    points(std::integral_constant<int, 2>{});
+  else
+    points(std::integral_constant<int, 1>{});
 }
 
 // V[p] = sum_k (k == own ? vcell[p] : vpart_k[p]) over the atoms k of the
@@ -2909,12 +3020,14 @@ struct dg_handle {
   double *knots = nullptr, *invh = nullptr, *KD = nullptr;
   double *rho_lm = nullptr, *U = nullptr, *tab = nullptr;
   int* blocks = nullptr;
-  // cross-atom potentials: work items, their points by spline interval, their tasks
-  CrossItem* items = nullptr;
-  unsigned short* perm = nullptr;
-  unsigned* task = nullptr;
-  int* ntask = nullptr;
-  int nitems = 0, max_tasks = 0, item_pts = 0;
+  // cross-atom potentials: the points of the other cells by spline interval, their tasks
+  unsigned* perm = nullptr;
+  CrossTask* task = nullptr;
+  int *sort_cnt = nullptr, *ntask = nullptr;
+  const int* sort_chunk0 = nullptr;  // behind coef_grp
+  int2* sort_group = nullptr;
+  int sort_chunks = 0, sort_len = 4096, max_tasks = 0;
+  unsigned char* coef_used = nullptr;
   double *coef = nullptr, *mono = nullptr;
   int4* coef_grp = nullptr;
   // screening masks
@@ -2934,11 +3047,11 @@ struct dg_handle {
   double *mol_z = nullptr, *mol_fac = nullptr, *mol_qraw = nullptr, *atom_exc = nullptr, *atom_ej = nullptr;
   int* bchunks = nullptr;   // contraction chunks {m, p_begin, p_end}
   int* mol_chunk0 = nullptr;
-  int nbchunks = 0, max_mol_shells = 0, max_mol_atoms = 0, bchunk_len = 2048, item_len = 2048;
+  int nbchunks = 0, max_mol_shells = 0, max_mol_atoms = 0, bchunk_len = 2048;
   long packed = 0;  // sum of nbf_m^2
   std::vector<int> h_mol_atom0, h_mol_nbf;
   std::vector<long> h_mol_poff;
-  size_t items_cap = 0, task_cap = 0, bchunks_cap = 0;
+  size_t bchunks_cap = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   const void* graph_key[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -2985,9 +3098,8 @@ struct dg_handle {
       if (t.order) dfree(t.order);
     if (vbase) dfree(vbase);
     if (perm) dfree(perm);
-    if (items) dfree(items);
-    if (task) dfree(task);
     if (coef_grp) dfree(coef_grp);
+    for (void* b : {(void*)task, (void*)sort_cnt, (void*)sort_group, (void*)coef_used}) dfree(b);
     if (mol_poff) dfree(mol_poff);
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (graph) (void)hipGraphDestroy(graph);
@@ -3082,13 +3194,19 @@ void tile_block_lists(const std::vector<unsigned>& mk, const std::vector<int>& c
   }
 }
 
-// Groups the points of every cross-potential item by spline interval.
-int sort_items(dg_handle* h) {
-  if (h->nitems == 0) return DG_OK;
-  return run(h, "sort_items", [&] {
-    hipLaunchKernelGGL(k_sort_items, dim3(h->nitems), dim3(kCrossThreads), 3 * sizeof(int) * (h->nrad + 1), h->stream,
-                       h->items, h->atoms, h->px, h->py, h->pz, h->knots, h->vbase, h->nrad, h->nang, h->max_tasks,
-                       h->perm, h->task, h->ntask);
+// Sorts the points of the cross potentials and makes their tasks (once per handle).
+int sort_cross(dg_handle* h) {
+  if (h->sort_chunks == 0) return DG_OK;
+  const CrossSort s{h->atoms,       h->rad,    h->leb,       h->knots,      h->vbase,       h->atom_mol,
+                    h->mol_atom0,   h->sort_chunk0, h->natoms, h->nrad,     h->nang,        h->sort_len,
+                    h->cell,        1.0 / h->nang,  1.0 / h->nrad, h->vpart, h->sort_cnt,   h->sort_group,
+                    h->ntask,       h->coef_used,   h->perm,   h->task};
+  const dim3 grid(h->sort_chunks), block(256);
+  const size_t lds = sizeof(int) * (h->nrad + 1);
+  return run(h, "sort_cross", [&] {
+    hipLaunchKernelGGL(k_cross_count, grid, block, lds + sizeof(double) * h->nrad, h->stream, s);
+    hipLaunchKernelGGL(k_cross_scan, dim3(h->natoms), dim3(64), 0, h->stream, s);
+    hipLaunchKernelGGL(k_cross_tasks, grid, block, lds, h->stream, s);
   });
 }
 
@@ -3278,13 +3396,13 @@ void launch_rho_lm(dg_handle* h, int ti) {
 #undef DG_RHO
 }
 
-void launch_cross(dg_handle* h, const CrossArgs& a) {
-  const dim3 grid(h->nitems), block(kCrossThreads);
-  const size_t lds = sizeof(double) * h->item_pts;
+// Tasks [a.task0, a.task0 + n); those past the last one there is return at once.
+void launch_cross(dg_handle* h, const CrossArgs& a, int n) {
+  const dim3 grid(nblocks(n, kCrossWaves)), block(64 * kCrossWaves);
   switch (h->lmax) {
-#define DG_L(N)                                                             \
-  case N:                                                                   \
-    hipLaunchKernelGGL(k_hartree_cross<N>, grid, block, lds, h->stream, a); \
+#define DG_L(N)                                                           \
+  case N:                                                                 \
+    hipLaunchKernelGGL(k_hartree_cross<N>, grid, block, 0, h->stream, a); \
     break;
     DG_L(0) DG_L(1) DG_L(2) DG_L(3) DG_L(4) DG_L(5) DG_L(6) DG_L(7) DG_L(8) DG_L(9) DG_L(10) DG_L(11) DG_L(12)
 #undef DG_L
@@ -3305,15 +3423,15 @@ int stage_hartree(dg_handle* h) {
   DG_TRY(run(h, "vcell", [&] {
     const long ntiles = (long)h->natoms * ti * ((h->nang + 15) / 16);
     const int nvb = (int)nblocks(ntiles, 4);
-    CoefArgs c{h->tab, h->invh, h->mono, h->coef_grp, h->nrad, h->nlm, h->lmax, 0, h->coef};
-    if (h->nitems > 0) c.total = (long)h->natoms * (h->nrad + 1) * h->nlm;
+    CoefArgs c{h->tab, h->invh, h->mono, h->coef_grp, h->coef_used, h->nrad, h->nlm, h->lmax, 0, h->coef};
+    if (h->max_tasks > 0) c.total = (long)h->natoms * (h->nrad + 1) * h->nlm;
     hipLaunchKernelGGL(k_vcell_coef, dim3(nvb + nblocks(c.total, 256)), dim3(256), 0, h->stream, h->U, h->ylm,
                        h->rad, h->nrad, h->nang, h->nlm, ntiles, h->vcell, nvb, c);
   }));
-  if (h->nitems > 0) {
-    const CrossArgs a{h->rad,  h->leb,   h->atoms, h->knots, h->coef, h->items,     h->perm,         h->task,
-                      h->ntask, h->vpart, h->vbase, h->nrad,  h->nang, h->max_tasks, 1.0f / h->nang};
-    DG_TRY(run(h, "hartree_cross", [&] { launch_cross(h, a); }));
+  for (int t0 = 0; t0 < h->max_tasks; t0 += kCrossLaunch) {
+    const CrossArgs a{h->rad,  h->leb,   h->atoms, h->knots, h->coef,         h->perm,      h->task,
+                      h->vpart, h->vbase, h->ntask + h->natoms, t0, h->nrad, h->nang, 1.0 / h->nang, 1.0 / h->nrad};
+    DG_TRY(run(h, "hartree_cross", [&] { launch_cross(h, a, std::min(kCrossLaunch, h->max_tasks - t0)); }));
   }
   DG_TRY(run(h, "vreduce", [&] {
     hipLaunchKernelGGL(k_vreduce, dim3(nblocks(h->npts_pad, 256)), dim3(256), 0, h->stream, h->vpart,
@@ -3806,10 +3924,6 @@ struct BatchSpec {
   int nmol = 0;
   std::vector<int> mol_atom0, mol_shell0;
 };
-constexpr int kItemCandidates[] = {1024, 2048, 4096};  // points per cross-potential item
-int cross_item_pts(const dg_handle* h, int len);
-int cross_item_len(const dg_handle* h);
-std::vector<CrossItem> cross_items(const dg_handle* h, int len);
 int batch_alloc(dg_handle* h, const BatchSpec* bs, const std::vector<int>& amol);
 int batch_setup(dg_handle* h);
 
@@ -4009,10 +4123,12 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
     h->tb[q].ncb = (int)cbs[q].size() / 4;
   }
   h->nlda_blocks = h->npts_pad / 256;
-  // radial grids up to this size are taken (one l's spline table within 150 KB)
-  if ((2 * h->nrad + (size_t)h->nrad * (2 * h->lmax + 1) * 2 + kMaxItem) * sizeof(double) > 150 * 1024)
+  // radial grids up to this size are taken: 3776 nodes at most, whose keys' counts fit the
+  // sort's LDS and whose keys fit a task
+  if ((long)h->nrad * (h->lmax + 1) > 3776)
     return fail(DG_ERR_UNSUPPORTED, "dg_create: radial grid too large for the Hartree kernel");
-  // groups of the cross-potential coefficients, in the order the kernel reads them, and the monomial coefficients of the harmonics' polynomials in cos(theta)
+  // groups of the cross-potential coefficients, in the order the kernel reads them, and
+  // the monomial coefficients of the harmonics' polynomials in cos(theta)
   std::vector<int> cgrp;
   const int L1 = h->lmax + 1;
   std::vector<double> mono((size_t)L1 * L1 * L1, 0.0);
@@ -4045,19 +4161,26 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
     for (int k = 0; k < h->natoms; ++k) vbase[k] = (long)k * h->npts_pad;
     vtotal = (long)h->natoms * h->npts_pad;
   }
-  h->item_len = cross_item_len(h);
-  std::vector<CrossItem> items = cross_items(h, h->item_len);
-  h->nitems = (int)items.size();
-  h->items_cap = std::max<size_t>(items.size(), 1);
-  h->task_cap = h->items_cap * cross_max_tasks(cross_item_pts(h, h->item_len), h->nrad);
-  if (bs)  // room for the item lengths the batch autotuner tries
-    for (int len : kItemCandidates) {
-      const size_t n = cross_items(h, len).size();
-      h->items_cap = std::max(h->items_cap, n);
-      h->task_cap = std::max(h->task_cap, n * cross_max_tasks(cross_item_pts(h, len), h->nrad));
-    }
-  h->item_pts = cross_item_pts(h, h->item_len);
-  h->max_tasks = cross_max_tasks(h->item_pts, h->nrad);
+  // chunks of the points outside each cell, for their sort: of 4096 points, halved down
+  // to 512 until there are four to a CU
+  long others = 0;
+  for (int k = 0; k < h->natoms; ++k)
+    others += ((bs ? bs->mol_atom0[amol[k] + 1] - bs->mol_atom0[amol[k]] : h->natoms) - 1) * h->cell;
+  while (h->sort_len > 512 && others < 4 * 256L * h->sort_len) h->sort_len /= 2;
+  std::vector<int> chunk0(h->natoms + 1, 0);
+  for (int k = 0; k < h->natoms; ++k) {
+    const int m = amol[k];
+    const long n = ((bs ? bs->mol_atom0[m + 1] - bs->mol_atom0[m] : h->natoms) - 1) * h->cell;
+    chunk0[k + 1] = chunk0[k] + (int)((n + h->sort_len - 1) / h->sort_len);
+    // at most one partial task to an interval that has points
+    const long most = n / kTaskPts + std::min<long>(n, h->nrad + 1);
+    if (h->max_tasks + most > 0x7fffffffL)
+      return fail(DG_ERR_UNSUPPORTED, "dg_create: more than 2^31 cross-potential tasks");
+    h->max_tasks += (int)most;
+  }
+  h->sort_chunks = chunk0[h->natoms];
+  const size_t chunk0_at = cgrp.size();
+  cgrp.insert(cgrp.end(), chunk0.begin(), chunk0.end());
   // host-side checks and tables are done: from here on the device is used
   HIP_TRY(hipGetDevice(&h->device));
   HIP_TRY(hipStreamCreate(&h->stream));
@@ -4118,13 +4241,17 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
   DG_TRY(dalloc(&h->U, (size_t)h->natoms * h->nrad * h->nlm));
   DG_TRY(dalloc(&h->tab, (size_t)h->natoms * h->nrad * h->nlm * 2));
   DG_TRY(dalloc(&h->blocks, blocks.size()));
-  DG_TRY(dalloc(&h->items, h->items_cap));
-  DG_TRY(dalloc(&h->ntask, h->items_cap));
-  DG_TRY(dalloc(&h->task, h->task_cap));
-  DG_TRY(dalloc(&h->perm, h->nitems > 0 ? (size_t)vtotal : 1));
-  DG_TRY(dalloc(&h->coef, h->nitems > 0 ? (size_t)h->natoms * (h->nrad + 1) * h->nlm * 4 : 1));
+  const size_t nkeys = h->sort_chunks ? (size_t)h->natoms * (h->nrad + 1) : 0;
+  DG_TRY(dalloc(&h->ntask, h->natoms + 1));
+  DG_TRY(dalloc(&h->perm, nkeys ? (size_t)vtotal : 1));
+  DG_TRY(dalloc(&h->task, h->max_tasks));
+  DG_TRY(dalloc(&h->sort_cnt, (size_t)h->sort_chunks * (h->nrad + 1)));
+  DG_TRY(dalloc(&h->sort_group, nkeys));
+  DG_TRY(dalloc(&h->coef, nkeys * h->nlm * 4));
+  DG_TRY(dalloc(&h->coef_used, nkeys));
   DG_TRY(dalloc(&h->mono, mono.size()));
-  DG_TRY(dalloc(&h->coef_grp, cgrp.size() / 4));
+  DG_TRY(dalloc(&h->coef_grp, (cgrp.size() + 3) / 4));
+  h->sort_chunk0 = (int*)h->coef_grp + chunk0_at;
   if (h->ntb <= 5) DG_TRY(dalloc(&h->cpart, (size_t)h->nsplit_small * h->ngroups * 2 * 1024));
   for (int q = 0; q < 2; ++q) {
     DG_TRY(dalloc(&h->tb[q].cb, cbs[q].size()));
@@ -4167,7 +4294,6 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
     HIP_TRY(up(h->tb[q].cb, cbs[q].data(), cbs[q].size() * 4));
     HIP_TRY(up(h->tb[q].groups, cbg[q].data(), cbg[q].size() * 4));
   }
-  if (!items.empty()) HIP_TRY(up(h->items, items.data(), items.size() * sizeof(CrossItem)));
   HIP_TRY(up(h->mono, mono.data(), mono.size() * 8));
   HIP_TRY(up(h->coef_grp, cgrp.data(), cgrp.size() * 4));
   HIP_TRY(hipMemsetAsync(h->phi, 0, (size_t)(np + 1) * h->ldphi * 8, h->stream));
@@ -4209,7 +4335,7 @@ static int create_impl(const dg_molecule* mol, const dg_basis* basis, const dg_g
                          np * h->ldphi, h->phf);
     }));
   }
-  DG_TRY(sort_items(h));
+  DG_TRY(sort_cross(h));
   DG_TRY(tile_reach(h, cbs));
   DG_TRY(sync(h));
   guard.release();

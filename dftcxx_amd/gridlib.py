@@ -488,7 +488,7 @@ class Batch:
         _check(lib().dg_batch_set_stream(self.b, C.c_void_p(stream_ptr)))
 
     def autotune(self):
-        """(contraction chunk length, cross item length, their best ms) chosen on this batch."""
+        """(contraction chunk length, points of a cross-potential work-group, their ms) on this batch."""
         c, i = C.c_int(), C.c_int()
         ms = np.zeros(2)
         _check(lib().dg_batch_autotune(self.b, C.byref(c), C.byref(i), _d(ms)))

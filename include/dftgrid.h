@@ -317,9 +317,10 @@ int dg_batch_set_stream(dg_batch* b, void* stream);
 int dg_batch_build_device(dg_batch* b, const double* dP, double* dJ, double* dXC, double* dscalars);
 /* The same from and to host buffers (synchronous); any output may be NULL. */
 int dg_batch_build(dg_batch* b, const double* P, double* J, double* XC, double* scalars);
-/* Times the candidate contraction chunk lengths and cross-potential item
- * lengths on the batch (after one build) and keeps the fastest of each;
- * best_ms (2 doubles, may be NULL) receives their times. */
+/* Times the candidate contraction chunk lengths on the batch (after one build) and
+ * keeps the fastest; item_len receives the points of a work-group of the
+ * cross-potential kernel, which has one length, and best_ms (2 doubles, may be NULL)
+ * the times of the contraction and of the Hartree potential. */
 int dg_batch_autotune(dg_batch* b, int* chunk_len, int* item_len, double* best_ms);
 
 /* Runs the reference SCF (dg_scf_run) for every molecule of a batch, all of
