@@ -26,6 +26,7 @@
 
 #include "../../include/dftgrid.h"
 #include "atom_order.h"
+#include "device_math.h"
 #include "device_pool.h"
 #include "grid_tables.h"
 #include "unroll.h"
@@ -45,6 +46,8 @@ void dg::set_last_error(const std::string& msg) { g_last_error = msg; }
 
 namespace {
 
+using dg::rcp64;
+using dg::rsqrt64;
 using dg::static_for;
 
 #define HIP_TRY(expr)                                                                      \
@@ -91,18 +94,6 @@ __device__ __forceinline__ double wave_total(double v) {
   v += dpp_move<0x142, 0xa>(v);  // row_bcast15 into rows 1 and 3
   v += dpp_move<0x143, 0xc>(v);  // row_bcast31 into rows 2 and 3
   return v;
-}
-
-// 1/sqrt(x) and 1/x from the hardware estimates (about 2^-26) and Newton steps.
-__device__ __forceinline__ double rsqrt64(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  for (int k = 0; k < 2; ++k) y = y * __fma_rn(-0.5 * x * y, y, 1.5);
-  return y;
-}
-__device__ __forceinline__ double rcp64(double x) {
-  double y = __builtin_amdgcn_rcp(x);
-  for (int k = 0; k < 2; ++k) y = __fma_rn(y, __fma_rn(-x, y, 1.0), y);
-  return y;
 }
 
 constexpr int kMaxL = 12;  // largest lmax compiled
@@ -3644,7 +3635,9 @@ double amplitude_reach(const dg_basis* b, const double* cn0, const double* cn1) 
 
 // The density's launches beyond 7 tiles: the blocks sorted by the number of
 // tiles that count there, a launch for every kernel size (kDensityTiles) that
-// at least kDensityClassMin blocks come to; fewer join the next larger one.
+// at least kDensityClassMin blocks come to; fewer join the next larger one.  Any minimum
+// from 64 to 4096 is the same within 1 % (C30H62 build 11.6 to 11.8 ms, C10H22 1.36 to
+// 1.38); without the sizes, all blocks in the largest, C30H62 takes 15.0.
 constexpr int kDensityTiles[] = {4, 6, 8, 9, 10, 11, 12, 13, 14, 15, 16, 18, 20, 22, 25, 28, 32};
 constexpr long kDensityClassMin = 512;
 int block_classes(const std::vector<unsigned>& mk, int nt, BlockClasses& r) {

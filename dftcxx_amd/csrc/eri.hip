@@ -33,11 +33,13 @@
 #include <vector>
 
 #include "../../include/dftgrid.h"
+#include "device_math.h"
 #include "grid_tables.h"
 #include "unroll.h"
 
 namespace {
 
+using dg::rsqrt64;
 using dg::static_for;
 
 constexpr int kRec = 20;         // doubles per primitive-pair record
@@ -224,13 +226,6 @@ __global__ void k_boys_table(double* tab) {
   for (int n = 0; n < 12; ++n) tab[row * kBoysCols + n] = row ? F[n] : 1.0 / (2 * n + 1);  // (boys_dev clamps T)
   for (int n = 12; n < 15; ++n) tab[row * kBoysCols + n] = 0.0;
   tab[row * kBoysCols + 15] = exp(-T);
-}
-
-// 1/sqrt(x) from the hardware estimate (about 2^-26) and two Newton steps.
-__device__ __forceinline__ double rsqrt64(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  for (int k = 0; k < 2; ++k) y = y * __fma_rn(-0.5 * x * y, y, 1.5);
-  return y;
 }
 
 // F_n(T), n = 0..L, T clamped to >= 1e-8 (src/gamma.cpp:41-46).  Below T = 50, F_L by
