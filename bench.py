@@ -364,6 +364,7 @@ def main():
                 "pair_share": tile_pair_share(mol, grid.get_positions()),
                 "cross_launches": max(1, prof.get("hartree_cross", (0, nprof))[1] // nprof)}
         out["tile_pair_share"] = info["pair_share"]
+        out["amplitude_reach"] = 2.0 ** -106 if nbf > 80 and args.screen == 0.0 else args.screen
         dom = max(prof.items(), key=lambda kv: kv[1][0])[0]
         ms, cnt = prof[dom]
         avg_s = ms / cnt / 1e3
@@ -391,6 +392,8 @@ def main():
             if kname is not None:
                 roof["traffic"] = t[kname]
                 roof["traffic_source"] = f"profiles/traffic_{args.workload}.json[{kname}]"
+                roof["hbm_GBs"] = t[kname] / avg_s / 1e9
+                roof["hbm_frac"] = roof["hbm_GBs"] / PEAK_HBM_GBS
         out["roofline"] = roof
 
     # the reference's call sequence with host buffers (P in, J and XC out over PCIe,
