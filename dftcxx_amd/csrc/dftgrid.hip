@@ -366,8 +366,8 @@ __device__ __forceinline__ void bare_barrier() {
 // ahead of the MFMAs: C30H62 2.85 ms at the default reach, 5.55 ms dense.)
 // 8 N registers hold the amplitudes, which leaves two waves per SIMD up to 25
 // tiles and one beyond (three and four waves with 8 KB chunks on the small sizes:
-// 3 % slower).  C30H62 at the default reach: 2.3 ms, 70 % of the MFMA rate; what is
-// left is the start of each block, whose amplitudes wait on HBM.
+// 3 % slower).  C30H62 at the default reach: 2.5 ms, the MFMA pipes 48 to 71 % busy by
+// size; what is left is the start of each block, whose amplitudes wait on HBM.
 template <int N>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N <= 25 ? 2 : 1))) void
 k_density_ring(const double* __restrict__ phi, int ldphi, const double* __restrict__ frag, double* rho,
@@ -1445,6 +1445,8 @@ constexpr int kGroupEnd = 1 << 31;
 // later steps in flight.  Slot layout (doubles): the 4 points' rows of tiles
 // I0..I0+3 (point-major, 64 each), of tiles J0..J0+NJ-1 (16 NJ each), then
 // u0 and u1 of the 4 points.  The epilogue's LDS reduction reuses the ring.
+// C30H62, two outputs: 5.8 ms, in which 28.6 GB move (Phi's rows four times: tiles of one
+// block far apart in space) at 4.9 TB/s, with the MFMA pipes 78 % busy.
 template <int NOUT, int NJ, int D>
 __global__ __launch_bounds__(256, 3) void k_contract2d_lds(const double* __restrict__ phi, int ldphi,
                                                           const double* __restrict__ u0,
@@ -3068,7 +3070,10 @@ struct dg_handle {
     if (stream) {
       int cur = device;
       const bool other = hipGetDevice(&cur) == hipSuccess && cur != device && hipSetDevice(device) == hipSuccess;
-      if (hipDeviceSynchronize() != hipSuccess) (void)hipStreamSynchronize(stream);
+      if (hipDeviceSynchronize() != hipSuccess) {  // a capture somewhere in the process
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(stream);
+      }
       if (other) (void)hipSetDevice(cur);
     }
     double* bufs[] = {atoms, invR,  rad,   wrad,   leb,   px,     py,    pz,   w,     wb,
