@@ -2885,10 +2885,10 @@ __global__ void k_mfma_probe(double* out) {
 // program that makes a grid per geometry allocates the same sizes again and again,
 // and hipMalloc, hipFree and the mapping behind them take longer than the set-up's
 // kernels (C10H22 / 75 x 302: closing a handle 5.2 ms, the set-up's kernels 2).
-// At most 2 GiB per process, under 1 % of the device's memory, and all of it goes back
-// before an allocation of the library fails.  A block comes here only when the work
-// that used it is over, so any stream of the device may have it next; what it holds
-// then is not defined, as with hipMalloc.
+// At most 2.5 GiB per process, under 1 % of the device's memory, and all of it goes back
+// before an allocation of the library fails (a C10H22 / 75 x 302 handle with forces
+// takes 2.2).  A block comes here only when the work that used it is over, so any stream
+// of the device may have it next; what it holds then is not defined, as with hipMalloc.
 struct HipMemory {
   static constexpr int kNoMemory = hipErrorOutOfMemory;
   static int device(int* d) { return hipGetDevice(d); }
@@ -2902,7 +2902,7 @@ struct HipMemory {
 
 dg::DevicePool<HipMemory>& pool() {
   // not destroyed: handles may outlive static objects
-  static auto* p = new dg::DevicePool<HipMemory>((size_t)2 << 30);
+  static auto* p = new dg::DevicePool<HipMemory>((size_t)5 << 29);
   return *p;
 }
 

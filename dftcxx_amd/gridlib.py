@@ -515,7 +515,7 @@ class Batch:
 
 
 def release_memory():
-    """Gives the device memory kept from closed grids (at most 2 GiB) back to the device,
+    """Gives the device memory kept from closed grids (at most 2.5 GiB) back to the device,
     for other allocators of the process."""
     _check(lib().dg_release_memory())
 

@@ -91,7 +91,7 @@ int dg_lebedev_available(int npoints);
  * + create_grid() (src/moleculargrid.h:84,104,118; src/moleculargrid.cpp:175-261). */
 int dg_create(const dg_molecule* mol, const dg_basis* basis, const dg_grid_params* params,
               dg_handle** out);
-/* Device memory of a closed handle is kept for later ones, up to 2 GiB a process; it
+/* Device memory of a closed handle is kept for later ones, up to 2.5 GiB a process; it
  * goes back to the device before an allocation of this library fails, and with
  * dg_release_memory, for other allocators of the process. */
 int dg_destroy(dg_handle* h);
